@@ -366,6 +366,8 @@ extern "C" int okmi_basis_destroy(okmi_basis* b)
         if (p) (void)hipFree(p);
     if (b->d_padrows) (void)hipFree(b->d_padrows);
     if (b->d_colmap) (void)hipFree(b->d_colmap);
+    if (b->d_lshells) (void)hipFree(b->d_lshells);
+    if (b->d_lgroups) (void)hipFree(b->d_lgroups);
     delete[] b->h_shells;
     delete[] b->h_prims;
     delete[] b->h_T;

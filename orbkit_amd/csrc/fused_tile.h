@@ -94,6 +94,31 @@ struct FusedArgs {
     double* norm_part;        // FP64 kernel: per tile sum_p Phi_m(p)^2, [tile][mpad] (null: not wanted)
 };
 
+// Arguments of the FP64 kernel: the shells one by one (sorted by angular
+// momentum, row0 = C column, prim0 = first primitive group), C and the
+// occupations as the caller gave them.
+struct F64Args {
+    const ShellRec* shells;
+    const PrimGroup* groups;
+    int nsh;
+    int nmo, nao;
+    int need_mask;
+    const double* T;
+    GridDesc grid;
+    int64_t p0, np;
+    const double* C;          // [nmo][nao]
+    const double* occ;        // [nmo]
+    double* rho;
+    double* term;             // [.][ld_term]: code c's term in row term_row[c]
+    double* term2;            // as FusedArgs
+    int64_t ld_term;
+    int term_row[10];
+    int brick;
+    int tlx, tly, tlz;
+    int64_t nbx, nby, nbz;
+    double* norm_part;
+};
+
 template <int PASS> struct PassCodes;
 template <> struct PassCodes<0> { static constexpr int n = 1; static constexpr int c[4] = {0, 0, 0, 0}; };
 template <> struct PassCodes<1> { static constexpr int n = 4; static constexpr int c[4] = {0, 1, 2, 3}; };
@@ -102,7 +127,8 @@ template <> struct PassCodes<3> { static constexpr int n = 4; static constexpr i
 
 // brick coordinates of a tile (32-bit arithmetic: the host keeps the brick
 // count below 2^32)
-__device__ __forceinline__ void brick_of(const FusedArgs& a, int64_t tile, int64_t& bx, int64_t& by, int64_t& bz)
+template <typename Args>
+__device__ __forceinline__ void brick_of(const Args& a, int64_t tile, int64_t& bx, int64_t& by, int64_t& bz)
 {
     unsigned t = (unsigned)tile;
     const unsigned nbz = (unsigned)a.nbz, nby = (unsigned)a.nby;
@@ -114,7 +140,8 @@ __device__ __forceinline__ void brick_of(const FusedArgs& a, int64_t tile, int64
 
 // point of lane `ln` of this block's tile: index relative to p0, validity,
 // and the (clamped) coordinates
-__device__ __forceinline__ void tile_point(const FusedArgs& a, int64_t tile, int ln, int64_t& p, bool& act, double& px,
+template <typename Args>
+__device__ __forceinline__ void tile_point(const Args& a, int64_t tile, int ln, int64_t& p, bool& act, double& px,
                                            double& py, double& pz)
 {
     if (a.brick) {
@@ -180,8 +207,8 @@ struct Box {
 
 // output rows of one shell and AO set from its canonical Cartesian values
 // into the LDS tile (element type T: rounded once to FP32, or FP64)
-template <int L, typename E>
-__device__ __forceinline__ void store_rows(const FusedArgs& a, const ShellRec& sh, const double* c, E* dst)
+template <int L, typename Args, typename E>
+__device__ __forceinline__ void store_rows(const Args& a, const ShellRec& sh, const double* c, E* dst)
 {
     constexpr int NC = ncart(L);
     constexpr int LD = tile_ld<E>();
@@ -220,9 +247,12 @@ __device__ __forceinline__ void prim_sums(const PrimGroup& pg, double rr, double
     }
 }
 
-template <int L, int PASS, typename T>
-__device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const ShellRec& sh, double d2, double px,
-                                                 double py, double pz, int k0, T* lds, int lane)
+// One shell at the lane's point into the LDS tile, its first row at row
+// sh.row0 - k0, AO sets SS elements apart.  a: any argument struct with the
+// primitive groups (sh.prim0 the shell's first) and the general transforms.
+template <int L, int PASS, int SS, typename Args, typename T>
+__device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& sh, double d2, double px, double py,
+                                                 double pz, int k0, T* lds, int lane)
 {
     constexpr bool EXACT = std::is_same<T, double>::value;
     constexpr int LD = tile_ld<T>();
@@ -270,7 +300,7 @@ __device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const Shell
             } else {
                 first_deriv<L, 2, 0, double>(m, u, Z * S1, c);
             }
-            store_rows<L>(a, sh, c, lds + s * KC * LD + (sh.row0 - k0) * LD + lane);
+            store_rows<L>(a, sh, c, lds + s * SS + (sh.row0 - k0) * LD + lane);
         }
         return;
     }
@@ -289,7 +319,7 @@ __device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const Shell
         case 8: cart_all<L, 8, double>(P, S0, S1, S2, c); break;
         default: cart_all<L, 9, double>(P, S0, S1, S2, c); break;
         }
-        store_rows<L>(a, sh, c, lds + s * KC * LD + (sh.row0 - k0) * LD + lane);
+        store_rows<L>(a, sh, c, lds + s * SS + (sh.row0 - k0) * LD + lane);
     }
 }
 
@@ -431,12 +461,12 @@ __device__ __forceinline__ void eval_chunk(const FusedArgs& a, int ch, const Box
         if (d2 < sh.rcut2) {
             if (lane == 0) *live = tag;
             switch (sh.l) {
-            case 0: eval_shell_chunk<0, PASS>(a, sh, d2, px, py, pz, k0, L, lane); break;
-            case 1: eval_shell_chunk<1, PASS>(a, sh, d2, px, py, pz, k0, L, lane); break;
-            case 2: eval_shell_chunk<2, PASS>(a, sh, d2, px, py, pz, k0, L, lane); break;
-            case 3: eval_shell_chunk<3, PASS>(a, sh, d2, px, py, pz, k0, L, lane); break;
+            case 0: eval_shell_chunk<0, PASS, KC * LD>(a, sh, d2, px, py, pz, k0, L, lane); break;
+            case 1: eval_shell_chunk<1, PASS, KC * LD>(a, sh, d2, px, py, pz, k0, L, lane); break;
+            case 2: eval_shell_chunk<2, PASS, KC * LD>(a, sh, d2, px, py, pz, k0, L, lane); break;
+            case 3: eval_shell_chunk<3, PASS, KC * LD>(a, sh, d2, px, py, pz, k0, L, lane); break;
             default:
-                if constexpr (LM >= 4) eval_shell_chunk<4, PASS>(a, sh, d2, px, py, pz, k0, L, lane);
+                if constexpr (LM >= 4) eval_shell_chunk<4, PASS, KC * LD>(a, sh, d2, px, py, pz, k0, L, lane);
                 break;
             }
         } else {
@@ -577,7 +607,8 @@ __device__ __forceinline__ double2 axis_span(const double* ax, int64_t b, int tl
 // Bounding box of the tile's points: for a brick of a regular grid from the
 // (at most 2^tl) axis values it spans, otherwise by wave reductions over the
 // lanes' points (px, py, pz: lane l holds point l of the tile).
-__device__ __forceinline__ Box tile_box(const FusedArgs& a, int64_t tile, double px, double py, double pz)
+template <typename Args>
+__device__ __forceinline__ Box tile_box(const Args& a, int64_t tile, double px, double py, double pz)
 {
     Box box;
     if (a.brick) {
@@ -807,8 +838,8 @@ int launch_pass(const FusedArgs& a, int pass, int mt, int lm, hipStream_t st)
 }
 
 // FP64 kernel (rho_fused_f64.hip, compiled with FP64 MFMAs in the VGPR form);
-// mpad: MOs padded to a multiple of 4, a.mpad the same
-int launch_pass_f64(const FusedArgs& a, int pass, int mpad, int lm, hipStream_t st);
+// mpad: MOs padded to a multiple of 4
+int launch_pass_f64(const F64Args& a, int pass, int mpad, int lm, hipStream_t st);
 // mo_norm[m] += sum_t part[t][m] for m < nmo (the FP64 kernel's per-tile norms)
 int launch_norm_reduce(const double* part, int64_t ntile, int mpad, int nmo, double* mo_norm, hipStream_t st);
 

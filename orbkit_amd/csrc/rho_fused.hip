@@ -159,15 +159,15 @@ int prepare_fused_tables(OkmiBasis* b)
     std::vector<int> colmap(nkpad, -1);
     for (size_t j = 0; j < work.size(); ++j)
         for (int r = 0; r < b->h_shells[work[j]].nrow; ++r) colmap[krow[work[j]] + r] = b->h_shells[work[j]].row0 + r;
-    auto tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
-                      std::vector<PrimGroup>& groups, std::vector<ShellRec>& is, std::vector<ShellRec>& wsh,
-                      std::vector<PrimRec>& fp) {
-        fs.assign(work.size(), ShellRec{});
+    // shells `list` in that order with the given radii, and their primitive groups
+    auto group_tables = [&](const std::vector<int>& list, const std::vector<double>& frc2,
+                            const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
+                            std::vector<PrimGroup>& groups) {
+        fs.assign(list.size(), ShellRec{});
         groups.clear();
-        for (size_t j = 0; j < work.size(); ++j) {
-            const int i = work[j];
+        for (size_t j = 0; j < list.size(); ++j) {
+            const int i = list[j];
             fs[j] = b->h_shells[i];
-            fs[j].row0 = krow[i];
             fs[j].rcut2 = frc2[i];
             fs[j].prim0 = (int)groups.size();
             const ShellRec& hs = b->h_shells[i];
@@ -187,6 +187,12 @@ int prepare_fused_tables(OkmiBasis* b)
                 groups.push_back(pg);
             }
         }
+    };
+    auto tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
+                      std::vector<PrimGroup>& groups, std::vector<ShellRec>& is, std::vector<ShellRec>& wsh,
+                      std::vector<PrimRec>& fp) {
+        group_tables(work, frc2, fprc2, fs, groups);
+        for (size_t j = 0; j < work.size(); ++j) fs[j].row0 = krow[work[j]];
         // the same shells writing their internal rows (the many-MO and
         // staged paths stage the AO sets in the fused row order), also in
         // work order, and the primitives with these radii
@@ -205,6 +211,16 @@ int prepare_fused_tables(OkmiBasis* b)
     std::vector<PrimRec> fp, fp_s;
     tables(b->h_frcut2, b->h_fprcut2, fs, groups, is, wsh, fp);
     tables(b->h_frcut2s, b->h_fprcut2s, fs_s, groups_s, is_s, wsh_s, fp_s);
+    // by angular momentum, then by primitives (the costliest first)
+    std::vector<int> by_l(b->nshell);
+    for (int i = 0; i < b->nshell; ++i) by_l[i] = i;
+    std::stable_sort(by_l.begin(), by_l.end(), [&](int x, int y) {
+        const ShellRec &p = b->h_shells[x], &q = b->h_shells[y];
+        return p.l != q.l ? p.l > q.l : p.nprim > q.nprim;
+    });
+    std::vector<ShellRec> ls;
+    std::vector<PrimGroup> lgroups;
+    group_tables(by_l, b->h_frcut2, b->h_fprcut2, ls, lgroups);
     std::vector<ShellRec> os(b->h_shells, b->h_shells + b->nshell);
     for (int i = 0; i < b->nshell; ++i) os[i].rcut2 = b->h_frcut2[i];
     std::vector<int> padrows;
@@ -224,7 +240,10 @@ int prepare_fused_tables(OkmiBasis* b)
     if (!rc) rc = upload(&b->d_ishells_s, is_s, "rho_fused: internal-row shells (FP32 bound)");
     if (!rc) rc = upload(&b->d_wshells_s, wsh_s, "rho_fused: work-order shells (FP32 bound)");
     if (!rc) rc = upload(&b->d_fprims_s, fp_s, "rho_fused: primitives (FP32 bound)");
+    if (!rc) rc = upload(&b->d_lshells, ls, "rho_fused: shells by angular momentum");
+    if (!rc) rc = upload(&b->d_lgroups, lgroups, "rho_fused: their primitive groups");
     if (rc) return rc;
+    b->h_lshells = ls;
     b->nchunk = nchunk;
     b->nkpad = nkpad;
     b->npadrows = (int)padrows.size();
@@ -303,11 +322,8 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     double* term2 = term + 10 * chunk;
     double* norm_part = mo_norm ? (double*)(w + fixed + align256(FUSED_PT_BYTES * (size_t)chunk)) : nullptr;
 
-    hipLaunchKernelGGL(k_prep_c, dim3((unsigned)((mpad * kpad + 255) / 256)), dim3(256), 0, st, d_c, nmo, b->nao,
-                       prec, mpad, kpad, (const int*)b->d_colmap, cpl);
-    hipLaunchKernelGGL(k_pad_occ, dim3(1), dim3(256), 0, st, d_occ, nmo, (int)mpad, occp);
-
     int need = 0;
+    bool direct = prec == OKMI_PREC_F64;   // every output is a first derivative, each once: written where it belongs
     GatherCodes gc{};
     gc.n = nout;
     for (int r = 0; r < nout; ++r) {
@@ -315,6 +331,7 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
             okmi_set_error("The selection `drv=%d` is not valid!", drv_out[r]);
             return 1;
         }
+        if (drv_out[r] < 1 || drv_out[r] > 3 || (need >> drv_out[r] & 1)) direct = false;
         need |= 1 << drv_out[r];
         gc.c[r] = drv_out[r];
     }
@@ -322,39 +339,57 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     int lm = 0;   // highest angular momentum of the basis
     for (int i = 0; i < b->nshell; ++i) lm = std::max(lm, b->h_shells[i].l);
 
-    FusedArgs a{};
     // FP64 screens with the FP64 bound, the paths ending in FP32 with theirs
-    const bool split = prec != OKMI_PREC_F64;
-    a.shells = split ? b->d_fshells_s : b->d_fshells;
-    a.groups = split ? b->d_fgroups_s : b->d_fgroups;
-    a.T = b->d_T; a.chunks = b->d_chunks;
-    a.grid = g; a.nao = b->nao; a.nchunk = b->nchunk;
-    a.C = cpl; a.kpad = kpad; a.mpad = mpad; a.occ = occp;
-    a.term = term; a.term2 = term2; a.ld_term = chunk; a.need_mask = need;
-    a.brick = brick;
-    a.tlx = a.tly = a.tlz = 2;
-    a.nbx = (g.nx + 3) / 4; a.nby = (g.ny + 3) / 4; a.nbz = (g.nz + 3) / 4;
+    FusedArgs a{};
+    F64Args f{};
+    if (prec == OKMI_PREC_F64) {
+        f.shells = b->d_lshells; f.groups = b->d_lgroups; f.nsh = b->nshell; f.T = b->d_T;
+        f.grid = g; f.nmo = nmo; f.nao = b->nao; f.C = d_c; f.occ = d_occ;
+        f.term = term; f.term2 = term2; f.ld_term = chunk; f.need_mask = need;
+        for (int c = 0; c < 10; ++c) f.term_row[c] = c;
+        f.brick = brick;
+        f.tlx = f.tly = f.tlz = 2;
+        f.nbx = (g.nx + 3) / 4; f.nby = (g.ny + 3) / 4; f.nbz = (g.nz + 3) / 4;
+        f.norm_part = norm_part;   // read by the first pass (rho) only
+        if (direct) {
+            f.ld_term = ld_delta;
+            for (int r = 0; r < nout; ++r) f.term_row[drv_out[r]] = r;
+        }
+    } else {
+        hipLaunchKernelGGL(k_prep_c, dim3((unsigned)((mpad * kpad + 255) / 256)), dim3(256), 0, st, d_c, nmo, b->nao,
+                           prec, mpad, kpad, (const int*)b->d_colmap, cpl);
+        hipLaunchKernelGGL(k_pad_occ, dim3(1), dim3(256), 0, st, d_occ, nmo, (int)mpad, occp);
+        a.shells = b->d_fshells_s;
+        a.groups = b->d_fgroups_s;
+        a.T = b->d_T; a.chunks = b->d_chunks;
+        a.grid = g; a.nao = b->nao; a.nchunk = b->nchunk;
+        a.C = cpl; a.kpad = kpad; a.mpad = mpad; a.occ = occp;
+        a.term = term; a.term2 = term2; a.ld_term = chunk; a.need_mask = need;
+        a.brick = brick;
+        a.tlx = a.tly = a.tlz = 2;
+        a.nbx = (g.nx + 3) / 4; a.nby = (g.ny + 3) / 4; a.nbz = (g.nz + 3) / 4;
+    }
     for (int64_t c0 = 0; c0 < np; c0 += chunk) {
         const int64_t n = np - c0 < chunk ? np - c0 : chunk;
-        a.p0 = p0 + c0;
-        a.np = n;
-        a.rho = rho + c0;
+        a.p0 = f.p0 = p0 + c0;
+        a.np = f.np = n;
+        a.rho = f.rho = rho + c0;
+        if (direct) f.term = delta + c0;
         auto pass = [&](int ps) {
             switch (prec) {
-            case OKMI_PREC_F64: return launch_pass_f64(a, ps, (int)mpad, lm, st);
+            case OKMI_PREC_F64: return launch_pass_f64(f, ps, (int)mpad, lm, st);
             case OKMI_PREC_F32: return launch_pass<OKMI_PREC_F32>(a, ps, mt, lm, st);
             case OKMI_PREC_BF16X3: return launch_pass<OKMI_PREC_BF16X3>(a, ps, mt, lm, st);
             default: return launch_pass<OKMI_PREC_BF16X6>(a, ps, mt, lm, st);
             }
         };
-        a.norm_part = norm_part;   // read by the first pass (rho) only
         int r = pass(p1 ? 1 : 0);
         if (!r && p2) r = pass(2);
         if (!r && p3) r = pass(3);
         if (!r && mo_norm) r = launch_norm_reduce(norm_part, brick ? nbrick : (n + PTS - 1) / PTS, (int)mpad, nmo,
                                                   mo_norm, st);
         if (r) return r;
-        if (nout > 0)
+        if (nout > 0 && !direct)
             hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rho + c0, term, term2,
                                chunk, gc, delta + c0, ld_delta, n);
     }

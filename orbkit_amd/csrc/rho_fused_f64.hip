@@ -34,48 +34,69 @@
 // With block b = point group (points 4 b .. 4 b + 3 of the column), i = MO
 // and k = AO row, B lane l is AO row k0 + l / 16 at point l % 16 (the
 // 16x16x4 B operand) and D lane l is MO m0 + l / 16 at point l % 16.
-#include "fused_tile.h"
+#include "live_shells.h"
 
 namespace okmi_fused {
 namespace {
 
+// rows per chunk: whole shells up to this many AO rows
+template <int PASS> constexpr int chunk_rows() { return PASS == 0 ? 64 : 32; }
+
 // MOs of a launch: MT tiles of 16 and MR groups of 4
-template <int MT, int MR> struct MoSplit {
+template <int PASS, int MT, int MR> struct MoSplit {
     static constexpr int MP = 16 * MT + 4 * MR;   // padded MO count
     static constexpr int T = MT > 0 ? MT : 1;     // array extents
     static constexpr int R = MR > 0 ? MR : 1;
-    static constexpr int CR = (MP * KC + 255) / 256;   // C elements per thread per chunk
+    static constexpr int KR = chunk_rows<PASS>();
+    static constexpr int LC = MP + 1;             // row stride of the C stage (odd: its writes, k fastest, are conflict-free)
+    static constexpr int CR = (MP * KR + 255) / 256;   // C elements per thread per chunk
+    // list entries held at a time (fewer where two workgroups would otherwise not fit a CU's LDS)
+    static constexpr int LCAP = MP == 56 ? 128 : 256;
 };
 
 // acc[mt][s] (16x16x4 tiles) and accr[r][s] (4x4x4 groups) += C * AO_s over
-// one chunk, for the 16-point column `col`; C from the chunk's LDS stage
-// cs[k][m] (MP MOs per row), AO from the LDS tile
+// the nk K steps of one chunk, for the 16-point column `col`; C from the
+// chunk's LDS stage cs[k][m], AO from the LDS tile.  The operands of a step
+// are read before the MFMAs of the step before it.
 template <int PASS, int MT, int MR>
-__device__ __forceinline__ void contract_f64(const double* L, const double* cs, int col, int g, int n16,
-                                             d4 (&acc)[MoSplit<MT, MR>::T][PassCodes<PASS>::n],
-                                             double (&accr)[MoSplit<MT, MR>::R][PassCodes<PASS>::n])
+__device__ __forceinline__ void contract_f64(const double* L, const double* cs, int col, int g, int n16, int nk,
+                                             d4 (&acc)[MoSplit<PASS, MT, MR>::T][PassCodes<PASS>::n],
+                                             double (&accr)[MoSplit<PASS, MT, MR>::R][PassCodes<PASS>::n])
 {
+    using M = MoSplit<PASS, MT, MR>;
     constexpr int NS = PassCodes<PASS>::n;
     constexpr int LD = Tile<OKMI_PREC_F64>::LD;
-    constexpr int MP = MoSplit<MT, MR>::MP;
-#pragma unroll
-    for (int ks = 0; ks < KC / 4; ++ks) {
+    struct Operands {
+        double cv[M::T], cr[M::R], bv[NS];
+    };
+    auto read = [&](int ks, Operands& o) {
         const int k = 4 * ks + g;
-        double cv[MoSplit<MT, MR>::T], cr[MoSplit<MT, MR>::R], bv[NS];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) cv[mt] = cs[k * MP + 16 * mt + n16];
+        for (int mt = 0; mt < MT; ++mt) o.cv[mt] = cs[k * M::LC + 16 * mt + n16];
 #pragma unroll
-        for (int r = 0; r < MR; ++r) cr[r] = cs[k * MP + 16 * MT + 4 * r + (n16 & 3)];
+        for (int r = 0; r < MR; ++r) o.cr[r] = cs[k * M::LC + 16 * MT + 4 * r + (n16 & 3)];
 #pragma unroll
-        for (int q = 0; q < NS; ++q) bv[q] = L[(q * KC + k) * LD + col * 16 + n16];
+        for (int q = 0; q < NS; ++q) o.bv[q] = L[(q * M::KR + k) * LD + col * 16 + n16];
+    };
+    auto mma = [&](const Operands& o) {
 #pragma unroll
         for (int q = 0; q < NS; ++q) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                acc[mt][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[mt], bv[q], acc[mt][q], 0, 0, 0);
+                acc[mt][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.cv[mt], o.bv[q], acc[mt][q], 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < MR; ++r) accr[r][q] = __builtin_amdgcn_mfma_f64_4x4x4f64(cr[r], bv[q], accr[r][q], 0, 0, 0);
+            for (int r = 0; r < MR; ++r)
+                accr[r][q] = __builtin_amdgcn_mfma_f64_4x4x4f64(o.cr[r], o.bv[q], accr[r][q], 0, 0, 0);
         }
+    };
+    Operands x, y;
+    read(0, x);
+    for (int ks = 0; ks < nk; ks += 2) {
+        read(min(ks + 1, nk - 1), y);
+        mma(x);
+        if (ks + 1 >= nk) break;
+        read(min(ks + 2, nk - 1), x);
+        mma(y);
     }
 }
 
@@ -84,11 +105,11 @@ __device__ __forceinline__ void contract_f64(const double* L, const double* cs, 
 // added through LDS (red: 4 x MP doubles, free after the chunk loop's last
 // barrier), one row of norm_part per tile.  Called by every thread.
 template <int PASS, int MT, int MR>
-__device__ __forceinline__ void tile_norms(const FusedArgs& a, int64_t tile, int col, int lane, bool act, double* red,
-                                           const d4 (&acc)[MoSplit<MT, MR>::T][PassCodes<PASS>::n],
-                                           const double (&accr)[MoSplit<MT, MR>::R][PassCodes<PASS>::n])
+__device__ __forceinline__ void tile_norms(const F64Args& a, int64_t tile, int col, int lane, bool act, double* red,
+                                           const d4 (&acc)[MoSplit<PASS, MT, MR>::T][PassCodes<PASS>::n],
+                                           const double (&accr)[MoSplit<PASS, MT, MR>::R][PassCodes<PASS>::n])
 {
-    constexpr int MP = MoSplit<MT, MR>::MP;
+    constexpr int MP = MoSplit<PASS, MT, MR>::MP;
     const int g = lane >> 4, n16 = lane & 15;
     auto put = [&](int m, double f) {
         double v = act ? f * f : 0.0;
@@ -112,9 +133,9 @@ __device__ __forceinline__ void tile_norms(const FusedArgs& a, int64_t tile, int
 // Density terms of the column from its MO values: item i of acc[mt][s] is
 // Phi_s[16 mt + 4 i + g][point n16], accr[r][s] is Phi_s[16 MT + 4 r + g][point n16]
 template <int PASS, int MT, int MR>
-__device__ __forceinline__ void epilogue_f64(const FusedArgs& a, int64_t tile, int col, int lane,
-                                             const d4 (&acc)[MoSplit<MT, MR>::T][PassCodes<PASS>::n],
-                                             const double (&accr)[MoSplit<MT, MR>::R][PassCodes<PASS>::n])
+__device__ __forceinline__ void epilogue_f64(const F64Args& a, int64_t tile, int col, int lane,
+                                             const d4 (&acc)[MoSplit<PASS, MT, MR>::T][PassCodes<PASS>::n],
+                                             const double (&accr)[MoSplit<PASS, MT, MR>::R][PassCodes<PASS>::n])
 {
     constexpr int NS = PassCodes<PASS>::n;
     const int g = lane >> 4, n16 = lane & 15;
@@ -123,6 +144,8 @@ __device__ __forceinline__ void epilogue_f64(const FusedArgs& a, int64_t tile, i
     for (int s = 0; s < (NS > 1 ? NS - 1 : 1); ++s) t[s] = 0.0;
 #pragma unroll
     for (int q = 0; q < 6; ++q) u[q] = 0.0;
+    // padding MOs repeat the last one's values and weigh nothing
+    auto occ = [&](int m) { return m < a.nmo ? a.occ[m] : 0.0; };
     auto add = [&](double w, const double* f) {   // f[s]: Phi_s of one MO at this point
         if constexpr (PASS <= 1) r0 += w * (f[0] * f[0]);
 #pragma unroll
@@ -143,14 +166,14 @@ __device__ __forceinline__ void epilogue_f64(const FusedArgs& a, int64_t tile, i
             double f[NS];
 #pragma unroll
             for (int s = 0; s < NS; ++s) f[s] = acc[mt][s][i];
-            add(a.occ[16 * mt + 4 * i + g], f);
+            add(occ(16 * mt + 4 * i + g), f);
         }
 #pragma unroll
     for (int r = 0; r < MR; ++r) {
         double f[NS];
 #pragma unroll
         for (int s = 0; s < NS; ++s) f[s] = accr[r][s];
-        add(a.occ[16 * MT + 4 * r + g], f);
+        add(occ(16 * MT + 4 * r + g), f);
     }
     r0 += __shfl_xor(r0, 16);
     r0 += __shfl_xor(r0, 32);
@@ -175,7 +198,7 @@ __device__ __forceinline__ void epilogue_f64(const FusedArgs& a, int64_t tile, i
 #pragma unroll
         for (int s = 1; s < NS; ++s) {
             const int code = PassCodes<PASS>::c[s];
-            if (a.need_mask >> code & 1) a.term[code * a.ld_term + p] = t[s - 1];
+            if (a.need_mask >> code & 1) a.term[a.term_row[code] * a.ld_term + p] = t[s - 1];
         }
         if constexpr (PASS == 1) {
 #pragma unroll
@@ -186,32 +209,26 @@ __device__ __forceinline__ void epilogue_f64(const FusedArgs& a, int64_t tile, i
 }
 
 template <int PASS, int MT, int MR, int LM>
-__global__ __launch_bounds__(256, 2) void k_rho_fused_f64(FusedArgs a)
+__global__ __launch_bounds__(256, 2) void k_rho_fused_f64(F64Args a)
 {
-    using M = MoSplit<MT, MR>;
+    using M = MoSplit<PASS, MT, MR>;
     constexpr int NS = PassCodes<PASS>::n;
-    constexpr int MP = M::MP;
-    __shared__ double lds[NS * KC * Tile<OKMI_PREC_F64>::LD];
-    __shared__ double cs[KC * MP];   // the chunk's C columns, [k][m]
-    __shared__ int next[1];          // next work entry of the chunk being evaluated
-    __shared__ int live[1];          // last chunk with a live shell
-    __shared__ unsigned long long lmask[LIVE_WORDS];   // chunks with a shell in reach of the tile
+    constexpr int LD = Tile<OKMI_PREC_F64>::LD;
+    constexpr int KR = M::KR, MP = M::MP, LC = M::LC, LCAP = M::LCAP;
+    __shared__ double lds[NS * KR * LD];
+    __shared__ double cs[KR * LC];   // the chunk's C columns, [k][m]
+    __shared__ uint2 ent[LCAP + 1];  // shells in reach of the tile
+    __shared__ int col[2][KR];       // C column of each row of this chunk and the next
+    __shared__ int wsum[8];
 
     const int64_t tile = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n16 = lane & 15;
-    if (threadIdx.x == 0) {
-        next[0] = 0;
-        live[0] = -1;
-    }
-    __syncthreads();
     int64_t pidx;
     bool pact;
     double px, py, pz;
     tile_point(a, tile, lane, pidx, pact, px, py, pz);   // lane l of every wave: point l of the tile
     const Box box = tile_box(a, tile, px, py, pz);
-    live_chunks(a, box, wave, lane, lmask);
-    __syncthreads();
     // the coordinates are consumed here so that the evaluation does not count
     // their loads as outstanding (it would then also wait for the C loads)
     asm volatile("" ::"v"(px), "v"(py), "v"(pz));
@@ -229,29 +246,67 @@ __global__ __launch_bounds__(256, 2) void k_rho_fused_f64(FusedArgs a)
 
     typedef const __attribute__((address_space(1))) double gdouble;
     gdouble* C = (gdouble*)a.C;
-    for (int ch = next_live(a, lmask, 0); ch < a.nchunk; ch = next_live(a, lmask, ch + 1)) {
-        const int k0 = ch * KC;
-        // this thread's C elements e = threadIdx.x + 256 j of [m][k] (k
-        // fastest: coalesced rows); clamped to the last element
-        double creg[M::CR];
-#pragma unroll
-        for (int j = 0; j < M::CR; ++j) {
-            const int e = min((int)threadIdx.x + 256 * j, MP * KC - 1);
-            creg[j] = C[(int64_t)(e / KC) * a.kpad + k0 + e % KC];
+    int t0 = 0;
+    while (t0 < a.nsh) {
+        // shells in reach, as many as the list holds
+        const int base = t0;
+        int cnt = 0, rows = 0;
+        while (t0 < a.nsh && t0 - base < (int)LIST_ID_MASK - LCAP) {
+            const int n = append_live<LCAP, LCAP>(a.shells, a.nsh, t0, base, box, ent, wsum, cnt, rows);
+            __syncthreads();
+            if (n < 0) break;
+            cnt += n;
+            t0 += LCAP;
         }
-        eval_chunk<PASS, LM>(a, ch, box, px, py, pz, lds, &next[0], &live[0], ch, wave == 0, lane);
-        // the stage is free: every wave read it before the previous barrier
+        ListChunk ck;
+        ck.next<KR>(ent, 0, cnt, lane);
+        if (wave == 0) ck.columns(col[0], lane);
+        __syncthreads();
+        for (int s = 0, buf = 0; s < cnt; buf ^= 1) {
+            // this thread's C elements e = threadIdx.x + 256 j of [m][k] (k
+            // fastest), held through the evaluation; rows past the chunk's
+            // last read its first column, MOs past the last the last one
+            double creg[M::CR];
 #pragma unroll
-        for (int j = 0; j < M::CR; ++j) {
-            const int e = (int)threadIdx.x + 256 * j;
-            if (e < MP * KC) cs[(e % KC) * MP + e / KC] = creg[j];
+            for (int j = 0; j < M::CR; ++j) {
+                const int e = min((int)threadIdx.x + 256 * j, MP * KR - 1);
+                const int k = e % KR;
+                creg[j] = C[(int64_t)min(e / KR, a.nmo - 1) * a.nao + col[buf][k < ck.used ? k : 0]];
+            }
+            for (int e = wave; e < ck.n; e += 4) {
+                ShellRec sh = load_shell(a.shells, base + ck.shell(e));
+                sh.row0 = ck.row(e);
+                const double d2 = box.dist2(sh);
+                switch (sh.l) {
+                case 0: eval_shell_chunk<0, PASS, KR * LD>(a, sh, d2, px, py, pz, 0, lds, lane); break;
+                case 1: eval_shell_chunk<1, PASS, KR * LD>(a, sh, d2, px, py, pz, 0, lds, lane); break;
+                case 2: eval_shell_chunk<2, PASS, KR * LD>(a, sh, d2, px, py, pz, 0, lds, lane); break;
+                case 3: eval_shell_chunk<3, PASS, KR * LD>(a, sh, d2, px, py, pz, 0, lds, lane); break;
+                default:
+                    if constexpr (LM >= 4) eval_shell_chunk<4, PASS, KR * LD>(a, sh, d2, px, py, pz, 0, lds, lane);
+                    break;
+                }
+            }
+            const int nk = (ck.used + 3) / 4;
+            if (wave == 3) {   // rows that fill the last K step
+                for (int q = 0; q < NS; ++q)
+                    for (int r = ck.used; r < 4 * nk; ++r) lds[(q * KR + r) * LD + lane] = 0.0;
+            }
+            // the stage is free: every wave read it before the previous barrier
+#pragma unroll
+            for (int j = 0; j < M::CR; ++j) {
+                const int e = (int)threadIdx.x + 256 * j;
+                if (e < MP * KR) cs[(e % KR) * LC + e / KR] = e % KR < ck.used ? creg[j] : 0.0;
+            }
+            __syncthreads();
+            s += ck.n;
+            if (s < cnt) {   // uniform
+                ck.next<KR>(ent, s, cnt, lane);
+                if (wave == 0) ck.columns(col[buf ^ 1], lane);
+            }
+            contract_f64<PASS, MT, MR>(lds, cs, wave, g, n16, nk, acc, accr);
+            __syncthreads();
         }
-        __syncthreads();
-        // every wave finished taking from the counter before the barrier and
-        // takes from it again after the next one
-        if (threadIdx.x == 0) next[0] = 0;
-        if (live[0] == ch) contract_f64<PASS, MT, MR>(lds, cs, wave, g, n16, acc, accr);
-        __syncthreads();
     }
     epilogue_f64<PASS, MT, MR>(a, tile, wave, lane, acc, accr);
     if constexpr (PASS <= 1) {
@@ -284,7 +339,7 @@ __global__ void k_norm_reduce(const double* part, int64_t ntile, int mpad, int n
 }
 
 template <int PASS, int LM, int MT, int MR>
-int launch_f64_one(const FusedArgs& a, hipStream_t st)
+int launch_f64_one(const F64Args& a, hipStream_t st)
 {
     const int64_t ntile = a.brick ? a.nbx * a.nby * a.nbz : (a.np + PTS - 1) / PTS;
     if (ntile >= ((int64_t)1 << 31)) {   // one workgroup per tile; brick indices are 32-bit
@@ -299,7 +354,7 @@ int launch_f64_one(const FusedArgs& a, hipStream_t st)
 
 // mpad: MOs padded to a multiple of 4 (4 .. 64)
 template <int PASS, int LM>
-int launch_f64_m(const FusedArgs& a, int mpad, hipStream_t st)
+int launch_f64_m(const F64Args& a, int mpad, hipStream_t st)
 {
     switch (mpad) {
 #define OKMI_F64_CASE(MT, MR) \
@@ -325,7 +380,7 @@ int launch_norm_reduce(const double* part, int64_t ntile, int mpad, int nmo, dou
     return 0;
 }
 
-int launch_pass_f64(const FusedArgs& a, int pass, int mpad, int lm, hipStream_t st)
+int launch_pass_f64(const F64Args& a, int pass, int mpad, int lm, hipStream_t st)
 {
     const bool l3 = lm <= 3;
     switch (pass) {
