@@ -175,10 +175,45 @@ __device__ __forceinline__ void cart_drv(const ShellPows<L, R>& P, int d, R S0, 
     }
 }
 
-// exp(-t) in FP64 for t >= 0; t beyond 746 underflows to +0 exactly as libm.
+// a b + c.  A compile-time constant c goes in a scalar register pair of one
+// v_fma_f64: left to itself the compiler takes the two-operand form for a
+// polynomial step and copies the coefficient into its result first, two
+// vector instructions per coefficient.
+__device__ __forceinline__ double fma_coef(double a, double b, double c)
+{
+    if (__builtin_constant_p(c)) {
+        double d;
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+        return d;
+    }
+    return fma(a, b, c);
+}
+
+// exp(-t) in FP64 for t >= 0, within one ulp: Cody-Waite reduction
+// -t = s - k ln2, |s| <= ln2/2 (ln2 in a high part exact in 32 bits and a low
+// part), exp(s) by the Chebyshev interpolant of degree 11 on that interval
+// (relative error below 1e-17), and 2^-k by exponent adjustment, which
+// underflows to +0.  Even and odd coefficients run in two chains: most shells
+// have one primitive in reach of a tile, so the chain of its exponential is
+// what a wave waits for.  Branch-free: t is clamped to 1e4 (+0 in FP64).
 __device__ __forceinline__ double gauss_f64(double t)
 {
-    return t < 746.0 ? exp(-t) : 0.0;
+    t = fmin(t, 1.0e4);
+    const double k = __builtin_rint(t * 1.4426950408889634);
+    double s = fma(k, 6.93147180369123816490e-01, -t);
+    s = fma(k, 1.90821492927058770002e-10, s);
+    const double q = s * s;
+    double e = fma_coef(q, 2.763263963904103e-07, 2.4801485482328494e-05);
+    double o = fma_coef(q, 2.5110037605963777e-08, 2.755724091857897e-06);
+    e = fma_coef(e, q, 0.0013888888952314775);
+    o = fma_coef(o, q, 0.00019841269890047113);
+    e = fma_coef(e, q, 0.0416666666664881);
+    o = fma_coef(o, q, 0.008333333333319601);
+    e = fma_coef(e, q, 0.5000000000000019);
+    o = fma_coef(o, q, 0.1666666666666668);
+    e = fma_coef(e, q, 1.0);
+    o = fma_coef(o, q, 1.0);
+    return ldexp(fma(o, s, e), -(int)k);
 }
 
 // exp(-t) to FP32 accuracy for any t >= 0 given in FP64: the range reduction
@@ -210,6 +245,7 @@ __device__ __forceinline__ double gauss_f64_fast(double t)
     double r = fma(-k, 6.93147180369123816490e-01, t);
     r = fma(-k, 1.90821492927058770002e-10, r);
     const double s = -r;
+    const auto fma = fma_coef;
     double p = 0.0013941118940759135;
     p = fma(p, s, 0.0083751347746787615);
     p = fma(p, s, 0.041666352770387056);
@@ -283,5 +319,105 @@ __device__ __forceinline__ void cart_rows_to(const double* c, Store&& store)
     if constexpr (R < ncart(L)) {
         store(R, c[R] * cart_norm(L, R));
         cart_rows_to<L, R + 1>(c, store);
+    }
+}
+
+// Rows of a standard spherical (sph_row) or Cartesian (component norms)
+// shell straight from the monomials, instead of the Cartesian values of each
+// AO set first and their combinations after: with row polynomial
+// P = sum_t v_t m_t of the degree-L monomials,
+//   chi = P S0,  d_a chi = P (R_a S1) + (d_a P) S0,
+//   d_aa chi = P (S1 + R_a^2 S2) + (d_a P) (2 R_a S1) + (d_aa P) S0.
+template <int L, bool SPH> __host__ __device__ constexpr int shell_rows() { return SPH ? 2 * L + 1 : ncart(L); }
+template <int L, bool SPH, int R> __host__ __device__ constexpr SphRow shell_row()
+{
+    if constexpr (SPH) return sph_row(L, R);
+    else return SphRow{1, {{R, cart_norm(L, R)}, {0, 0.0}, {0, 0.0}}};
+}
+
+// sum_t v_t m_t
+template <int L, bool SPH, int R>
+__device__ __forceinline__ double row_poly(const double* m)
+{
+    constexpr SphRow row = shell_row<L, SPH, R>();
+    double v = row.t[0].v == 1.0 ? m[row.t[0].c] : row.t[0].v * m[row.t[0].c];
+    if constexpr (row.n > 1) v = fma(row.t[1].v, m[row.t[1].c], v);
+    if constexpr (row.n > 2) v = fma(row.t[2].v, m[row.t[2].c], v);
+    return v;
+}
+
+// acc + sum over the row's terms of v_t e (e - 1) ... (N factors of axis A's
+// exponent) u[component with that exponent lowered by N]; u: the degree
+// L - N monomials (times a radial sum)
+template <int L, bool SPH, int R, int A, int N, int T = 0>
+__device__ __forceinline__ double row_lowered(const double* u, double acc)
+{
+    constexpr SphRow row = shell_row<L, SPH, R>();
+    if constexpr (T < row.n) {
+        constexpr int c = row.t[T].c;
+        constexpr int e[3] = {cart_exp(L, c, 0), cart_exp(L, c, 1), cart_exp(L, c, 2)};
+        if constexpr (e[A] >= N) {
+            constexpr double f = row.t[T].v * (N == 1 ? e[A] : e[A] * (e[A] - 1));
+            constexpr int lo = cart_index(L - N, e[0] - N * (A == 0), e[1] - N * (A == 1), e[2] - N * (A == 2));
+            acc = f == 1.0 ? acc + u[lo] : fma(f, u[lo], acc);
+        }
+        return row_lowered<L, SPH, R, A, N, T + 1>(u, acc);
+    } else {
+        return acc;
+    }
+}
+
+// value rows: store(row, value)
+template <int L, bool SPH, int R = 0, typename Store>
+__device__ __forceinline__ void rows_value(const double* m, double S0, Store&& store)
+{
+    if constexpr (R < shell_rows<L, SPH>()) {
+        store(R, row_poly<L, SPH, R>(m) * S0);
+        rows_value<L, SPH, R + 1>(m, S0, store);
+    }
+}
+
+// value and first derivatives: store(set, row, value); u: degree L - 1
+// monomials times S0, RS1[a] = R_a S1
+template <int L, bool SPH, int R = 0, typename Store>
+__device__ __forceinline__ void rows_first(const double* m, const double* u, double S0, const double (&RS1)[3],
+                                           Store&& store)
+{
+    if constexpr (R < shell_rows<L, SPH>()) {
+        const double P = row_poly<L, SPH, R>(m);
+        store(0, R, P * S0);
+        store(1, R, row_lowered<L, SPH, R, 0, 1>(u, P * RS1[0]));
+        store(2, R, row_lowered<L, SPH, R, 1, 1>(u, P * RS1[1]));
+        store(3, R, row_lowered<L, SPH, R, 2, 1>(u, P * RS1[2]));
+        rows_first<L, SPH, R + 1>(m, u, S0, RS1, store);
+    }
+}
+
+// diagonal second derivatives: store(axis, row, value); u1: degree L - 1
+// monomials, u2: degree L - 2 monomials times S0, RS1[a] = 2 R_a S1,
+// RS2[a] = S1 + R_a^2 S2
+template <int L, bool SPH, int R = 0, typename Store>
+__device__ __forceinline__ void rows_second(const double* m, const double* u1, const double* u2,
+                                            const double (&RS1)[3], const double (&RS2)[3], Store&& store)
+{
+    if constexpr (R < shell_rows<L, SPH>()) {
+        const double P = row_poly<L, SPH, R>(m);
+        store(0, R, fma(row_lowered<L, SPH, R, 0, 1>(u1, 0.0), RS1[0], row_lowered<L, SPH, R, 0, 2>(u2, P * RS2[0])));
+        store(1, R, fma(row_lowered<L, SPH, R, 1, 1>(u1, 0.0), RS1[1], row_lowered<L, SPH, R, 1, 2>(u2, P * RS2[1])));
+        store(2, R, fma(row_lowered<L, SPH, R, 2, 1>(u1, 0.0), RS1[2], row_lowered<L, SPH, R, 2, 2>(u2, P * RS2[2])));
+        rows_second<L, SPH, R + 1>(m, u1, u2, RS1, RS2, store);
+    }
+}
+
+// the degree-L monomials times f
+template <int L, int C = 0>
+__device__ __forceinline__ void scaled_monos(double X, double Y, double Z, double f, double* u)
+{
+    if constexpr (L >= 0) {
+        ShellPows<(L > 0 ? L : 0), double> P;
+        P.init(X, Y, Z);
+        first_mono<(L > 0 ? L : 0), 0, double>(P, u);
+#pragma unroll
+        for (int c = 0; c < ncart(L > 0 ? L : 0); ++c) u[c] *= f;
     }
 }

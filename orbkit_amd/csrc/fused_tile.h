@@ -206,30 +206,25 @@ struct Box {
 };
 
 // output rows of one shell and AO set from its canonical Cartesian values
-// into the LDS tile (element type T: rounded once to FP32, or FP64)
+// through its general transform block, into the LDS tile (element type T:
+// rounded once to FP32, or FP64)
 template <int L, typename Args, typename E>
 __device__ __forceinline__ void store_rows(const Args& a, const ShellRec& sh, const double* c, E* dst)
 {
     constexpr int NC = ncart(L);
     constexpr int LD = tile_ld<E>();
-    auto store = [&](int r, double v) { dst[r * LD] = (E)v; };
-    if (sh.kind == SHELL_T_SPHERICAL) {
-        sph_rows_to<L, 0>(c, store);
-    } else if (sh.kind == SHELL_T_CARTESIAN) {
-        cart_rows_to<L, 0>(c, store);
-    } else {
-        const OKMI_CONST double* T = cptr(a.T) + sh.t0;
-        for (int r = 0; r < sh.nrow; ++r) {
-            double v = 0.0;
+    const OKMI_CONST double* T = cptr(a.T) + sh.t0;
+    for (int r = 0; r < sh.nrow; ++r) {
+        double v = 0.0;
 #pragma unroll
-            for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
-            store(r, v);
-        }
+        for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
+        dst[r * LD] = (E)v;
     }
 }
 
 // radial sums of the first N primitives of a group:
-// S0 = sum d e, S1 = sum -2 alpha d e, S2 = sum 4 alpha^2 d e, e = exp(-alpha r^2)
+// S0 += sum d e, S1 += sum alpha d e, S2 += sum alpha^2 d e, e = exp(-alpha r^2)
+// (the caller applies the powers of two of -2 alpha and 4 alpha^2)
 // (EXACT: the full-accuracy FP64 exponential, else the one accurate to
 // 2.6e-9 for values that end in FP32)
 template <int N, bool need1, bool need2, bool EXACT>
@@ -242,8 +237,50 @@ __device__ __forceinline__ void prim_sums(const PrimGroup& pg, double rr, double
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         S0 += de[j];
-        if constexpr (need1) S1 = fma(-2.0 * pg.alpha[j], de[j], S1);
-        if constexpr (need2) S2 = fma(4.0 * pg.alpha[j] * pg.alpha[j], de[j], S2);
+        if constexpr (need1) S1 = fma(pg.alpha[j], de[j], S1);
+        if constexpr (need2) S2 = fma(pg.alpha[j] * pg.alpha[j], de[j], S2);
+    }
+}
+
+// Rows of a standard shell of one pass into the LDS tile (rounded once to T)
+template <int L, bool SPH, int PASS, int SS, typename T>
+__device__ __forceinline__ void eval_rows(double X, double Y, double Z, double S0, double S1, double S2, T* dst)
+{
+    constexpr int LD = tile_ld<T>();
+    double m[ncart(L)];
+    scaled_monos<L>(X, Y, Z, 1.0, m);
+    auto put = [&](int s, int r, double v) { dst[s * SS + r * LD] = (T)v; };
+    if constexpr (PASS == 0) {
+        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
+    } else if constexpr (PASS == 1) {
+        double u[L > 0 ? ncart(L - 1) : 1];
+        scaled_monos<L - 1>(X, Y, Z, S0, u);
+        const double RS1[3] = {X * S1, Y * S1, Z * S1};
+        rows_first<L, SPH>(m, u, S0, RS1, put);
+    } else if constexpr (PASS == 2) {
+        double u1[L > 0 ? ncart(L - 1) : 1], u2[L > 1 ? ncart(L - 2) : 1];
+        scaled_monos<L - 1>(X, Y, Z, 1.0, u1);
+        scaled_monos<L - 2>(X, Y, Z, S0, u2);
+        const double RS1[3] = {2.0 * X * S1, 2.0 * Y * S1, 2.0 * Z * S1};
+        const double RS2[3] = {fma(X * X, S2, S1), fma(Y * Y, S2, S1), fma(Z * Z, S2, S1)};
+        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
+        rows_second<L, SPH>(m, u1, u2, RS1, RS2, [&](int a, int r, double v) { put(1 + a, r, v); });
+    } else {   // mixed second derivatives: orbkit's formula, by Cartesian component
+        ShellPows<L, double> P;
+        P.init(X, Y, Z);
+        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
+        double c[ncart(L)];
+        auto rows = [&](int s) {
+            auto store = [&](int r, double v) { put(s, r, v); };
+            if constexpr (SPH) sph_rows_to<L, 0>(c, store);
+            else cart_rows_to<L, 0>(c, store);
+        };
+        cart_all<L, 7, double>(P, S0, S1, S2, c);
+        rows(1);
+        cart_all<L, 8, double>(P, S0, S1, S2, c);
+        rows(2);
+        cart_all<L, 9, double>(P, S0, S1, S2, c);
+        rows(3);
     }
 }
 
@@ -280,6 +317,17 @@ __device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& 
         }
         if (nl < 4) break;
     }
+    S1 *= -2.0;
+    S2 *= 4.0;
+    // standard shells: rows straight from the monomials
+    T* dst = lds + (sh.row0 - k0) * LD + lane;
+    if (sh.kind != SHELL_T_GENERAL && (L <= 3 || sh.kind == SHELL_T_CARTESIAN)) {
+        if (L <= 3 && sh.kind == SHELL_T_SPHERICAL)
+            eval_rows<(L <= 3 ? L : 0), true, PASS, SS>(X, Y, Z, S0, S1, S2, dst);
+        else
+            eval_rows<L, false, PASS, SS>(X, Y, Z, S0, S1, S2, dst);
+        return;
+    }
     ShellPows<L, double> P;
     P.init(X, Y, Z);
     constexpr int NC = ncart(L);
@@ -300,7 +348,7 @@ __device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& 
             } else {
                 first_deriv<L, 2, 0, double>(m, u, Z * S1, c);
             }
-            store_rows<L>(a, sh, c, lds + s * SS + (sh.row0 - k0) * LD + lane);
+            store_rows<L>(a, sh, c, dst + s * SS);
         }
         return;
     }
@@ -319,7 +367,7 @@ __device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& 
         case 8: cart_all<L, 8, double>(P, S0, S1, S2, c); break;
         default: cart_all<L, 9, double>(P, S0, S1, S2, c); break;
         }
-        store_rows<L>(a, sh, c, lds + s * SS + (sh.row0 - k0) * LD + lane);
+        store_rows<L>(a, sh, c, dst + s * SS);
     }
 }
 

@@ -146,11 +146,12 @@ __device__ __forceinline__ void epilogue_f64(const F64Args& a, int64_t tile, int
     for (int q = 0; q < 6; ++q) u[q] = 0.0;
     // padding MOs repeat the last one's values and weigh nothing
     auto occ = [&](int m) { return m < a.nmo ? a.occ[m] : 0.0; };
+    const bool second = PASS == 1 && a.need_mask >> 4;   // uniform: f_a f_b halves wanted
     auto add = [&](double w, const double* f) {   // f[s]: Phi_s of one MO at this point
         if constexpr (PASS <= 1) r0 += w * (f[0] * f[0]);
 #pragma unroll
         for (int s = 1; s < NS; ++s) t[s - 1] += 2.0 * w * (f[0] * f[s]);
-        if constexpr (PASS == 1) {
+        if (second) {
             u[0] += 2.0 * w * (f[1] * f[1]);
             u[1] += 2.0 * w * (f[2] * f[2]);
             u[2] += 2.0 * w * (f[3] * f[3]);
@@ -182,7 +183,7 @@ __device__ __forceinline__ void epilogue_f64(const F64Args& a, int64_t tile, int
         t[s] += __shfl_xor(t[s], 16);
         t[s] += __shfl_xor(t[s], 32);
     }
-    if constexpr (PASS == 1) {
+    if (second) {
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
             u[q] += __shfl_xor(u[q], 16);
