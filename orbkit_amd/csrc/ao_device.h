@@ -335,16 +335,55 @@ template <int L, bool SPH, int R> __host__ __device__ constexpr SphRow shell_row
     else return SphRow{1, {{R, cart_norm(L, R)}, {0, 0.0}, {0, 0.0}}};
 }
 
-// sum_t v_t m_t
-template <int L, bool SPH, int R>
-__device__ __forceinline__ double row_poly(const double* m)
-{
-    constexpr SphRow row = shell_row<L, SPH, R>();
-    double v = row.t[0].v == 1.0 ? m[row.t[0].c] : row.t[0].v * m[row.t[0].c];
-    if constexpr (row.n > 1) v = fma(row.t[1].v, m[row.t[1].c], v);
-    if constexpr (row.n > 2) v = fma(row.t[2].v, m[row.t[2].c], v);
-    return v;
-}
+// Row polynomials of a shell at one point.  Standard spherical d and f rows
+// (sph_row's coefficients) in factored form from the quadratic monomials
+// (fewer operations and registers than the ten cubic ones); other rows from
+// the degree-L monomials.
+template <int L, bool SPH> struct RowPolys {
+    double m[ncart(L)];
+    __device__ __forceinline__ RowPolys(double X, double Y, double Z)
+    {
+        ShellPows<L, double> P;
+        P.init(X, Y, Z);
+        first_mono<L, 0, double>(P, m);
+    }
+    template <int R> __device__ __forceinline__ double row() const
+    {
+        constexpr SphRow row = shell_row<L, SPH, R>();
+        double v = row.t[0].v == 1.0 ? m[row.t[0].c] : row.t[0].v * m[row.t[0].c];
+        if constexpr (row.n > 1) v = fma(row.t[1].v, m[row.t[1].c], v);
+        if constexpr (row.n > 2) v = fma(row.t[2].v, m[row.t[2].c], v);
+        return v;
+    }
+};
+template <> struct RowPolys<2, true> {
+    double X, Y, Z;
+    __device__ __forceinline__ RowPolys(double x, double y, double z) : X(x), Y(y), Z(z) {}
+    template <int R> __device__ __forceinline__ double row() const
+    {
+        constexpr double q = sph_row(2, 0).t[2].v;   // 1 / sqrt(3); x^2 + y^2 has -q/2
+        if constexpr (R == 0) return q * fma(Z, Z, -0.5 * fma(X, X, Y * Y));
+        if constexpr (R == 1) return X * Z;
+        if constexpr (R == 2) return Y * Z;
+        if constexpr (R == 3) return 0.5 * (X - Y) * (X + Y);
+        return X * Y;
+    }
+};
+template <> struct RowPolys<3, true> {
+    double X, Y, Z;
+    __device__ __forceinline__ RowPolys(double x, double y, double z) : X(x), Y(y), Z(z) {}
+    template <int R> __device__ __forceinline__ double row() const
+    {
+        constexpr double a0 = sph_row(3, 0).t[0].v, a1 = sph_row(3, 1).t[2].v, a5 = sph_row(3, 5).t[0].v;
+        if constexpr (R == 0) return a0 * (Z * fma(Z, Z, -1.5 * fma(X, X, Y * Y)));
+        if constexpr (R == 1) return a1 * (X * fma(Z, Z, -0.25 * fma(X, X, Y * Y)));
+        if constexpr (R == 2) return a1 * (Y * fma(Z, Z, -0.25 * fma(X, X, Y * Y)));
+        if constexpr (R == 3) return 0.5 * Z * ((X - Y) * (X + Y));
+        if constexpr (R == 4) return X * Y * Z;
+        if constexpr (R == 5) return a5 * (X * fma(X, X, -3.0 * (Y * Y)));
+        return a5 * (Y * fma(3.0 * X, X, -(Y * Y)));
+    }
+};
 
 // acc + sum over the row's terms of v_t e (e - 1) ... (N factors of axis A's
 // exponent) u[component with that exponent lowered by N]; u: the degree
@@ -367,48 +406,6 @@ __device__ __forceinline__ double row_lowered(const double* u, double acc)
     }
 }
 
-// value rows: store(row, value)
-template <int L, bool SPH, int R = 0, typename Store>
-__device__ __forceinline__ void rows_value(const double* m, double S0, Store&& store)
-{
-    if constexpr (R < shell_rows<L, SPH>()) {
-        store(R, row_poly<L, SPH, R>(m) * S0);
-        rows_value<L, SPH, R + 1>(m, S0, store);
-    }
-}
-
-// value and first derivatives: store(set, row, value); u: degree L - 1
-// monomials times S0, RS1[a] = R_a S1
-template <int L, bool SPH, int R = 0, typename Store>
-__device__ __forceinline__ void rows_first(const double* m, const double* u, double S0, const double (&RS1)[3],
-                                           Store&& store)
-{
-    if constexpr (R < shell_rows<L, SPH>()) {
-        const double P = row_poly<L, SPH, R>(m);
-        store(0, R, P * S0);
-        store(1, R, row_lowered<L, SPH, R, 0, 1>(u, P * RS1[0]));
-        store(2, R, row_lowered<L, SPH, R, 1, 1>(u, P * RS1[1]));
-        store(3, R, row_lowered<L, SPH, R, 2, 1>(u, P * RS1[2]));
-        rows_first<L, SPH, R + 1>(m, u, S0, RS1, store);
-    }
-}
-
-// diagonal second derivatives: store(axis, row, value); u1: degree L - 1
-// monomials, u2: degree L - 2 monomials times S0, RS1[a] = 2 R_a S1,
-// RS2[a] = S1 + R_a^2 S2
-template <int L, bool SPH, int R = 0, typename Store>
-__device__ __forceinline__ void rows_second(const double* m, const double* u1, const double* u2,
-                                            const double (&RS1)[3], const double (&RS2)[3], Store&& store)
-{
-    if constexpr (R < shell_rows<L, SPH>()) {
-        const double P = row_poly<L, SPH, R>(m);
-        store(0, R, fma(row_lowered<L, SPH, R, 0, 1>(u1, 0.0), RS1[0], row_lowered<L, SPH, R, 0, 2>(u2, P * RS2[0])));
-        store(1, R, fma(row_lowered<L, SPH, R, 1, 1>(u1, 0.0), RS1[1], row_lowered<L, SPH, R, 1, 2>(u2, P * RS2[1])));
-        store(2, R, fma(row_lowered<L, SPH, R, 2, 1>(u1, 0.0), RS1[2], row_lowered<L, SPH, R, 2, 2>(u2, P * RS2[2])));
-        rows_second<L, SPH, R + 1>(m, u1, u2, RS1, RS2, store);
-    }
-}
-
 // the degree-L monomials times f
 template <int L, int C = 0>
 __device__ __forceinline__ void scaled_monos(double X, double Y, double Z, double f, double* u)
@@ -419,5 +416,85 @@ __device__ __forceinline__ void scaled_monos(double X, double Y, double Z, doubl
         first_mono<(L > 0 ? L : 0), 0, double>(P, u);
 #pragma unroll
         for (int c = 0; c < ncart(L > 0 ? L : 0); ++c) u[c] *= f;
+    }
+}
+
+// The AO sets of one pass (PassCodes) of each row of a standard shell
+template <int L, bool SPH, int PASS> struct RowSets {
+    static constexpr int NS = PASS == 0 ? 1 : PASS == 4 ? 7 : 4;
+    RowPolys<L, SPH> m;
+    double S0, R1[3], R2[3];
+    double u1[L > 0 ? ncart(L - 1) : 1];                 // degree L - 1 monomials (PASS 1: times S0)
+    double u2[PASS >= 2 && L > 1 ? ncart(L - 2) : 1];    // degree L - 2 monomials times S0
+    ShellPows<L, double> P;                              // PASS 3
+    double s1, s2;
+
+    __device__ __forceinline__ RowSets(double X, double Y, double Z, double s0_, double s1_, double s2_)
+        : m(X, Y, Z), S0(s0_), s1(s1_), s2(s2_)
+    {
+        if constexpr (PASS == 1 || PASS == 2 || PASS == 4) {
+            R1[0] = X * s1_;
+            R1[1] = Y * s1_;
+            R1[2] = Z * s1_;
+            scaled_monos<L - 1>(X, Y, Z, PASS == 1 ? s0_ : 1.0, u1);
+        }
+        if constexpr (PASS == 2 || PASS == 4) {
+            R2[0] = fma(X * X, s2_, s1_);
+            R2[1] = fma(Y * Y, s2_, s1_);
+            R2[2] = fma(Z * Z, s2_, s1_);
+            scaled_monos<L - 2>(X, Y, Z, s0_, u2);
+        }
+        if constexpr (PASS == 3) P.init(X, Y, Z);
+    }
+    template <int R, int D, int T = 0> __device__ __forceinline__ double mixed(double acc) const
+    {
+        constexpr SphRow row = shell_row<L, SPH, R>();
+        if constexpr (T < row.n) {
+            return mixed<R, D, T + 1>(fma(row.t[T].v, cart_comp<L, row.t[T].c, D, double>(P, S0, s1, s2), acc));
+        } else {
+            return acc;
+        }
+    }
+    // d_aa of the row: p its polynomial, d its derivative along axis A
+    template <int R, int A> __device__ __forceinline__ double second(double p, double d) const
+    {
+        return fma(d, 2.0 * R1[A], row_lowered<L, SPH, R, A, 2>(u2, p * R2[A]));
+    }
+    template <int R> __device__ __forceinline__ void row(double (&v)[NS]) const
+    {
+        const double p = m.template row<R>();
+        v[0] = p * S0;
+        if constexpr (PASS == 1) {
+            v[1] = row_lowered<L, SPH, R, 0, 1>(u1, p * R1[0]);
+            v[2] = row_lowered<L, SPH, R, 1, 1>(u1, p * R1[1]);
+            v[3] = row_lowered<L, SPH, R, 2, 1>(u1, p * R1[2]);
+        } else if constexpr (PASS == 2 || PASS == 4) {
+            const double d[3] = {row_lowered<L, SPH, R, 0, 1>(u1, 0.0), row_lowered<L, SPH, R, 1, 1>(u1, 0.0),
+                                 row_lowered<L, SPH, R, 2, 1>(u1, 0.0)};
+            if constexpr (PASS == 4) {
+                v[1] = fma(d[0], S0, p * R1[0]);
+                v[2] = fma(d[1], S0, p * R1[1]);
+                v[3] = fma(d[2], S0, p * R1[2]);
+            }
+            v[NS - 3] = second<R, 0>(p, d[0]);
+            v[NS - 2] = second<R, 1>(p, d[1]);
+            v[NS - 1] = second<R, 2>(p, d[2]);
+        } else if constexpr (PASS == 3) {
+            v[1] = mixed<R, 7>(0.0);
+            v[2] = mixed<R, 8>(0.0);
+            v[3] = mixed<R, 9>(0.0);
+        }
+    }
+};
+
+// f(row, values of the sets) for every row from R on
+template <int R, int L, bool SPH, int PASS, typename F>
+__device__ __forceinline__ void each_row(const RowSets<L, SPH, PASS>& rows, F&& f)
+{
+    if constexpr (R < shell_rows<L, SPH>()) {
+        double v[RowSets<L, SPH, PASS>::NS];
+        rows.template row<R>(v);
+        f(R, v);
+        each_row<R + 1>(rows, f);
     }
 }

@@ -36,6 +36,7 @@
 //                        every second derivative (orbkit/core.py:287-302)
 //   PASS 2  {0,xx,yy,zz} f0 f_aa halves of the diagonal second derivatives
 //   PASS 3  {0,xy,xz,yz} f0 f_ab halves of the mixed ones
+//   PASS 4  {0,x,y,z,xx,yy,zz} (FP64 kernel) passes 1 and 2 at once
 // Each term is written to its own FP64 buffer (no read-modify-write); a
 // gather kernel then forms orbkit's output rows.
 #pragma once
@@ -94,12 +95,27 @@ struct FusedArgs {
     double* norm_part;        // FP64 kernel: per tile sum_p Phi_m(p)^2, [tile][mpad] (null: not wanted)
 };
 
-// Arguments of the FP64 kernel: the shells one by one (sorted by angular
-// momentum, row0 = C column, prim0 = first primitive group), C and the
-// occupations as the caller gave them.
+// n / d for n < 2^31 by a multiplication (all scalar instructions; a division
+// of wave-uniform integers is a dozen vector ones)
+struct FastDiv {
+    unsigned d, m, s;
+    void set(unsigned div)
+    {
+        d = div;
+        int l = 0;
+        while (((uint64_t)1 << l) < div) ++l;
+        m = l ? (unsigned)((((uint64_t)1 << (31 + l)) + div - 1) / div) : 0;
+        s = l ? l - 1 : 0;
+    }
+    __device__ __forceinline__ unsigned div(unsigned n) const { return d == 1 ? n : __umulhi(n, m) >> s; }
+};
+
+// Arguments of the FP64 kernel (fused_f64.h): the shells one by one (sorted by
+// angular momentum, row0 = C column), C and the occupations as the caller gave
+// them.
 struct F64Args {
-    const ShellRec* shells;
-    const PrimGroup* groups;
+    const ListRec* shells;
+    const PrimGroup* more;
     int nsh;
     int nmo, nao;
     int need_mask;
@@ -107,16 +123,28 @@ struct F64Args {
     GridDesc grid;
     int64_t p0, np;
     const double* C;          // [nmo][nao]
+    const double* ct;         // [nao][MOs padded to 4], zero padded; null: C is read as it is
     const double* occ;        // [nmo]
     double* rho;
     double* term;             // [.][ld_term]: code c's term in row term_row[c]
     double* term2;            // as FusedArgs
     int64_t ld_term;
+    int64_t ld_set;           // MO values: stride between the sets of term
     int term_row[10];
-    int brick;
-    int tlx, tly, tlz;
-    int64_t nbx, nby, nbz;
-    double* norm_part;
+    int brick;                // regular grid in bricks of 4x4x4 points (p0 = 0, all points)
+    int64_t ntile;            // tiles of 64 points
+    FastDiv dz, dy;           // bricks per axis
+    double* norm_part;        // per tile sum_p Phi_m(p)^2, [tile][groups of 4 MOs x 4] (null: not wanted)
+
+    // grid, np set: bricks or runs of 64 points
+    void set_bricks(bool on)
+    {
+        brick = on;
+        const int64_t bx = (grid.nx + 3) / 4, by = (grid.ny + 3) / 4, bz = (grid.nz + 3) / 4;
+        ntile = on ? bx * by * bz : (np + 63) / 64;
+        dz.set(on ? (unsigned)bz : 1);
+        dy.set(on ? (unsigned)by : 1);
+    }
 };
 
 template <int PASS> struct PassCodes;
@@ -124,11 +152,11 @@ template <> struct PassCodes<0> { static constexpr int n = 1; static constexpr i
 template <> struct PassCodes<1> { static constexpr int n = 4; static constexpr int c[4] = {0, 1, 2, 3}; };
 template <> struct PassCodes<2> { static constexpr int n = 4; static constexpr int c[4] = {0, 4, 5, 6}; };
 template <> struct PassCodes<3> { static constexpr int n = 4; static constexpr int c[4] = {0, 7, 8, 9}; };
+template <> struct PassCodes<4> { static constexpr int n = 7; static constexpr int c[7] = {0, 1, 2, 3, 4, 5, 6}; };
 
 // brick coordinates of a tile (32-bit arithmetic: the host keeps the brick
 // count below 2^32)
-template <typename Args>
-__device__ __forceinline__ void brick_of(const Args& a, int64_t tile, int64_t& bx, int64_t& by, int64_t& bz)
+__device__ __forceinline__ void brick_of(const FusedArgs& a, int64_t tile, int64_t& bx, int64_t& by, int64_t& bz)
 {
     unsigned t = (unsigned)tile;
     const unsigned nbz = (unsigned)a.nbz, nby = (unsigned)a.nby;
@@ -140,8 +168,7 @@ __device__ __forceinline__ void brick_of(const Args& a, int64_t tile, int64_t& b
 
 // point of lane `ln` of this block's tile: index relative to p0, validity,
 // and the (clamped) coordinates
-template <typename Args>
-__device__ __forceinline__ void tile_point(const Args& a, int64_t tile, int ln, int64_t& p, bool& act, double& px,
+__device__ __forceinline__ void tile_point(const FusedArgs& a, int64_t tile, int ln, int64_t& p, bool& act, double& px,
                                            double& py, double& pz)
 {
     if (a.brick) {
@@ -208,8 +235,8 @@ struct Box {
 // output rows of one shell and AO set from its canonical Cartesian values
 // through its general transform block, into the LDS tile (element type T:
 // rounded once to FP32, or FP64)
-template <int L, typename Args, typename E>
-__device__ __forceinline__ void store_rows(const Args& a, const ShellRec& sh, const double* c, E* dst)
+template <int L, typename E>
+__device__ __forceinline__ void store_rows(const FusedArgs& a, const ShellRec& sh, const double* c, E* dst)
 {
     constexpr int NC = ncart(L);
     constexpr int LD = tile_ld<E>();
@@ -242,59 +269,50 @@ __device__ __forceinline__ void prim_sums(const PrimGroup& pg, double rr, double
     }
 }
 
-// Rows of a standard shell of one pass into the LDS tile (rounded once to T)
-template <int L, bool SPH, int PASS, int SS, typename T>
-__device__ __forceinline__ void eval_rows(double X, double Y, double Z, double S0, double S1, double S2, T* dst)
+// Rows of a shell of one pass into the LDS tile from its first row's place,
+// AO sets SS elements apart (rounded once to T)
+template <int L, int PASS, int SS, typename T>
+__device__ __forceinline__ void shell_rows_to(const FusedArgs& a, const ShellRec& sh, double X, double Y, double Z,
+                                              double S0, double S1, double S2, T* dst)
 {
     constexpr int LD = tile_ld<T>();
-    double m[ncart(L)];
-    scaled_monos<L>(X, Y, Z, 1.0, m);
-    auto put = [&](int s, int r, double v) { dst[s * SS + r * LD] = (T)v; };
-    if constexpr (PASS == 0) {
-        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
-    } else if constexpr (PASS == 1) {
-        double u[L > 0 ? ncart(L - 1) : 1];
-        scaled_monos<L - 1>(X, Y, Z, S0, u);
-        const double RS1[3] = {X * S1, Y * S1, Z * S1};
-        rows_first<L, SPH>(m, u, S0, RS1, put);
-    } else if constexpr (PASS == 2) {
-        double u1[L > 0 ? ncart(L - 1) : 1], u2[L > 1 ? ncart(L - 2) : 1];
-        scaled_monos<L - 1>(X, Y, Z, 1.0, u1);
-        scaled_monos<L - 2>(X, Y, Z, S0, u2);
-        const double RS1[3] = {2.0 * X * S1, 2.0 * Y * S1, 2.0 * Z * S1};
-        const double RS2[3] = {fma(X * X, S2, S1), fma(Y * Y, S2, S1), fma(Z * Z, S2, S1)};
-        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
-        rows_second<L, SPH>(m, u1, u2, RS1, RS2, [&](int a, int r, double v) { put(1 + a, r, v); });
-    } else {   // mixed second derivatives: orbkit's formula, by Cartesian component
+    constexpr int NS = PassCodes<PASS>::n;
+    auto put = [&](int r, const double (&v)[NS]) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) dst[s * SS + r * LD] = (T)v[s];
+    };
+    if (L <= 3 && sh.kind == SHELL_T_SPHERICAL) {
+        each_row<0>(RowSets<(L <= 3 ? L : 0), true, PASS>(X, Y, Z, S0, S1, S2), put);
+    } else if (sh.kind == SHELL_T_CARTESIAN) {
+        each_row<0>(RowSets<L, false, PASS>(X, Y, Z, S0, S1, S2), put);
+    } else {
         ShellPows<L, double> P;
         P.init(X, Y, Z);
-        rows_value<L, SPH>(m, S0, [&](int r, double v) { put(0, r, v); });
         double c[ncart(L)];
-        auto rows = [&](int s) {
-            auto store = [&](int r, double v) { put(s, r, v); };
-            if constexpr (SPH) sph_rows_to<L, 0>(c, store);
-            else cart_rows_to<L, 0>(c, store);
+        auto set = [&](auto code, int s) {
+            cart_all<L, decltype(code)::value, double>(P, S0, S1, S2, c);
+            store_rows<L>(a, sh, c, dst + s * SS);
         };
-        cart_all<L, 7, double>(P, S0, S1, S2, c);
-        rows(1);
-        cart_all<L, 8, double>(P, S0, S1, S2, c);
-        rows(2);
-        cart_all<L, 9, double>(P, S0, S1, S2, c);
-        rows(3);
+        set(std::integral_constant<int, 0>{}, 0);
+        if constexpr (NS > 1) {
+            set(std::integral_constant<int, PassCodes<PASS>::c[1]>{}, 1);
+            set(std::integral_constant<int, PassCodes<PASS>::c[2]>{}, 2);
+            set(std::integral_constant<int, PassCodes<PASS>::c[3]>{}, 3);
+        }
     }
 }
 
 // One shell at the lane's point into the LDS tile, its first row at row
 // sh.row0 - k0, AO sets SS elements apart.  a: any argument struct with the
 // primitive groups (sh.prim0 the shell's first) and the general transforms.
-template <int L, int PASS, int SS, typename Args, typename T>
-__device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& sh, double d2, double px, double py,
+template <int L, int PASS, int SS, typename T>
+__device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const ShellRec& sh, double d2, double px, double py,
                                                  double pz, int k0, T* lds, int lane)
 {
     constexpr bool EXACT = std::is_same<T, double>::value;
     constexpr int LD = tile_ld<T>();
     constexpr int NS = PassCodes<PASS>::n;
-    constexpr bool need1 = PASS == 1 || PASS == 2;
+    constexpr bool need1 = PASS == 1 || PASS == 2 || PASS == 4;
     constexpr bool need2 = PASS >= 2;
     const double X = px - sh.cx, Y = py - sh.cy, Z = pz - sh.cz;
     const double rr = X * X + Y * Y + Z * Z;
@@ -319,56 +337,7 @@ __device__ __forceinline__ void eval_shell_chunk(const Args& a, const ShellRec& 
     }
     S1 *= -2.0;
     S2 *= 4.0;
-    // standard shells: rows straight from the monomials
-    T* dst = lds + (sh.row0 - k0) * LD + lane;
-    if (sh.kind != SHELL_T_GENERAL && (L <= 3 || sh.kind == SHELL_T_CARTESIAN)) {
-        if (L <= 3 && sh.kind == SHELL_T_SPHERICAL)
-            eval_rows<(L <= 3 ? L : 0), true, PASS, SS>(X, Y, Z, S0, S1, S2, dst);
-        else
-            eval_rows<L, false, PASS, SS>(X, Y, Z, S0, S1, S2, dst);
-        return;
-    }
-    ShellPows<L, double> P;
-    P.init(X, Y, Z);
-    constexpr int NC = ncart(L);
-    if constexpr (PASS == 1) {
-        // value and x, y, z derivatives from shared monomials
-        double m[NC], u[L > 0 ? ncart(L - 1) : 1], c[NC];
-        first_mono<L, 0, double>(P, m);
-        lower_mono<L, 0, double>(P, S0, u);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            if (s == 0) {
-#pragma unroll
-                for (int k = 0; k < NC; ++k) c[k] = m[k] * S0;
-            } else if (s == 1) {
-                first_deriv<L, 0, 0, double>(m, u, X * S1, c);
-            } else if (s == 2) {
-                first_deriv<L, 1, 0, double>(m, u, Y * S1, c);
-            } else {
-                first_deriv<L, 2, 0, double>(m, u, Z * S1, c);
-            }
-            store_rows<L>(a, sh, c, dst + s * SS);
-        }
-        return;
-    }
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        double c[NC];
-        switch (PassCodes<PASS>::c[s]) {
-        case 0: cart_all<L, 0, double>(P, S0, S1, S2, c); break;
-        case 1: cart_all<L, 1, double>(P, S0, S1, S2, c); break;
-        case 2: cart_all<L, 2, double>(P, S0, S1, S2, c); break;
-        case 3: cart_all<L, 3, double>(P, S0, S1, S2, c); break;
-        case 4: cart_all<L, 4, double>(P, S0, S1, S2, c); break;
-        case 5: cart_all<L, 5, double>(P, S0, S1, S2, c); break;
-        case 6: cart_all<L, 6, double>(P, S0, S1, S2, c); break;
-        case 7: cart_all<L, 7, double>(P, S0, S1, S2, c); break;
-        case 8: cart_all<L, 8, double>(P, S0, S1, S2, c); break;
-        default: cart_all<L, 9, double>(P, S0, S1, S2, c); break;
-        }
-        store_rows<L>(a, sh, c, dst + s * SS);
-    }
+    shell_rows_to<L, PASS, SS>(a, sh, X, Y, Z, S0, S1, S2, lds + (sh.row0 - k0) * LD + lane);
 }
 
 template <int PREC, int PASS>
@@ -655,8 +624,7 @@ __device__ __forceinline__ double2 axis_span(const double* ax, int64_t b, int tl
 // Bounding box of the tile's points: for a brick of a regular grid from the
 // (at most 2^tl) axis values it spans, otherwise by wave reductions over the
 // lanes' points (px, py, pz: lane l holds point l of the tile).
-template <typename Args>
-__device__ __forceinline__ Box tile_box(const Args& a, int64_t tile, double px, double py, double pz)
+__device__ __forceinline__ Box tile_box(const FusedArgs& a, int64_t tile, double px, double py, double pz)
 {
     Box box;
     if (a.brick) {
@@ -887,7 +855,9 @@ int launch_pass(const FusedArgs& a, int pass, int mt, int lm, hipStream_t st)
 
 // FP64 kernel (rho_fused_f64.hip, compiled with FP64 MFMAs in the VGPR form);
 // mpad: MOs padded to a multiple of 4
-int launch_pass_f64(const F64Args& a, int pass, int mpad, int lm, hipStream_t st);
+// standard: every shell l <= 3 with real spherical or Cartesian rows
+int launch_pass_f64(const F64Args& a, int pass, int mpad, bool standard, hipStream_t st);
+int launch_pass_f64_d2(const F64Args& a, int pass, int mpad, bool standard, hipStream_t st);
 // mo_norm[m] += sum_t part[t][m] for m < nmo (the FP64 kernel's per-tile norms)
 int launch_norm_reduce(const double* part, int64_t ntile, int mpad, int nmo, double* mo_norm, hipStream_t st);
 

@@ -3,110 +3,89 @@
 // 20-atom molecule and 7% of those of 200 atoms, where fixed 32-row chunks
 // holding at least one such shell make up 55% and 20%.
 //
-// The shells are taken from a table sorted by angular momentum (highest
-// first), so that the shells of one chunk cost about the same and the four
-// waves that share a chunk finish together.
+// The shells come from a table sorted by class (angular momentum, highest
+// first, and kind of row map), so that four consecutive entries mostly share
+// one: they are evaluated together, one per 16 lanes of a wave.
 #pragma once
 #include "fused_tile.h"
 
 namespace okmi_fused {
 
-// One list entry: x = shell (relative to the list's base index) and the
-// number of AO rows before it, y = its first AO row (C column).  The entry
-// after the last holds the total row count.
-constexpr int LIST_ID_BITS = 18;
-constexpr unsigned LIST_ID_MASK = (1u << LIST_ID_BITS) - 1;
+// One list entry: the shell (relative to the list's base index) and its class,
+// its first AO row (C column) and its live primitives among the first four,
+// its squared distance to the tile's box.
+struct alignas(16) LiveShell {
+    unsigned idcls, rowlive;
+    double d2;
+};
+constexpr int LIST_ID_BITS = 18, LIST_ROW_BITS = 29;
+constexpr unsigned LIST_ID_MASK = (1u << LIST_ID_BITS) - 1, LIST_ROW_MASK = (1u << LIST_ROW_BITS) - 1;
 
-// value of the previous lanes' bits: population count of m below this lane
+// population count of the bits of m below this lane
 __device__ __forceinline__ int bits_below(unsigned long long m)
 {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
 }
 
-// Tests the table's next BLK shells (from t0; thread i < BLK takes shell
+// Bounding box of the tile's points into sbox (lo x, y, z, hi x, y, z): wave w
+// < 3 reduces axis w over its lanes (lane l holds point l of the tile).  Ready
+// after the next barrier.
+__device__ __forceinline__ void shared_box(int wave, double px, double py, double pz, double* sbox)
+{
+    if (wave < 3) {
+        const double v = wave == 0 ? px : wave == 1 ? py : pz;
+        double lo = v, hi = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            lo = fmin(lo, __shfl_xor(lo, o));
+            hi = fmax(hi, __shfl_xor(hi, o));
+        }
+        sbox[wave] = lo;       // (every lane the same value)
+        sbox[3 + wave] = hi;
+    }
+}
+
+// Tests the table's next LCAP shells (from t0; thread i < LCAP takes shell
 // t0 + i) against the box and appends those in reach to ent, which holds
-// `cnt` entries and `rows` rows so far and has room for LCAP.  Returns the
-// entries added, or -1 if they do not fit (nothing is appended).  Called by
-// all 256 threads; ent is ready after the next barrier.  wsum: 8 ints, free
-// again after the next barrier.
-template <int LCAP, int BLK>
-__device__ __forceinline__ int append_live(const ShellRec* shells, int nsh, int t0, int base, const Box& box,
-                                           uint2* ent, int* wsum, int cnt, int& rows)
+// `cnt` entries and has room for LCAP.  Returns the entries added, or -1 if
+// they do not fit (nothing is appended).  Called by all NW waves; ent is ready
+// after the next barrier.  wsum: NW ints, free again after the next barrier.
+template <int LCAP, int NW>
+__device__ __forceinline__ int append_live(const ListRec* shells, int nsh, int t0, int base, const double* sbox,
+                                           LiveShell* ent, int* wsum, int cnt)
 {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = t0 + (int)threadIdx.x;
-    int nrow = 0, row0 = 0;
-    if ((int)threadIdx.x < BLK && i < nsh) {
-        const ShellRec sh = shells[i];
-        row0 = sh.row0;
-        if (box.dist2(sh) < sh.rcut2) nrow = sh.nrow;
-    }
-    const unsigned long long hit = __builtin_amdgcn_ballot_w64(nrow > 0);
-    int before = 0, total = 0;   // rows of the wave's live shells before this lane, and in all
+    bool hit = false;
+    unsigned idcls = 0, rowlive = 0;
+    double d2 = 0.0;
+    if ((int)threadIdx.x < LCAP && i < nsh) {
+        const ListRec& sh = shells[i];
 #pragma unroll
-    for (int b = 0; b < 6; ++b) {   // nrow <= 32
-        const unsigned long long m = __builtin_amdgcn_ballot_w64((nrow >> b & 1) != 0);
-        before += bits_below(m) << b;
-        total += __builtin_popcountll(m) << b;
-    }
-    if (lane == 0) {
-        wsum[2 * wave] = __builtin_popcountll(hit);
-        wsum[2 * wave + 1] = total;
-    }
-    __syncthreads();
-    int n = 0, nr = 0, n0 = 0, r0 = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        if (w == wave) {
-            n0 = n;
-            r0 = nr;
+        for (int k = 0; k < 3; ++k) {
+            const double d = fmax(fmax(sbox[k] - sh.c[k], sh.c[k] - sbox[3 + k]), 0.0);
+            d2 = fma(d, d, d2);
         }
-        n += wsum[2 * w];
-        nr += wsum[2 * w + 1];
+        hit = d2 < sh.rcut2;
+        int live = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) live += d2 < sh.prcut2[q];
+        idcls = (unsigned)(i - base) | (unsigned)sh.cls << LIST_ID_BITS;
+        rowlive = (unsigned)sh.row0 | (unsigned)live << LIST_ROW_BITS;
     }
-    n = __builtin_amdgcn_readfirstlane(n);
-    nr = __builtin_amdgcn_readfirstlane(nr);
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+    if (lane == 0) wsum[wave] = __builtin_popcountll(m);
+    __syncthreads();
+    int n = 0, n0 = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const int c = __builtin_amdgcn_readfirstlane(wsum[w]);
+        if (w < wave) n0 += c;
+        n += c;
+    }
     if (cnt + n > LCAP) return -1;
-    if (nrow > 0)
-        ent[cnt + n0 + bits_below(hit)] =
-            uint2{(unsigned)(i - base) | (unsigned)(rows + r0 + before) << LIST_ID_BITS, (unsigned)row0};
-    rows += nr;
-    if (threadIdx.x == 0) ent[cnt + n].x = (unsigned)rows << LIST_ID_BITS;
+    if (hit) ent[cnt + n0 + bits_below(m)] = LiveShell{idcls, rowlive, d2};
     return n;
 }
-
-// The next chunk of a list: entries s .. s + n - 1, whole shells of at most
-// KR rows in all.  Lane j holds entry s + j (ex, ey).
-struct ListChunk {
-    unsigned ex, ey;
-    int n, r0, used;   // entries, the first one's row, rows
-
-    template <int KR>
-    __device__ __forceinline__ void next(const uint2* ent, int s, int cnt, int lane)
-    {
-        const uint2 v = ent[min(s + lane, cnt)];
-        ex = v.x;
-        ey = v.y;
-        const unsigned after = ent[min(s + 1 + lane, cnt)].x >> LIST_ID_BITS;
-        r0 = __builtin_amdgcn_readfirstlane(ex >> LIST_ID_BITS);
-        const unsigned long long fit = __builtin_amdgcn_ballot_w64(s + lane < cnt && (int)after - r0 <= KR);
-        n = __builtin_popcountll(fit);
-        used = n > 0 ? (int)__builtin_amdgcn_readlane(after, n - 1) - r0 : 0;
-    }
-    __device__ __forceinline__ int shell(int j) const { return __builtin_amdgcn_readlane(ex, j) & LIST_ID_MASK; }
-    __device__ __forceinline__ int row(int j) const
-    {
-        return (int)((unsigned)__builtin_amdgcn_readlane(ex, j) >> LIST_ID_BITS) - r0;
-    }
-    // C column of each row of the chunk, written by one wave
-    __device__ __forceinline__ void columns(int* col, int lane) const
-    {
-        const int first = (int)(ex >> LIST_ID_BITS) - r0;
-        // rows of this lane's shell: up to the next lane's first row
-        const int last = __shfl_down((int)(ex >> LIST_ID_BITS), 1) - r0;
-        if (lane < n)
-            for (int r = first; r < (lane == n - 1 ? used : last); ++r) col[r] = (int)ey + r - first;
-    }
-};
 
 }  // namespace okmi_fused

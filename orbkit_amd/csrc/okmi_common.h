@@ -49,6 +49,19 @@ struct PrimGroup {
 };
 static_assert(sizeof(PrimGroup) == 96, "PrimGroup layout");
 
+// A shell with its first four primitives (by screening radius, largest
+// first; unused slots alpha = d = 0, prcut2 = -1) for the kernels that list the
+// shells in reach of a tile: read by one wide scalar load.
+struct ListRec {
+    double c[3], rcut2;
+    double prcut2[4];
+    double alpha[4], d[4];
+    int l, kind, nprim, more;   // more: first group of four of the primitives past the fourth
+    int row0, nrow, t0;
+    int cls;   // l | kind << 3 | (general row maps) rows << 5
+};
+static_assert(sizeof(ListRec) == 160, "ListRec layout");
+
 // Points: either a vector grid (x[i], y[i], z[i]) or a regular grid given by
 // its axes, flattened with x slowest and z fastest (orbkit/cy_grid.pyx:12-30).
 struct GridDesc {

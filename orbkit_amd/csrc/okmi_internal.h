@@ -47,11 +47,11 @@ struct OkmiBasis {
     PrimGroup* d_fgroups_s = nullptr;
     int* d_colmap = nullptr;         // [nkpad]
     // the FP64 kernels that list the shells in reach of a tile: shells by
-    // angular momentum (highest first) with output rows, and their
-    // primitives in groups of 4 (radii of OKMI_SCREEN_FUSED)
-    ShellRec* d_lshells = nullptr;
+    // angular momentum (highest first) with output rows, and the primitives
+    // past a shell's fourth in groups of 4 (radii of OKMI_SCREEN_FUSED)
+    ListRec* d_lshells = nullptr;
     PrimGroup* d_lgroups = nullptr;
-    std::vector<ShellRec> h_lshells;
+    bool standard = false;   // every shell l <= 3 with real spherical or Cartesian rows
     int nchunk = 0;
     int nkpad = 0;
     std::vector<double> h_frcut2, h_fprcut2;     // radii (squared) for OKMI_SCREEN_FUSED

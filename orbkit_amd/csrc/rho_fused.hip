@@ -14,7 +14,8 @@ struct GatherCodes {
     int c[16];
 };
 
-// out[r][p] = term[c] (+ term2[c] for second derivatives), or 2 rho for c = 0
+// out[r][p] = term[c] (+ term2[c] for second derivatives where they come in
+// halves), or 2 rho for c = 0
 __global__ void k_gather(const double* rho, const double* term, const double* term2, int64_t ld_term,
                          GatherCodes codes, double* out, int64_t ld_out, int64_t np)
 {
@@ -23,8 +24,25 @@ __global__ void k_gather(const double* rho, const double* term, const double* te
     for (int r = 0; r < codes.n; ++r) {
         const int c = codes.c[r];
         double v = c == 0 ? 2.0 * rho[p] : term[c * ld_term + p];
-        if (c >= 4) v += term2[c * ld_term + p];
+        if (c >= 4 && term2) v += term2[c * ld_term + p];
         out[r * ld_out + p] = v;
+    }
+}
+
+// C [nmo][nao] -> [nao][mpad], zero padded: one 32 x 32 block per workgroup of
+// 256 threads, through LDS
+__global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, int nao, int mpad, double* out)
+{
+    __shared__ double t[32][33];
+    const int r0 = 32 * blockIdx.x, m0 = 32 * blockIdx.y;
+    for (int i = threadIdx.x; i < 1024; i += 256) {
+        const int m = m0 + i / 32, r = r0 + i % 32;
+        t[i / 32][i % 32] = m < nmo && r < nao ? C[(int64_t)m * nao + r] : 0.0;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 1024; i += 256) {
+        const int r = r0 + i / 32, m = m0 + i % 32;
+        if (r < nao && m < mpad) out[(int64_t)r * mpad + m] = t[i % 32][i / 32];
     }
 }
 
@@ -159,40 +177,39 @@ int prepare_fused_tables(OkmiBasis* b)
     std::vector<int> colmap(nkpad, -1);
     for (size_t j = 0; j < work.size(); ++j)
         for (int r = 0; r < b->h_shells[work[j]].nrow; ++r) colmap[krow[work[j]] + r] = b->h_shells[work[j]].row0 + r;
-    // shells `list` in that order with the given radii, and their primitive groups
-    auto group_tables = [&](const std::vector<int>& list, const std::vector<double>& frc2,
-                            const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
-                            std::vector<PrimGroup>& groups) {
-        fs.assign(list.size(), ShellRec{});
-        groups.clear();
-        for (size_t j = 0; j < list.size(); ++j) {
-            const int i = list[j];
-            fs[j] = b->h_shells[i];
-            fs[j].rcut2 = frc2[i];
-            fs[j].prim0 = (int)groups.size();
-            const ShellRec& hs = b->h_shells[i];
-            // primitives by screening radius, largest first (ties keep file order)
-            std::vector<int> order(hs.nprim);
-            for (int k = 0; k < hs.nprim; ++k) order[k] = hs.prim0 + k;
-            std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return fprc2[x] > fprc2[y]; });
-            for (int q = 0; q < hs.nprim; q += 4) {
-                PrimGroup pg;
-                for (int k = 0; k < 4; ++k) {
-                    const bool used = q + k < hs.nprim;
-                    const int pi = used ? order[q + k] : 0;
-                    pg.alpha[k] = used ? b->h_prims[pi].alpha : 0.0;
-                    pg.d[k] = used ? b->h_prims[pi].d : 0.0;
-                    pg.rcut2[k] = used ? fprc2[pi] : -1.0;
-                }
-                groups.push_back(pg);
-            }
+    // the primitives of a shell by screening radius, largest first (ties keep file order)
+    auto sorted_prims = [&](const ShellRec& hs, const std::vector<double>& fprc2) {
+        std::vector<int> order(hs.nprim);
+        for (int k = 0; k < hs.nprim; ++k) order[k] = hs.prim0 + k;
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return fprc2[x] > fprc2[y]; });
+        return order;
+    };
+    // primitives q .. q + 3 of that order
+    auto prim_group = [&](const std::vector<int>& order, int q, const std::vector<double>& fprc2) {
+        PrimGroup pg;
+        for (int k = 0; k < 4; ++k) {
+            const bool used = q + k < (int)order.size();
+            const int pi = used ? order[q + k] : 0;
+            pg.alpha[k] = used ? b->h_prims[pi].alpha : 0.0;
+            pg.d[k] = used ? b->h_prims[pi].d : 0.0;
+            pg.rcut2[k] = used ? fprc2[pi] : -1.0;
         }
+        return pg;
     };
     auto tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
                       std::vector<PrimGroup>& groups, std::vector<ShellRec>& is, std::vector<ShellRec>& wsh,
                       std::vector<PrimRec>& fp) {
-        group_tables(work, frc2, fprc2, fs, groups);
-        for (size_t j = 0; j < work.size(); ++j) fs[j].row0 = krow[work[j]];
+        fs.assign(work.size(), ShellRec{});
+        groups.clear();
+        for (size_t j = 0; j < work.size(); ++j) {
+            const int i = work[j];
+            fs[j] = b->h_shells[i];
+            fs[j].row0 = krow[i];
+            fs[j].rcut2 = frc2[i];
+            fs[j].prim0 = (int)groups.size();
+            const std::vector<int> order = sorted_prims(b->h_shells[i], fprc2);
+            for (int q = 0; q < b->h_shells[i].nprim; q += 4) groups.push_back(prim_group(order, q, fprc2));
+        }
         // the same shells writing their internal rows (the many-MO and
         // staged paths stage the AO sets in the fused row order), also in
         // work order, and the primitives with these radii
@@ -211,16 +228,34 @@ int prepare_fused_tables(OkmiBasis* b)
     std::vector<PrimRec> fp, fp_s;
     tables(b->h_frcut2, b->h_fprcut2, fs, groups, is, wsh, fp);
     tables(b->h_frcut2s, b->h_fprcut2s, fs_s, groups_s, is_s, wsh_s, fp_s);
-    // by angular momentum, then by primitives (the costliest first)
+    // by class (angular momentum, kind of row map), then by primitives
     std::vector<int> by_l(b->nshell);
     for (int i = 0; i < b->nshell; ++i) by_l[i] = i;
     std::stable_sort(by_l.begin(), by_l.end(), [&](int x, int y) {
         const ShellRec &p = b->h_shells[x], &q = b->h_shells[y];
-        return p.l != q.l ? p.l > q.l : p.nprim > q.nprim;
+        if (p.l != q.l) return p.l > q.l;
+        if (p.kind != q.kind) return p.kind > q.kind;
+        if (p.nrow != q.nrow) return p.nrow > q.nrow;
+        return p.nprim > q.nprim;
     });
-    std::vector<ShellRec> ls;
+    std::vector<ListRec> ls(b->nshell);
     std::vector<PrimGroup> lgroups;
-    group_tables(by_l, b->h_frcut2, b->h_fprcut2, ls, lgroups);
+    bool standard = true;
+    for (int j = 0; j < b->nshell; ++j) {
+        const ShellRec& hs = b->h_shells[by_l[j]];
+        ListRec& r = ls[j];
+        r = ListRec{{hs.cx, hs.cy, hs.cz}, b->h_frcut2[by_l[j]], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)lgroups.size(),
+                    hs.row0, hs.nrow, hs.t0, hs.l | hs.kind << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
+        const std::vector<int> order = sorted_prims(hs, b->h_fprcut2);
+        const PrimGroup first = prim_group(order, 0, b->h_fprcut2);
+        for (int k = 0; k < 4; ++k) {
+            r.prcut2[k] = first.rcut2[k];
+            r.alpha[k] = first.alpha[k];
+            r.d[k] = first.d[k];
+        }
+        for (int q = 4; q < hs.nprim; q += 4) lgroups.push_back(prim_group(order, q, b->h_fprcut2));
+        standard = standard && hs.l <= 3 && hs.kind != SHELL_T_GENERAL;
+    }
     std::vector<ShellRec> os(b->h_shells, b->h_shells + b->nshell);
     for (int i = 0; i < b->nshell; ++i) os[i].rcut2 = b->h_frcut2[i];
     std::vector<int> padrows;
@@ -240,10 +275,10 @@ int prepare_fused_tables(OkmiBasis* b)
     if (!rc) rc = upload(&b->d_ishells_s, is_s, "rho_fused: internal-row shells (FP32 bound)");
     if (!rc) rc = upload(&b->d_wshells_s, wsh_s, "rho_fused: work-order shells (FP32 bound)");
     if (!rc) rc = upload(&b->d_fprims_s, fp_s, "rho_fused: primitives (FP32 bound)");
-    if (!rc) rc = upload(&b->d_lshells, ls, "rho_fused: shells by angular momentum");
+    if (!rc) rc = upload(&b->d_lshells, ls, "rho_fused: shells by class");
     if (!rc) rc = upload(&b->d_lgroups, lgroups, "rho_fused: their primitive groups");
     if (rc) return rc;
-    b->h_lshells = ls;
+    b->standard = standard;
     b->nchunk = nchunk;
     b->nkpad = nkpad;
     b->npadrows = (int)padrows.size();
@@ -256,6 +291,11 @@ int prepare_fused_tables(OkmiBasis* b)
 
 // Per point: up to 20 FP64 term rows; FP64 with MO norms also one row of
 // per-tile norms per 64 points (at most 64 MOs: 8 bytes per point)
+// Tiles from which the FP64 kernel takes its C transposed: reading the caller's
+// C costs a tile about 8 ns more than whole lines of C^T, the transposition
+// and its launch about 3 us.
+constexpr int64_t TRANSPOSE_TILES = 512;
+
 constexpr size_t FUSED_PT_BYTES = 20 * 8, NORM_PT_BYTES = 8;
 
 size_t okmi_fused_ws_bytes(const OkmiBasis* b, int nmo, int prec, int64_t np)
@@ -323,7 +363,9 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     double* norm_part = mo_norm ? (double*)(w + fixed + align256(FUSED_PT_BYTES * (size_t)chunk)) : nullptr;
 
     int need = 0;
-    bool direct = prec == OKMI_PREC_F64;   // every output is a first derivative, each once: written where it belongs
+    // FP64: every output a first or diagonal second derivative, each once: the
+    // kernel writes them where they belong
+    bool direct = prec == OKMI_PREC_F64;
     GatherCodes gc{};
     gc.n = nout;
     for (int r = 0; r < nout; ++r) {
@@ -331,11 +373,15 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
             okmi_set_error("The selection `drv=%d` is not valid!", drv_out[r]);
             return 1;
         }
-        if (drv_out[r] < 1 || drv_out[r] > 3 || (need >> drv_out[r] & 1)) direct = false;
+        if (drv_out[r] < 1 || drv_out[r] > 6 || (need >> drv_out[r] & 1)) direct = false;
         need |= 1 << drv_out[r];
         gc.c[r] = drv_out[r];
     }
     const bool p1 = (need & ~1) != 0, p2 = (need & (7 << 4)) != 0, p3 = (need & (7 << 7)) != 0;
+    // FP64 with diagonal second derivatives and no mixed ones: all seven AO
+    // sets in one pass, as far as the registers hold their accumulators
+    const bool p4 = prec == OKMI_PREC_F64 && p2 && !p3 && nmo <= 48;
+    if (p2 && !p4) direct = false;
     int lm = 0;   // highest angular momentum of the basis
     for (int i = 0; i < b->nshell; ++i) lm = std::max(lm, b->h_shells[i].l);
 
@@ -343,14 +389,18 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     FusedArgs a{};
     F64Args f{};
     if (prec == OKMI_PREC_F64) {
-        f.shells = b->d_lshells; f.groups = b->d_lgroups; f.nsh = b->nshell; f.T = b->d_T;
+        f.shells = b->d_lshells; f.more = b->d_lgroups; f.nsh = b->nshell; f.T = b->d_T;
         f.grid = g; f.nmo = nmo; f.nao = b->nao; f.C = d_c; f.occ = d_occ;
         f.term = term; f.term2 = term2; f.ld_term = chunk; f.need_mask = need;
         for (int c = 0; c < 10; ++c) f.term_row[c] = c;
-        f.brick = brick;
-        f.tlx = f.tly = f.tlz = 2;
-        f.nbx = (g.nx + 3) / 4; f.nby = (g.ny + 3) / 4; f.nbz = (g.nz + 3) / 4;
+        f.np = std::min(np, chunk);
+        f.set_bricks(brick);
         f.norm_part = norm_part;   // read by the first pass (rho) only
+        if (f.ntile * (1 + p2 + p3) >= TRANSPOSE_TILES) {
+            hipLaunchKernelGGL(k_transpose_c, dim3((unsigned)((b->nao + 31) / 32), (unsigned)((mpad + 31) / 32)), dim3(256),
+                               0, st, d_c, nmo, b->nao, (int)mpad, (double*)cpl);
+            f.ct = (const double*)cpl;
+        }
         if (direct) {
             f.ld_term = ld_delta;
             for (int r = 0; r < nout; ++r) f.term_row[drv_out[r]] = r;
@@ -373,25 +423,26 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
         const int64_t n = np - c0 < chunk ? np - c0 : chunk;
         a.p0 = f.p0 = p0 + c0;
         a.np = f.np = n;
+        if (!brick) f.set_bricks(false);
         a.rho = f.rho = rho + c0;
         if (direct) f.term = delta + c0;
         auto pass = [&](int ps) {
             switch (prec) {
-            case OKMI_PREC_F64: return launch_pass_f64(f, ps, (int)mpad, lm, st);
+            case OKMI_PREC_F64: return launch_pass_f64(f, ps, (int)mpad, b->standard, st);
             case OKMI_PREC_F32: return launch_pass<OKMI_PREC_F32>(a, ps, mt, lm, st);
             case OKMI_PREC_BF16X3: return launch_pass<OKMI_PREC_BF16X3>(a, ps, mt, lm, st);
             default: return launch_pass<OKMI_PREC_BF16X6>(a, ps, mt, lm, st);
             }
         };
-        int r = pass(p1 ? 1 : 0);
-        if (!r && p2) r = pass(2);
+        int r = pass(p4 ? 4 : p1 ? 1 : 0);
+        if (!r && p2 && !p4) r = pass(2);
         if (!r && p3) r = pass(3);
         if (!r && mo_norm) r = launch_norm_reduce(norm_part, brick ? nbrick : (n + PTS - 1) / PTS, (int)mpad, nmo,
                                                   mo_norm, st);
         if (r) return r;
         if (nout > 0 && !direct)
-            hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rho + c0, term, term2,
-                               chunk, gc, delta + c0, ld_delta, n);
+            hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rho + c0, term,
+                               p4 ? nullptr : term2, chunk, gc, delta + c0, ld_delta, n);
     }
     return okmi_check_launch("rho_fused");
 }
