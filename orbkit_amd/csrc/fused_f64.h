@@ -186,6 +186,54 @@ __device__ __forceinline__ void quad_rows(const RowSets<L, SPH, PASS>& rows, con
     }
 }
 
+// v = t on the lanes where on
+template <int NS>
+__device__ __forceinline__ void take(bool on, const double (&t)[NS], double (&v)[NS])
+{
+#pragma unroll
+    for (int s = 0; s < NS; ++s) v[s] = on ? t[s] : v[s];
+}
+
+// Rows of one (W = 4) or two (W = 2) standard shells left over at the end of
+// their class, each held by W lane groups: group w of a shell's W (lane's w)
+// gives row R + w to the K step, so the shell takes 1 / W of the K steps that a
+// quad with empty places would.  `row`: the shell's first C row; c: row w.
+template <int PASS, int W, int L, bool SPH, int R, int NT, int NR, int NS>
+__device__ __forceinline__ void split_rows(const RowSets<L, SPH, PASS>& rows, CWhere<NT, NR>& cw, unsigned row, int w,
+                                           const COps<NT, NR>& c, MoAcc<NT, NR, NS>& acc)
+{
+    constexpr int N = shell_rows<L, SPH>();
+    if constexpr (R < N) {
+        COps<NT, NR> next;
+        if constexpr (R + W < N) {
+            // (places past the last row repeat it)
+            cw.shell(row + R + W + (R + 2 * W <= N ? w : min(w, N - 1 - R - W)));
+            cw.load(0, next);
+        }
+        double v[NS], t[NS];
+        rows.template row<R>(v);
+        auto place = [&](auto i) {
+            constexpr int I = decltype(i)::value;
+            if constexpr (I < W) {
+                if constexpr (R + I < N) {
+                    rows.template row<R + I>(t);
+                } else {
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) t[s] = 0.0;
+                }
+                take(w == I, t, v);
+            }
+        };
+        place(std::integral_constant<int, 1>{});
+        place(std::integral_constant<int, 2>{});
+        place(std::integral_constant<int, 3>{});
+#pragma unroll
+        for (int s = 0; s < NS; ++s) mma_set(acc, c, s, v[s]);
+        __builtin_amdgcn_sched_barrier(0);
+        split_rows<PASS, W, L, SPH, R + W>(rows, cw, row, w, next, acc);
+    }
+}
+
 // Rows of four shells with general row maps (nrow each): set by set, the
 // Cartesian values through each lane's transform block
 template <int PASS, int L, int S, int NT, int NR, int NS>
@@ -333,37 +381,41 @@ __device__ __forceinline__ void store_mos(const F64Args& a, const TileWhere& W, 
     }
 }
 
-// The list's entries from s on that are of class L, KIND (for s and p shells any
-// standard kind), four at a time at the wave's points (lane: px, py, pz):
-// evaluated and contracted.  One loop per class, in the list's order: with the
-// classes as branches of a single loop the compiler moved the accumulators
+// The list's entries from s on that are of class L, KIND, at the wave's points
+// (lane: px, py, pz), evaluated and contracted: with W = 1 four at a time (three at the end), with W = 2 the two
+// and with W = 4 the one left over.  One loop per case, in the list's order: with
+// the cases as branches of a single loop the compiler moved the accumulators
 // through scratch.
-template <int PASS, int U, bool STD, int L, int KIND>
+template <int PASS, int U, bool STD, int L, int KIND, int W>
 __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* ent, int& s, int cnt, int base, double px,
                                            double py, double pz, int g, CWhere<U / 4, U % 4>& cw,
                                            typename MoSplit<PASS, U, STD>::Acc& acc)
 {
     using M = MoSplit<PASS, U, STD>;
     constexpr bool need1 = PASS == 1 || PASS == 2 || PASS == 4, need2 = PASS >= 2;
-    while (s < cnt) {
-        LiveShell e = ent[min(s + g, cnt - 1)];
-        const unsigned cls = __builtin_amdgcn_readfirstlane(e.idcls >> LIST_ID_BITS);
+    // leftovers have cases of their own (not where the rows take most registers)
+    constexpr bool split = L > 0 && KIND != SHELL_T_GENERAL && PASS != 3;
+    if constexpr (W == 1 || split) while (s < cnt) {
+        int at = min(s + g, cnt - 1);   // lane's entry
+        const unsigned idcls = ent[at].idcls, cls = __builtin_amdgcn_readfirstlane(idcls >> LIST_ID_BITS);
         const unsigned kind = cls >> 3 & 3;
-        if ((cls & 7) != L || (KIND == SHELL_T_GENERAL ? kind != SHELL_T_GENERAL
-                                                       : L > 1 ? kind != KIND : kind == SHELL_T_GENERAL)) return;
-        const bool mine = s + g < cnt && e.idcls >> LIST_ID_BITS == cls;
-        s += __builtin_popcountll(__builtin_amdgcn_ballot_w64(mine)) >> 4;
+        if ((cls & 7) != L || kind != KIND) return;
+        const bool mine = s + g < cnt && idcls >> LIST_ID_BITS == cls;
+        const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(mine)) >> 4;
+        if (W == 1 ? split && n < 3 : n != 4 / W) return;
+        const int w = g & (W - 1);
         // lanes without a shell repeat the first one with no primitive
-        const unsigned id0 = __builtin_amdgcn_readfirstlane(e.idcls), row0 = __builtin_amdgcn_readfirstlane(e.rowlive);
-        if (!mine) {
-            e.idcls = id0;
-            e.rowlive = row0 & LIST_ROW_MASK;
-        }
-        cw.shell(e.rowlive & LIST_ROW_MASK);
+        if (W > 1) at = s + g / W;
+        else if (!mine) at = s;
+        const LiveShell* e = ent + at;
+        const unsigned rowlive = e->rowlive;
+        const int live = W > 1 || mine ? rowlive >> LIST_ROW_BITS : 0;
+        s += n;
+        const unsigned row = rowlive & LIST_ROW_MASK;
+        cw.shell(row + w);
         COps<M::NT, M::NR> c;
         cw.load(0, c);
-        const ListRec* sh = a.shells + base + (e.idcls & LIST_ID_MASK);
-        const double X = px - sh->c[0], Y = py - sh->c[1], Z = pz - sh->c[2];
+        const double X = px - e->c[0], Y = py - e->c[1], Z = pz - e->c[2];
         const double rr = X * X + Y * Y + Z * Z;
         double S0 = 0.0, S1 = 0.0, S2 = 0.0;
         auto prim = [&](double alpha, double d) {
@@ -372,19 +424,19 @@ __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* en
             if constexpr (need1) S1 = fma(alpha, de, S1);
             if constexpr (need2) S2 = fma(alpha * alpha, de, S2);
         };
-        const int live = e.rowlive >> LIST_ROW_BITS;
         // as many primitives as one of the four has in reach (their radii descend)
 #pragma nounroll
         for (int q = 0; q < 4; ++q) {
             if (__builtin_amdgcn_ballot_w64(live > q) == 0) break;
-            const double alpha = sh->alpha[q], d = sh->d[q];
+            const double alpha = e->alpha[q], d = e->d[q];
             prim(alpha, live > q ? d : 0.0);
         }
-        if (__builtin_amdgcn_ballot_w64(live == 4 && sh->nprim > 4) != 0) {
+        if (__builtin_amdgcn_ballot_w64(live == 4) != 0) {   // all four in reach: those past them
+            const ListRec* sh = a.shells + base + (e->idcls & LIST_ID_MASK);
 #pragma nounroll
             for (int q = 4;; ++q) {
                 const PrimGroup* pg = a.more + sh->more + ((q - 4) >> 2);
-                const bool on = live == 4 && q < sh->nprim && e.d2 < pg->rcut2[q & 3];
+                const bool on = live == 4 && q < sh->nprim && e->d2 < pg->rcut2[q & 3];
                 if (__builtin_amdgcn_ballot_w64(on) == 0) break;
                 prim(on ? pg->alpha[q & 3] : 0.0, on ? pg->d[q & 3] : 0.0);
             }
@@ -395,10 +447,12 @@ __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* en
         if constexpr (KIND == SHELL_T_GENERAL) {
             ShellPows<L, double> P;
             P.init(X, Y, Z);
-            quad_general<PASS, L, 0>(a.T + sh->t0, (int)(cls >> 5), P, S0, S1, S2, cw, acc);
+            quad_general<PASS, L, 0>(a.T + a.shells[base + (e->idcls & LIST_ID_MASK)].t0, (int)(cls >> 5), P, S0, S1, S2, cw, acc);
         } else {
-            quad_rows<PASS, L, KIND == SHELL_T_SPHERICAL, 0>(RowSets<L, KIND == SHELL_T_SPHERICAL, PASS>(X, Y, Z, S0, S1, S2),
-                                                             cw, c, acc);
+            const RowSets<L, KIND == SHELL_T_SPHERICAL, PASS> rows(X, Y, Z, S0, S1, S2);
+            constexpr bool SPH = KIND == SHELL_T_SPHERICAL;
+            if constexpr (W > 1) split_rows<PASS, W, L, SPH, 0>(rows, cw, row, w, c, acc);
+            else quad_rows<PASS, L, SPH, 0>(rows, cw, c, acc);
         }
     }
 }
@@ -442,22 +496,27 @@ __global__ __launch_bounds__(256, (MoSplit<PASS, U, STD>::OCC)) void k_fused_f64
             t0 += LCAP;
         }
         int s = 0;
-#define OKMI_CLASS(L, KIND) class_loop<PASS, U, STD, L, KIND>(a, ent, s, cnt, base, qx, qy, qz, g, cw, acc)
+#define OKMI_LOOP(L, KIND, W) class_loop<PASS, U, STD, L, KIND, W>(a, ent, s, cnt, base, qx, qy, qz, g, cw, acc)
+#define OKMI_CLASS(L, KIND)        \
+    OKMI_LOOP(L, KIND, 1);         \
+    OKMI_LOOP(L, KIND, 2);         \
+    OKMI_LOOP(L, KIND, 4)
         if constexpr (!STD) {
             OKMI_CLASS(4, SHELL_T_CARTESIAN);
-            OKMI_CLASS(4, SHELL_T_GENERAL);
+            OKMI_LOOP(4, SHELL_T_GENERAL, 1);
         }
         OKMI_CLASS(3, SHELL_T_CARTESIAN);
         OKMI_CLASS(3, SHELL_T_SPHERICAL);
-        if constexpr (!STD) OKMI_CLASS(3, SHELL_T_GENERAL);
+        if constexpr (!STD) OKMI_LOOP(3, SHELL_T_GENERAL, 1);
         OKMI_CLASS(2, SHELL_T_CARTESIAN);
         OKMI_CLASS(2, SHELL_T_SPHERICAL);
-        if constexpr (!STD) OKMI_CLASS(2, SHELL_T_GENERAL);
+        if constexpr (!STD) OKMI_LOOP(2, SHELL_T_GENERAL, 1);
         OKMI_CLASS(1, SHELL_T_CARTESIAN);
-        if constexpr (!STD) OKMI_CLASS(1, SHELL_T_GENERAL);
-        OKMI_CLASS(0, SHELL_T_CARTESIAN);
-        if constexpr (!STD) OKMI_CLASS(0, SHELL_T_GENERAL);
+        if constexpr (!STD) OKMI_LOOP(1, SHELL_T_GENERAL, 1);
+        OKMI_LOOP(0, SHELL_T_CARTESIAN, 1);
+        if constexpr (!STD) OKMI_LOOP(0, SHELL_T_GENERAL, 1);
 #undef OKMI_CLASS
+#undef OKMI_LOOP
         if (t0 < a.nsh) __syncthreads();   // (uniform) the list is read before it is filled again
     }
     if constexpr (MO) {

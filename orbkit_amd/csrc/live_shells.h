@@ -13,10 +13,12 @@ namespace okmi_fused {
 
 // One list entry: the shell (relative to the list's base index) and its class,
 // its first AO row (C column) and its live primitives among the first four,
-// its squared distance to the tile's box.
+// its squared distance to the tile's box, and what its evaluation reads (from
+// LDS, where a load of the shell's record would be waited for).
 struct alignas(16) LiveShell {
     unsigned idcls, rowlive;
     double d2;
+    double alpha[4], d[4], c[3];
 };
 constexpr int LIST_ID_BITS = 18, LIST_ROW_BITS = 29;
 constexpr unsigned LIST_ID_MASK = (1u << LIST_ID_BITS) - 1, LIST_ROW_MASK = (1u << LIST_ROW_BITS) - 1;
@@ -57,21 +59,27 @@ __device__ __forceinline__ int append_live(const ListRec* shells, int nsh, int t
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = t0 + (int)threadIdx.x;
     bool hit = false;
-    unsigned idcls = 0, rowlive = 0;
-    double d2 = 0.0;
+    LiveShell e{};
     if ((int)threadIdx.x < LCAP && i < nsh) {
-        const ListRec& sh = shells[i];
+        const ListRec sh = shells[i];
+        double d2 = 0.0;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const double d = fmax(fmax(sbox[k] - sh.c[k], sh.c[k] - sbox[3 + k]), 0.0);
             d2 = fma(d, d, d2);
+            e.c[k] = sh.c[k];
         }
         hit = d2 < sh.rcut2;
         int live = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) live += d2 < sh.prcut2[q];
-        idcls = (unsigned)(i - base) | (unsigned)sh.cls << LIST_ID_BITS;
-        rowlive = (unsigned)sh.row0 | (unsigned)live << LIST_ROW_BITS;
+        for (int q = 0; q < 4; ++q) {
+            live += d2 < sh.prcut2[q];
+            e.alpha[q] = sh.alpha[q];
+            e.d[q] = sh.d[q];
+        }
+        e.d2 = d2;
+        e.idcls = (unsigned)(i - base) | (unsigned)sh.cls << LIST_ID_BITS;
+        e.rowlive = (unsigned)sh.row0 | (unsigned)live << LIST_ROW_BITS;
     }
     const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
     if (lane == 0) wsum[wave] = __builtin_popcountll(m);
@@ -84,7 +92,7 @@ __device__ __forceinline__ int append_live(const ListRec* shells, int nsh, int t
         n += c;
     }
     if (cnt + n > LCAP) return -1;
-    if (hit) ent[cnt + n0 + bits_below(m)] = LiveShell{idcls, rowlive, d2};
+    if (hit) ent[cnt + n0 + bits_below(m)] = e;
     return n;
 }
 

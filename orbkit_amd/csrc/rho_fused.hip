@@ -228,13 +228,17 @@ int prepare_fused_tables(OkmiBasis* b)
     std::vector<PrimRec> fp, fp_s;
     tables(b->h_frcut2, b->h_fprcut2, fs, groups, is, wsh, fp);
     tables(b->h_frcut2s, b->h_fprcut2s, fs_s, groups_s, is_s, wsh_s, fp_s);
-    // by class (angular momentum, kind of row map), then by primitives
+    // by class (angular momentum, kind of row map; real spherical s and p rows
+    // are the Cartesian ones), then by primitives
+    auto kind_of = [](const ShellRec& sh) {
+        return sh.l <= 1 && sh.kind == SHELL_T_SPHERICAL ? (int)SHELL_T_CARTESIAN : sh.kind;
+    };
     std::vector<int> by_l(b->nshell);
     for (int i = 0; i < b->nshell; ++i) by_l[i] = i;
     std::stable_sort(by_l.begin(), by_l.end(), [&](int x, int y) {
         const ShellRec &p = b->h_shells[x], &q = b->h_shells[y];
         if (p.l != q.l) return p.l > q.l;
-        if (p.kind != q.kind) return p.kind > q.kind;
+        if (kind_of(p) != kind_of(q)) return kind_of(p) > kind_of(q);
         if (p.nrow != q.nrow) return p.nrow > q.nrow;
         return p.nprim > q.nprim;
     });
@@ -245,7 +249,7 @@ int prepare_fused_tables(OkmiBasis* b)
         const ShellRec& hs = b->h_shells[by_l[j]];
         ListRec& r = ls[j];
         r = ListRec{{hs.cx, hs.cy, hs.cz}, b->h_frcut2[by_l[j]], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)lgroups.size(),
-                    hs.row0, hs.nrow, hs.t0, hs.l | hs.kind << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
+                    hs.row0, hs.nrow, hs.t0, hs.l | kind_of(hs) << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
         const std::vector<int> order = sorted_prims(hs, b->h_fprcut2);
         const PrimGroup first = prim_group(order, 0, b->h_fprcut2);
         for (int k = 0; k < 4; ++k) {
