@@ -368,6 +368,8 @@ extern "C" int okmi_basis_destroy(okmi_basis* b)
     if (b->d_colmap) (void)hipFree(b->d_colmap);
     if (b->d_lshells) (void)hipFree(b->d_lshells);
     if (b->d_lgroups) (void)hipFree(b->d_lgroups);
+    if (b->d_lshells_a) (void)hipFree(b->d_lshells_a);
+    if (b->d_lgroups_a) (void)hipFree(b->d_lgroups_a);
     delete[] b->h_shells;
     delete[] b->h_prims;
     delete[] b->h_T;
@@ -431,6 +433,16 @@ int64_t chunk_points(const okmi_basis* b, int nsets, int64_t np, size_t ws_bytes
     c &= ~(int64_t)63;
     return c;
 }
+
+// whether okmi_rho_staged's workspace holds its copy of C and a chunk
+bool staged_fits(const okmi_basis* b, const okmi_grid* g, int64_t p0, int64_t np, int nmo, int nsets, size_t ws_bytes)
+{
+    const bool brick = g->regular && p0 == 0 && np == g->nx * g->ny * g->nz;
+    const int64_t total = brick ? ((g->nx + 3) / 4) * ((g->ny + 3) / 4) * ((g->nz + 3) / 4) * 64 : np;
+    const size_t cbytes = (((size_t)nmo * b->nkpad * sizeof(double)) + 255) & ~(size_t)255;
+    return chunk_points(b, nsets, np, ws_bytes) > 0 && ws_bytes > cbytes + 256 &&
+           chunk_points(b, nsets, total, ws_bytes - cbytes - 256) > 0;
+}
 }  // namespace
 
 extern "C" size_t okmi_workspace_bytes(const okmi_basis* b, int nsets, int64_t chunk)
@@ -458,6 +470,16 @@ extern "C" int okmi_mo_eval(const okmi_basis* b, const okmi_grid* g, int64_t p0,
     }
     hipStream_t st = (hipStream_t)stream;
     const GridDesc gd = to_desc(g);
+    // the fused kernel where the workspace holds its copy of C and no code is
+    // asked for twice; otherwise AO values to memory and a product
+    int seen = 0;
+    bool once = true;
+    for (int j = 0; j < ndrv; ++j) {
+        once = once && !(seen >> drv[j] & 1);
+        seen |= 1 << drv[j];
+    }
+    if (once && b->max_nrow <= 32 && b->d_lshells_a && ws_bytes >= okmi_mo_f64_fused_bytes(b, nmo))
+        return okmi_launch_mo_f64_fused(b, gd, p0, np, drv, ndrv, d_c, nmo, d_mo, ld_mo, d_ws, st);
     for (int64_t c0 = 0; c0 < np; c0 += chunk) {
         const int64_t n = np - c0 < chunk ? np - c0 : chunk;
         int rc = okmi_launch_ao_eval(b, gd, p0 + c0, n, drv, ndrv, OKMI_F64, d_ws, chunk, (int64_t)b->nao * chunk, st);
@@ -621,6 +643,14 @@ extern "C" int okmi_rho(const okmi_basis* b, const okmi_grid* g, int64_t p0, int
     if (nmo <= 64 && b->max_nrow <= 32 && d_ws && ws_bytes >= okmi_fused_ws_bytes(mb, nmo, OKMI_PREC_F64, 64))
         return okmi_launch_rho_fused(mb, to_desc(g), p0, np, d_c, d_occ, nmo, OKMI_PREC_F64, drv_out, nout, d_rho,
                                      d_delta, ld_delta, d_mo_norm, d_ws, ws_bytes, (hipStream_t)stream);
+    // More: the same kernel over groups of MOs, each evaluating the shells in
+    // reach again (a quarter of a group's matrix time) instead of passing the AO
+    // sets through memory, when the workspace holds its copy of C.  (Workspaces
+    // that the staged path refuses stay refused.)
+    if (nmo > 64 && b->max_nrow <= 32 && b->nkpad > 0 && d_ws && staged_fits(b, g, p0, np, nmo, nsets, ws_bytes) &&
+        ws_bytes >= okmi_rho_f64_fused_min_bytes(b, nmo, drv_out, nout, d_mo_norm != nullptr))
+        return okmi_launch_rho_f64_fused(b, to_desc(g), p0, np, d_c, d_occ, nmo, drv_out, nout, d_rho, d_delta, ld_delta,
+                                         d_mo_norm, d_ws, ws_bytes, (hipStream_t)stream);
     return okmi_rho_staged(b, g, p0, np, d_c, d_occ, nmo, drv_out, nout, d_rho, d_delta, ld_delta, d_mo_norm, d_ws,
                            ws_bytes, stream);
 }

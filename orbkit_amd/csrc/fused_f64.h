@@ -128,7 +128,7 @@ template <int NT, int NR> struct CWhere {
     {
         base = (gchar*)(a.ct ? a.ct : a.C);
         ms = a.ct ? 8 : 8 * a.nao;
-        rs = a.ct ? 8 * mp : 8;
+        rs = a.ct ? 8 * a.ct_ld : 8;
         const int last = (a.ct ? mp : a.nmo) - 1;
         mt = n16 * ms;
         mtl = NR == 0 ? min(n16, last - 16 * (NT - 1)) * ms : mt;
@@ -344,18 +344,20 @@ __device__ __forceinline__ void epilogue_f64(const F64Args& a, const TileWhere& 
     int64_t p;
     const bool act = W.index(a, col * 16 + n16, p);
     if (g == 0 && act) {
-        if constexpr (Terms<PASS>::rho) a.rho[p] = T.r0;
+        // (a launch over further MOs adds to what the one before it wrote)
+        auto out = [&](double* o, double v) { *o = a.add ? *o + v : v; };
+        if constexpr (Terms<PASS>::rho) out(a.rho + p, T.r0);
 #pragma unroll
         for (int s = 1; s < NS; ++s) {
             const int code = PassCodes<PASS>::c[s];
             double v = T.t[s - 1];
             if (PASS == 4 && s > 3) v += T.u[s - 4];   // f0 f_aa + f_a^2
-            if (a.need_mask >> code & 1) a.term[a.term_row[code] * a.ld_term + p] = v;
+            if (a.need_mask >> code & 1) out(a.term + a.term_row[code] * a.ld_term + p, v);
         }
         if constexpr (PASS == 1) {
 #pragma unroll
             for (int q = 0; q < 6; ++q)
-                if (a.need_mask >> (4 + q) & 1) a.term2[(4 + q) * a.ld_term + p] = T.u[q];
+                if (a.need_mask >> (4 + q) & 1) out(a.term2 + (4 + q) * a.ld_term + p, T.u[q]);
         }
     }
 }
@@ -546,20 +548,18 @@ int launch_f64_one(const F64Args& a, hipStream_t st)
     return 0;
 }
 
-// u: groups of 4 MOs (1 .. 16)
-template <int PASS, bool STD>
-int launch_f64_u(const F64Args& a, int u, hipStream_t st)
+// One launch with the smallest of the instances U... (ascending) that holds
+// a.units groups of 4 MOs
+template <int PASS, bool STD, bool MO, int U, int... MORE>
+int launch_f64_units(const F64Args& a, hipStream_t st)
 {
-    switch (u) {
-#define OKMI_F64_CASE(U)     case U: return launch_f64_one<PASS, STD, U, false>(a, st);
-        OKMI_F64_CASE(1) OKMI_F64_CASE(2) OKMI_F64_CASE(3) OKMI_F64_CASE(4) OKMI_F64_CASE(5) OKMI_F64_CASE(6)
-        OKMI_F64_CASE(7) OKMI_F64_CASE(8) OKMI_F64_CASE(9) OKMI_F64_CASE(10) OKMI_F64_CASE(11) OKMI_F64_CASE(12)
-        OKMI_F64_CASE(13) OKMI_F64_CASE(14) OKMI_F64_CASE(15) OKMI_F64_CASE(16)
-#undef OKMI_F64_CASE
-    default: break;
+    if (a.units <= U) return launch_f64_one<PASS, STD, U, MO>(a, st);
+    if constexpr (sizeof...(MORE) > 0) {
+        return launch_f64_units<PASS, STD, MO, MORE...>(a, st);
+    } else {
+        okmi_set_error("rho_fused: no instance for %d groups of 4 MOs", a.units);
+        return 1;
     }
-    okmi_set_error("rho_fused: %d groups of 4 MOs (FP64: up to 16)", u);
-    return 1;
 }
 
 }  // namespace okmi_fused

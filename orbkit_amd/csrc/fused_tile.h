@@ -118,12 +118,15 @@ struct F64Args {
     const PrimGroup* more;
     int nsh;
     int nmo, nao;
+    int units;                // groups of 4 MOs of the instance (f64_units)
     int need_mask;
     const double* T;
     GridDesc grid;
     int64_t p0, np;
     const double* C;          // [nmo][nao]
-    const double* ct;         // [nao][MOs padded to 4], zero padded; null: C is read as it is
+    const double* ct;         // C^T, rows ct_ld doubles apart, this launch's MOs zero padded to 4; null: C is read as it is
+    int ct_ld;
+    int add;                  // 1: the launch adds its MOs' terms to the outputs
     const double* occ;        // [nmo]
     double* rho;
     double* term;             // [.][ld_term]: code c's term in row term_row[c]
@@ -853,11 +856,23 @@ int launch_pass(const FusedArgs& a, int pass, int mt, int lm, hipStream_t st)
     }
 }
 
-// FP64 kernel (rho_fused_f64.hip, compiled with FP64 MFMAs in the VGPR form);
-// mpad: MOs padded to a multiple of 4
-// standard: every shell l <= 3 with real spherical or Cartesian rows
-int launch_pass_f64(const F64Args& a, int pass, int mpad, bool standard, hipStream_t st);
-int launch_pass_f64_d2(const F64Args& a, int pass, int mpad, bool standard, hipStream_t st);
+// Launches of the FP64 kernel (fused_f64.h; instances compiled in several
+// files).  Groups of 4 MOs that a pass has an instance for, from the groups
+// asked for: every count for rho and rho with first derivatives of standard
+// bases (l <= 3, real spherical or Cartesian rows), and up to 10 for the pass of
+// seven AO sets; multiples of 4 for the others; MO values: every second count.
+inline int f64_units(int u, int pass, bool standard, bool mo)
+{
+    if (!standard || pass == 2 || pass == 3) return pass == 4 && u > 8 ? 10 : (u + 3) & ~3;
+    return mo && u > 2 ? (u + 1) & ~1 : u;
+}
+int launch_f64_p0(const F64Args& a, hipStream_t st);   // standard bases
+int launch_f64_p1(const F64Args& a, hipStream_t st);
+int launch_f64_p4(const F64Args& a, hipStream_t st);
+int launch_f64_p23(const F64Args& a, int pass, hipStream_t st);
+int launch_f64_general(const F64Args& a, int pass, hipStream_t st);   // any basis
+int launch_mo_f64(const F64Args& a, int pass, bool standard, hipStream_t st);
+
 // mo_norm[m] += sum_t part[t][m] for m < nmo (the FP64 kernel's per-tile norms)
 int launch_norm_reduce(const double* part, int64_t ntile, int mpad, int nmo, double* mo_norm, hipStream_t st);
 

@@ -51,6 +51,8 @@ struct OkmiBasis {
     // past a shell's fourth in groups of 4 (radii of OKMI_SCREEN_FUSED)
     ListRec* d_lshells = nullptr;
     PrimGroup* d_lgroups = nullptr;
+    ListRec* d_lshells_a = nullptr;   // the same with the radii of OKMI_SCREEN (MO values)
+    PrimGroup* d_lgroups_a = nullptr;
     bool standard = false;   // every shell l <= 3 with real spherical or Cartesian rows
     int nchunk = 0;
     int nkpad = 0;
@@ -146,6 +148,23 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
                           const double* d_occ, int nmo, int prec, const int* drv_out, int nout, double* rho,
                           double* delta, int64_t ld_delta, double* mo_norm, void* ws, size_t ws_bytes,
                           hipStream_t st);
+
+// bytes of the fused paths' copy of C (and occupations)
+size_t okmi_fused_c_bytes(const OkmiBasis* b, int nmo, int prec);
+// out[r][p]: density output rows from the term rows of a fused pass (term2
+// null: second derivatives come whole)
+void okmi_launch_gather(const double* rho, const double* term, const double* term2, int64_t ld_term, const int* codes,
+                        int n, double* out, int64_t ld_out, int64_t np, hipStream_t st);
+// FP64 fused density, any number of MOs (more than 64 in several launches over
+// groups of MOs); its workspace: at least the bytes for 64 points
+size_t okmi_rho_f64_fused_min_bytes(const OkmiBasis* b, int nmo, const int* drv_out, int nout, bool norms);
+int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const double* d_c,
+                              const double* d_occ, int nmo, const int* drv_out, int nout, double* rho, double* delta,
+                              int64_t ld_delta, double* mo_norm, void* ws, size_t ws_bytes, hipStream_t st);
+// FP64 MO values by the same kernel (d_ws: C transposed, okmi_mo_f64_fused_bytes)
+size_t okmi_mo_f64_fused_bytes(const OkmiBasis* b, int nmo);
+int okmi_launch_mo_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const int* drv, int ndrv,
+                             const double* d_c, int nmo, double* d_mo, int64_t ld_mo, void* ws, hipStream_t st);
 
 // many-MO density: FP32 AO sets per chunk + MFMA GEMM with density epilogue
 // (S AO sets: 1, 4, 7 or 10, the smallest holding the requested codes)

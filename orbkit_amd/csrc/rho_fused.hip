@@ -29,23 +29,6 @@ __global__ void k_gather(const double* rho, const double* term, const double* te
     }
 }
 
-// C [nmo][nao] -> [nao][mpad], zero padded: one 32 x 32 block per workgroup of
-// 256 threads, through LDS
-__global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, int nao, int mpad, double* out)
-{
-    __shared__ double t[32][33];
-    const int r0 = 32 * blockIdx.x, m0 = 32 * blockIdx.y;
-    for (int i = threadIdx.x; i < 1024; i += 256) {
-        const int m = m0 + i / 32, r = r0 + i % 32;
-        t[i / 32][i % 32] = m < nmo && r < nao ? C[(int64_t)m * nao + r] : 0.0;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 1024; i += 256) {
-        const int r = r0 + i / 32, m = m0 + i % 32;
-        if (r < nao && m < mpad) out[(int64_t)r * mpad + m] = t[i % 32][i / 32];
-    }
-}
-
 __global__ void k_pad_occ(const double* occ, int nmo, int mpad, double* out)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -242,24 +225,34 @@ int prepare_fused_tables(OkmiBasis* b)
         if (p.nrow != q.nrow) return p.nrow > q.nrow;
         return p.nprim > q.nprim;
     });
-    std::vector<ListRec> ls(b->nshell);
-    std::vector<PrimGroup> lgroups;
     bool standard = true;
-    for (int j = 0; j < b->nshell; ++j) {
-        const ShellRec& hs = b->h_shells[by_l[j]];
-        ListRec& r = ls[j];
-        r = ListRec{{hs.cx, hs.cy, hs.cz}, b->h_frcut2[by_l[j]], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)lgroups.size(),
-                    hs.row0, hs.nrow, hs.t0, hs.l | kind_of(hs) << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
-        const std::vector<int> order = sorted_prims(hs, b->h_fprcut2);
-        const PrimGroup first = prim_group(order, 0, b->h_fprcut2);
-        for (int k = 0; k < 4; ++k) {
-            r.prcut2[k] = first.rcut2[k];
-            r.alpha[k] = first.alpha[k];
-            r.d[k] = first.d[k];
+    for (int j = 0; j < b->nshell; ++j)
+        standard = standard && b->h_shells[j].l <= 3 && b->h_shells[j].kind != SHELL_T_GENERAL;
+    auto list_tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ListRec>& ls,
+                           std::vector<PrimGroup>& more) {
+        ls.resize(b->nshell);
+        for (int j = 0; j < b->nshell; ++j) {
+            const ShellRec& hs = b->h_shells[by_l[j]];
+            ListRec& r = ls[j];
+            r = ListRec{{hs.cx, hs.cy, hs.cz}, frc2[by_l[j]], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)more.size(),
+                        hs.row0, hs.nrow, hs.t0, hs.l | kind_of(hs) << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
+            const std::vector<int> order = sorted_prims(hs, fprc2);
+            const PrimGroup first = prim_group(order, 0, fprc2);
+            for (int k = 0; k < 4; ++k) {
+                r.prcut2[k] = first.rcut2[k];
+                r.alpha[k] = first.alpha[k];
+                r.d[k] = first.d[k];
+            }
+            for (int q = 4; q < hs.nprim; q += 4) more.push_back(prim_group(order, q, fprc2));
         }
-        for (int q = 4; q < hs.nprim; q += 4) lgroups.push_back(prim_group(order, q, b->h_fprcut2));
-        standard = standard && hs.l <= 3 && hs.kind != SHELL_T_GENERAL;
-    }
+    };
+    std::vector<ListRec> ls, ls_a;
+    std::vector<PrimGroup> lgroups, lgroups_a;
+    list_tables(b->h_frcut2, b->h_fprcut2, ls, lgroups);
+    std::vector<double> arc2(b->nshell), aprc2(b->nprim);   // radii of OKMI_SCREEN
+    for (int i = 0; i < b->nshell; ++i) arc2[i] = b->h_shells[i].rcut2;
+    for (int i = 0; i < b->nprim; ++i) aprc2[i] = b->h_prims[i].rcut2;
+    list_tables(arc2, aprc2, ls_a, lgroups_a);
     std::vector<ShellRec> os(b->h_shells, b->h_shells + b->nshell);
     for (int i = 0; i < b->nshell; ++i) os[i].rcut2 = b->h_frcut2[i];
     std::vector<int> padrows;
@@ -281,6 +274,8 @@ int prepare_fused_tables(OkmiBasis* b)
     if (!rc) rc = upload(&b->d_fprims_s, fp_s, "rho_fused: primitives (FP32 bound)");
     if (!rc) rc = upload(&b->d_lshells, ls, "rho_fused: shells by class");
     if (!rc) rc = upload(&b->d_lgroups, lgroups, "rho_fused: their primitive groups");
+    if (!rc) rc = upload(&b->d_lshells_a, ls_a, "mo_fused: shells by class");
+    if (!rc) rc = upload(&b->d_lgroups_a, lgroups_a, "mo_fused: their primitive groups");
     if (rc) return rc;
     b->standard = standard;
     b->nchunk = nchunk;
@@ -293,21 +288,30 @@ int prepare_fused_tables(OkmiBasis* b)
 }
 }  // namespace
 
-// Per point: up to 20 FP64 term rows; FP64 with MO norms also one row of
-// per-tile norms per 64 points (at most 64 MOs: 8 bytes per point)
-// Tiles from which the FP64 kernel takes its C transposed: reading the caller's
-// C costs a tile about 8 ns more than whole lines of C^T, the transposition
-// and its launch about 3 us.
-constexpr int64_t TRANSPOSE_TILES = 512;
-
-constexpr size_t FUSED_PT_BYTES = 20 * 8, NORM_PT_BYTES = 8;
+// Per point: up to 20 FP64 term rows
+constexpr size_t FUSED_PT_BYTES = 20 * 8;
 
 size_t okmi_fused_ws_bytes(const OkmiBasis* b, int nmo, int prec, int64_t np)
 {
     if (nmo > 64) return okmi_big_ws_bytes(b, nmo, prec, 7, np);
     size_t n = fused_fixed_bytes(b, nmo, prec) + align256(FUSED_PT_BYTES * np) + 256;
-    if (prec == OKMI_PREC_F64) n += align256(NORM_PT_BYTES * (np + 64)) + 256;
+    // FP64 with MO norms also one row of per-tile norms per 64 points (at most
+    // 64 MOs: 8 bytes per point)
+    if (prec == OKMI_PREC_F64) n += align256(8 * (np + 64)) + 256;
     return n;
+}
+
+size_t okmi_fused_c_bytes(const OkmiBasis* b, int nmo, int prec) { return fused_fixed_bytes(b, nmo, prec); }
+
+void okmi_launch_gather(const double* rho, const double* term, const double* term2, int64_t ld_term, const int* codes,
+                        int n, double* out, int64_t ld_out, int64_t np, hipStream_t st)
+{
+    if (n <= 0 || np <= 0) return;
+    GatherCodes gc{};
+    gc.n = n;
+    for (int r = 0; r < n; ++r) gc.c[r] = codes[r];
+    hipLaunchKernelGGL(k_gather, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, rho, term, term2, ld_term, gc, out,
+                       ld_out, np);
 }
 
 int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const double* d_c,
@@ -338,115 +342,71 @@ int okmi_launch_rho_fused(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     }
     int rc = prepare_fused_tables(b);
     if (rc) return rc;
-    // MOs padded to 16 (the FP32-accumulating MFMA tiles) or, for FP64, to 4
-    // (16-MO tiles plus 4-MO groups)
-    const int64_t mpad = prec == OKMI_PREC_F64 ? (nmo + 3) / 4 * 4 : mt * 16, kpad = b->nkpad;
+    if (prec == OKMI_PREC_F64)
+        return okmi_launch_rho_f64_fused(b, g, p0, np, d_c, d_occ, nmo, drv_out, nout, rho, delta, ld_delta, mo_norm, ws,
+                                         ws_bytes, st);
+    const int64_t mpad = mt * 16, kpad = b->nkpad;   // MOs padded to the MFMA tiles
     const size_t fixed = fused_fixed_bytes(b, nmo, prec);
-    // per point: the term rows, plus the per-tile MO norms (mpad doubles per
-    // 64-point tile) when wanted
-    const size_t per_pt = FUSED_PT_BYTES + (mo_norm ? NORM_PT_BYTES : 0);
-    const size_t slack = 256 + (mo_norm ? 256 + (size_t)mpad * 8 : 0);
-    if (!ws || ws_bytes < fixed + slack + per_pt * 64) {
+    if (!ws || ws_bytes < fixed + 256 + FUSED_PT_BYTES * 64) {
         okmi_set_error("rho_fused: workspace of %zu bytes is too small (need at least %zu)", ws_bytes,
-                       fixed + slack + per_pt * 64);
+                       fixed + 256 + FUSED_PT_BYTES * 64);
         return 1;
     }
-    const size_t avail = ws_bytes - fixed - slack;
+    const size_t avail = ws_bytes - fixed - 256;
     // a whole regular grid whose buffers fit is tiled in 4x4x4 bricks (the
     // faces may add tiles beyond np / 64)
-    const int64_t nbrick = ((g.nx + 3) / 4) * ((g.ny + 3) / 4) * ((g.nz + 3) / 4);
-    const bool brick = g.regular && p0 == 0 && np == g.nx * g.ny * g.nz &&
-                       FUSED_PT_BYTES * (size_t)np + (mo_norm ? (size_t)nbrick * mpad * 8 : 0) <= avail;
-    int64_t chunk = brick ? np : std::min<int64_t>(np, (int64_t)(avail / per_pt) & ~(int64_t)63);
+    const bool brick = g.regular && p0 == 0 && np == g.nx * g.ny * g.nz && FUSED_PT_BYTES * (size_t)np <= avail;
+    int64_t chunk = brick ? np : std::min<int64_t>(np, (int64_t)(avail / FUSED_PT_BYTES) & ~(int64_t)63);
     if (chunk <= 0) chunk = np;   // unreachable: avail holds 64 points
     char* w = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
     void* cpl = w;
     double* occp = (double*)(w + align256(c_elem_bytes(prec) * mpad * kpad));
     double* term = (double*)(w + fixed);
     double* term2 = term + 10 * chunk;
-    double* norm_part = mo_norm ? (double*)(w + fixed + align256(FUSED_PT_BYTES * (size_t)chunk)) : nullptr;
+
+    hipLaunchKernelGGL(k_prep_c, dim3((unsigned)((mpad * kpad + 255) / 256)), dim3(256), 0, st, d_c, nmo, b->nao,
+                       prec, mpad, kpad, (const int*)b->d_colmap, cpl);
+    hipLaunchKernelGGL(k_pad_occ, dim3(1), dim3(256), 0, st, d_occ, nmo, (int)mpad, occp);
 
     int need = 0;
-    // FP64: every output a first or diagonal second derivative, each once: the
-    // kernel writes them where they belong
-    bool direct = prec == OKMI_PREC_F64;
-    GatherCodes gc{};
-    gc.n = nout;
     for (int r = 0; r < nout; ++r) {
         if (drv_out[r] < 0 || drv_out[r] > 9) {
             okmi_set_error("The selection `drv=%d` is not valid!", drv_out[r]);
             return 1;
         }
-        if (drv_out[r] < 1 || drv_out[r] > 6 || (need >> drv_out[r] & 1)) direct = false;
         need |= 1 << drv_out[r];
-        gc.c[r] = drv_out[r];
     }
     const bool p1 = (need & ~1) != 0, p2 = (need & (7 << 4)) != 0, p3 = (need & (7 << 7)) != 0;
-    // FP64 with diagonal second derivatives and no mixed ones: all seven AO
-    // sets in one pass, as far as the registers hold their accumulators
-    const bool p4 = prec == OKMI_PREC_F64 && p2 && !p3 && nmo <= 48;
-    if (p2 && !p4) direct = false;
     int lm = 0;   // highest angular momentum of the basis
     for (int i = 0; i < b->nshell; ++i) lm = std::max(lm, b->h_shells[i].l);
 
-    // FP64 screens with the FP64 bound, the paths ending in FP32 with theirs
-    FusedArgs a{};
-    F64Args f{};
-    if (prec == OKMI_PREC_F64) {
-        f.shells = b->d_lshells; f.more = b->d_lgroups; f.nsh = b->nshell; f.T = b->d_T;
-        f.grid = g; f.nmo = nmo; f.nao = b->nao; f.C = d_c; f.occ = d_occ;
-        f.term = term; f.term2 = term2; f.ld_term = chunk; f.need_mask = need;
-        for (int c = 0; c < 10; ++c) f.term_row[c] = c;
-        f.np = std::min(np, chunk);
-        f.set_bricks(brick);
-        f.norm_part = norm_part;   // read by the first pass (rho) only
-        if (f.ntile * (1 + p2 + p3) >= TRANSPOSE_TILES) {
-            hipLaunchKernelGGL(k_transpose_c, dim3((unsigned)((b->nao + 31) / 32), (unsigned)((mpad + 31) / 32)), dim3(256),
-                               0, st, d_c, nmo, b->nao, (int)mpad, (double*)cpl);
-            f.ct = (const double*)cpl;
-        }
-        if (direct) {
-            f.ld_term = ld_delta;
-            for (int r = 0; r < nout; ++r) f.term_row[drv_out[r]] = r;
-        }
-    } else {
-        hipLaunchKernelGGL(k_prep_c, dim3((unsigned)((mpad * kpad + 255) / 256)), dim3(256), 0, st, d_c, nmo, b->nao,
-                           prec, mpad, kpad, (const int*)b->d_colmap, cpl);
-        hipLaunchKernelGGL(k_pad_occ, dim3(1), dim3(256), 0, st, d_occ, nmo, (int)mpad, occp);
-        a.shells = b->d_fshells_s;
-        a.groups = b->d_fgroups_s;
-        a.T = b->d_T; a.chunks = b->d_chunks;
-        a.grid = g; a.nao = b->nao; a.nchunk = b->nchunk;
-        a.C = cpl; a.kpad = kpad; a.mpad = mpad; a.occ = occp;
-        a.term = term; a.term2 = term2; a.ld_term = chunk; a.need_mask = need;
-        a.brick = brick;
-        a.tlx = a.tly = a.tlz = 2;
-        a.nbx = (g.nx + 3) / 4; a.nby = (g.ny + 3) / 4; a.nbz = (g.nz + 3) / 4;
-    }
+    FusedArgs a{};   // screened with the bound of the paths whose AO values end in FP32
+    a.shells = b->d_fshells_s;
+    a.groups = b->d_fgroups_s;
+    a.T = b->d_T; a.chunks = b->d_chunks;
+    a.grid = g; a.nao = b->nao; a.nchunk = b->nchunk;
+    a.C = cpl; a.kpad = kpad; a.mpad = mpad; a.occ = occp;
+    a.term = term; a.term2 = term2; a.ld_term = chunk; a.need_mask = need;
+    a.brick = brick;
+    a.tlx = a.tly = a.tlz = 2;
+    a.nbx = (g.nx + 3) / 4; a.nby = (g.ny + 3) / 4; a.nbz = (g.nz + 3) / 4;
     for (int64_t c0 = 0; c0 < np; c0 += chunk) {
         const int64_t n = np - c0 < chunk ? np - c0 : chunk;
-        a.p0 = f.p0 = p0 + c0;
-        a.np = f.np = n;
-        if (!brick) f.set_bricks(false);
-        a.rho = f.rho = rho + c0;
-        if (direct) f.term = delta + c0;
+        a.p0 = p0 + c0;
+        a.np = n;
+        a.rho = rho + c0;
         auto pass = [&](int ps) {
             switch (prec) {
-            case OKMI_PREC_F64: return launch_pass_f64(f, ps, (int)mpad, b->standard, st);
             case OKMI_PREC_F32: return launch_pass<OKMI_PREC_F32>(a, ps, mt, lm, st);
             case OKMI_PREC_BF16X3: return launch_pass<OKMI_PREC_BF16X3>(a, ps, mt, lm, st);
             default: return launch_pass<OKMI_PREC_BF16X6>(a, ps, mt, lm, st);
             }
         };
-        int r = pass(p4 ? 4 : p1 ? 1 : 0);
-        if (!r && p2 && !p4) r = pass(2);
+        int r = pass(p1 ? 1 : 0);
+        if (!r && p2) r = pass(2);
         if (!r && p3) r = pass(3);
-        if (!r && mo_norm) r = launch_norm_reduce(norm_part, brick ? nbrick : (n + PTS - 1) / PTS, (int)mpad, nmo,
-                                                  mo_norm, st);
         if (r) return r;
-        if (nout > 0 && !direct)
-            hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rho + c0, term,
-                               p4 ? nullptr : term2, chunk, gc, delta + c0, ld_delta, n);
+        okmi_launch_gather(rho + c0, term, term2, chunk, drv_out, nout, delta + c0, ld_delta, n, st);
     }
     return okmi_check_launch("rho_fused");
 }

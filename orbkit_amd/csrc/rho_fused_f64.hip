@@ -1,5 +1,5 @@
-// FP64 fused density kernel (fused_f64.h): rho, rho and first derivatives.
-#include "fused_f64.h"
+// FP64 fused density and MO values (fused_f64.h): the launch sequences.
+#include "fused_tile.h"
 
 namespace okmi_fused {
 namespace {
@@ -31,13 +31,242 @@ int launch_norm_reduce(const double* part, int64_t ntile, int mpad, int nmo, dou
     return 0;
 }
 
-int launch_pass_f64(const F64Args& a, int pass, int mpad, bool standard, hipStream_t st)
+int launch_rho_f64(F64Args a, int u, int pass, bool standard, hipStream_t st)
 {
+    a.units = f64_units(u, pass, standard, false);
+    if (!standard) return launch_f64_general(a, pass, st);
     switch (pass) {
-    case 0: return standard ? launch_f64_u<0, true>(a, mpad / 4, st) : launch_f64_u<0, false>(a, mpad / 4, st);
-    case 1: return standard ? launch_f64_u<1, true>(a, mpad / 4, st) : launch_f64_u<1, false>(a, mpad / 4, st);
-    default: return launch_pass_f64_d2(a, pass, mpad, standard, st);
+    case 0: return launch_f64_p0(a, st);
+    case 1: return launch_f64_p1(a, st);
+    case 4: return launch_f64_p4(a, st);
+    default: return launch_f64_p23(a, pass, st);
     }
 }
 
 }  // namespace okmi_fused
+
+namespace {
+
+using namespace okmi_fused;
+
+size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// C [nmo][nao] -> [nao][mpad], zero padded: one 32 x 32 block per workgroup of
+// 256 threads, through LDS
+__global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, int nao, int mpad, double* out)
+{
+    __shared__ double t[32][33];
+    const int r0 = 32 * blockIdx.x, m0 = 32 * blockIdx.y;
+    for (int i = threadIdx.x; i < 1024; i += 256) {
+        const int m = m0 + i / 32, r = r0 + i % 32;
+        t[i / 32][i % 32] = m < nmo && r < nao ? C[(int64_t)m * nao + r] : 0.0;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 1024; i += 256) {
+        const int r = r0 + i / 32, m = m0 + i % 32;
+        if (r < nao && m < mpad) out[(int64_t)r * mpad + m] = t[i % 32][i / 32];
+    }
+}
+
+// Tiles from which C is transposed first: reading the caller's C costs a tile
+// about 8 ns more than whole lines of C^T, the transposition and its launch
+// about 3 us.
+constexpr int64_t TRANSPOSE_TILES = 512;
+
+// Per point: up to 20 term rows; with MO norms one row of per-tile norms per
+// 64 points (at most 64 MOs a launch)
+constexpr size_t PT_BYTES = 20 * 8, NORM_PT_BYTES = 8;
+
+// The passes of a request, and its MOs in equal groups of at most as many as a
+// pass holds in registers: 64 at up to four AO sets, 40 at seven.
+struct Plan {
+    bool standard, p1, p2, p3, p4;
+    bool direct;            // every output a first or diagonal second derivative, each once
+    int need, groups, u;    // codes; launches over 4 u MOs each
+
+    Plan(const OkmiBasis* b, int nmo, const int* drv_out, int nout) : standard(b->standard), direct(true), need(0)
+    {
+        for (int r = 0; r < nout; ++r) {
+            const int d = drv_out[r];
+            if (d < 1 || d > 6 || (need >> d & 1)) direct = false;
+            need |= 1 << d;
+        }
+        p1 = (need & ~1) != 0;
+        p2 = (need & (7 << 4)) != 0;
+        p3 = (need & (7 << 7)) != 0;
+        // diagonal second derivatives and no mixed ones: all seven AO sets at
+        // once (bases with general row maps up to the MOs of one launch)
+        p4 = p2 && !p3 && (standard || nmo <= 40);
+        if (p2 && !p4) direct = false;
+        const int cap = p4 ? 40 : 64;
+        groups = (nmo + cap - 1) / cap;
+        u = ((nmo + groups - 1) / groups + 3) / 4;
+    }
+    int first() const { return p4 ? 4 : p1 ? 1 : 0; }
+    // MOs of a launch of the first pass, and width of C^T (the last group's
+    // padding included)
+    int64_t mp(int pass) const { return 4 * (int64_t)f64_units(u, pass, standard, false); }
+    int64_t mpt() const { return (groups - 1) * 4 * (int64_t)u + std::max(mp(first()), p2 || p3 ? mp(3) : 0); }
+    size_t c_bytes(const OkmiBasis* b, int nmo) const
+    {
+        const size_t n = align256(8 * (size_t)b->nao * mpt());
+        return nmo <= 64 ? std::max(n, okmi_fused_c_bytes(b, nmo, OKMI_PREC_F64)) : n;
+    }
+    size_t slack(bool norms) const { return 256 + (norms ? 256 + (size_t)mp(first()) * 8 : 0); }
+};
+
+F64Args basis_args(const OkmiBasis* b, const GridDesc& g, int nmo, const double* d_c)
+{
+    F64Args f{};
+    f.shells = b->d_lshells;
+    f.more = b->d_lgroups;
+    f.nsh = b->nshell;
+    f.T = b->d_T;
+    f.grid = g;
+    f.nmo = nmo;
+    f.nao = b->nao;
+    f.C = d_c;
+    for (int c = 0; c < 10; ++c) f.term_row[c] = c;
+    return f;
+}
+
+void transpose_c(const OkmiBasis* b, const double* d_c, int nmo, int64_t mpt, double* out, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_transpose_c, dim3((unsigned)((b->nao + 31) / 32), (unsigned)((mpt + 31) / 32)), dim3(256), 0, st,
+                       d_c, nmo, b->nao, (int)mpt, out);
+}
+
+}  // namespace
+
+size_t okmi_rho_f64_fused_min_bytes(const OkmiBasis* b, int nmo, const int* drv_out, int nout, bool norms)
+{
+    const Plan pl(b, nmo, drv_out, nout);
+    return pl.c_bytes(b, nmo) + pl.slack(norms) + (PT_BYTES + (norms ? NORM_PT_BYTES : 0)) * 64;
+}
+
+int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const double* d_c,
+                              const double* d_occ, int nmo, const int* drv_out, int nout, double* rho, double* delta,
+                              int64_t ld_delta, double* mo_norm, void* ws, size_t ws_bytes, hipStream_t st)
+{
+    for (int r = 0; r < nout; ++r)
+        if (drv_out[r] < 0 || drv_out[r] > 9) {
+            okmi_set_error("The selection `drv=%d` is not valid!", drv_out[r]);
+            return 1;
+        }
+    const Plan pl(b, nmo, drv_out, nout);
+    const int64_t mp = pl.mp(pl.first()), step = 4 * (int64_t)pl.u;   // MO norms of a tile; MOs of a group
+    const size_t fixed = pl.c_bytes(b, nmo), least = okmi_rho_f64_fused_min_bytes(b, nmo, drv_out, nout, mo_norm != nullptr);
+    if (!ws || ws_bytes < least) {
+        okmi_set_error("rho_fused: workspace of %zu bytes is too small (need at least %zu)", ws_bytes, least);
+        return 1;
+    }
+    // per point: the term rows, plus the per-tile MO norms (mp doubles per
+    // 64-point tile) when wanted
+    const size_t per_pt = PT_BYTES + (mo_norm ? NORM_PT_BYTES : 0);
+    const size_t avail = ws_bytes - fixed - pl.slack(mo_norm != nullptr);
+    // a whole regular grid whose buffers fit is tiled in 4x4x4 bricks (the
+    // faces may add tiles beyond np / 64); outputs written where they belong
+    // need no term rows
+    const size_t term_bytes = pl.direct ? 0 : PT_BYTES;
+    const int64_t nbrick = ((g.nx + 3) / 4) * ((g.ny + 3) / 4) * ((g.nz + 3) / 4);
+    const bool brick = g.regular && p0 == 0 && np == g.nx * g.ny * g.nz &&
+                       term_bytes * (size_t)np + (mo_norm ? (size_t)nbrick * mp * 8 : 0) <= avail;
+    int64_t chunk = brick ? np : std::min<int64_t>(np, (int64_t)(avail / per_pt) & ~(int64_t)63);
+    if (chunk <= 0) chunk = np;   // unreachable: avail holds 64 points
+    char* w = (char*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
+    double* ct = (double*)w;
+    double* term = (double*)(w + fixed);
+    double* norm_part = mo_norm ? (double*)(w + fixed + align256(term_bytes * (size_t)chunk)) : nullptr;
+
+    F64Args f = basis_args(b, g, nmo, d_c);
+    f.need_mask = pl.need;
+    f.np = std::min(np, chunk);
+    f.set_bricks(brick);
+    if (pl.groups > 1 || f.ntile * (1 + (pl.p2 && !pl.p4) + pl.p3) >= TRANSPOSE_TILES) {
+        transpose_c(b, d_c, nmo, pl.mpt(), ct, st);
+        f.ct_ld = (int)pl.mpt();
+    }
+    if (pl.direct) {
+        f.ld_term = ld_delta;
+        for (int r = 0; r < nout; ++r) f.term_row[drv_out[r]] = r;
+    } else {
+        f.term = term;
+        f.term2 = term + 10 * chunk;
+        f.ld_term = chunk;
+    }
+    for (int64_t c0 = 0; c0 < np; c0 += chunk) {
+        const int64_t n = std::min(np - c0, chunk);
+        f.p0 = p0 + c0;
+        f.np = n;
+        if (!brick) f.set_bricks(false);
+        f.rho = rho + c0;
+        if (pl.direct) f.term = delta + c0;
+        for (int gr = 0; gr < pl.groups; ++gr) {
+            const int m0 = gr * (int)step;
+            if (m0 >= nmo) break;
+            f.add = gr > 0;
+            f.nmo = std::min<int>(nmo - m0, (int)step);
+            f.C = d_c + (int64_t)m0 * b->nao;
+            f.occ = d_occ + m0;
+            if (f.ct_ld) f.ct = ct + m0;
+            f.norm_part = norm_part;   // read by the first pass (rho) only
+            int r = launch_rho_f64(f, pl.u, pl.first(), b->standard, st);
+            if (!r && pl.p2 && !pl.p4) r = launch_rho_f64(f, pl.u, 2, b->standard, st);
+            if (!r && pl.p3) r = launch_rho_f64(f, pl.u, 3, b->standard, st);
+            if (!r && mo_norm) r = launch_norm_reduce(norm_part, f.ntile, (int)mp, f.nmo, mo_norm + m0, st);
+            if (r) return r;
+        }
+        if (!pl.direct)
+            okmi_launch_gather(rho + c0, term, pl.p4 ? nullptr : f.term2, chunk, drv_out, nout, delta + c0, ld_delta, n, st);
+    }
+    return okmi_check_launch("rho_fused");
+}
+
+size_t okmi_mo_f64_fused_bytes(const OkmiBasis* b, int nmo)
+{
+    return 256 + align256(8 * (size_t)b->nao * ((nmo + 63) / 64 * 64 + 4));
+}
+
+// Codes in passes {0,x,y,z}, {0,xx,yy,zz}, {0,xy,xz,yz} (code 0 alone: {0}), MOs
+// in equal groups of at most 64.  Screened with the bound of the AO kernel
+// (OKMI_SCREEN), as MO values are wanted far from the molecule too.
+int okmi_launch_mo_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const int* drv, int ndrv,
+                             const double* d_c, int nmo, double* d_mo, int64_t ld_mo, void* ws, hipStream_t st)
+{
+    const int groups = (nmo + 63) / 64, u = ((nmo + groups - 1) / groups + 3) / 4, step = 4 * u;
+    double* ct = (double*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
+    const int64_t mpt = (groups - 1) * step + 64;   // (the widest instance's padding included)
+    transpose_c(b, d_c, nmo, mpt, ct, st);
+    F64Args f = basis_args(b, g, nmo, d_c);
+    f.shells = b->d_lshells_a;
+    f.more = b->d_lgroups_a;
+    f.ct_ld = (int)mpt;
+    f.p0 = p0;
+    f.np = np;
+    f.set_bricks(g.regular && p0 == 0 && np == g.nx * g.ny * g.nz);
+    f.ld_term = ld_mo;
+    f.ld_set = (int64_t)nmo * ld_mo;
+    int left = 0;
+    for (int j = 0; j < ndrv; ++j) {
+        left |= 1 << drv[j];
+        f.term_row[drv[j]] = j;
+    }
+    for (int pass = 0; pass <= 3; ++pass) {
+        static constexpr int codes[4] = {1, 0xf, 0x71, 0x381};
+        // code 0 by the first pass that takes a derivative, or alone
+        if (pass == 0 ? left != 1 : (left & codes[pass] & ~1) == 0) continue;
+        f.need_mask = left & codes[pass];
+        left &= ~codes[pass];
+        for (int gr = 0; gr < groups; ++gr) {
+            const int m0 = gr * step;
+            if (m0 >= nmo) break;
+            f.nmo = std::min(nmo - m0, step);
+            f.ct = ct + m0;
+            f.term = d_mo + (int64_t)m0 * ld_mo;
+            f.units = f64_units(u, pass, b->standard, true);
+            const int r = launch_mo_f64(f, pass, b->standard, st);
+            if (r) return r;
+        }
+    }
+    return okmi_check_launch("mo_eval");
+}
