@@ -189,13 +189,14 @@ __device__ __forceinline__ double fma_coef(double a, double b, double c)
     return fma(a, b, c);
 }
 
-// exp(-t) in FP64 for t >= 0, within one ulp: Cody-Waite reduction
-// -t = s - k ln2, |s| <= ln2/2 (ln2 in a high part exact in 32 bits and a low
-// part), exp(s) by the Chebyshev interpolant of degree 11 on that interval
-// (relative error below 1e-17), and 2^-k by exponent adjustment, which
-// underflows to +0.  Even and odd coefficients run in two chains: most shells
-// have one primitive in reach of a tile, so the chain of its exponential is
-// what a wave waits for.  Branch-free: t is clamped to 1e4 (+0 in FP64).
+// exp(-t) in FP64 for t >= 0, to rounding: Cody-Waite reduction -t = s - k ln2,
+// |s| <= ln2/2 (ln2 in a high part exact in 32 bits and a low part), exp(s) as
+// 1 + (s + s^2 R(s)) with R from the Chebyshev interpolant of degree 11 on that
+// interval (relative error below 2e-17; the sum's last addition leaves about half
+// an ulp), and 2^-k by exponent adjustment, which underflows to +0.  Even and odd
+// coefficients run in two chains: most shells have one primitive in reach of a
+// tile, so the chain of its exponential is what a wave waits for.  Branch-free:
+// t is clamped to 1e4 (+0 in FP64).
 __device__ __forceinline__ double gauss_f64(double t)
 {
     t = fmin(t, 1.0e4);
@@ -211,9 +212,7 @@ __device__ __forceinline__ double gauss_f64(double t)
     o = fma_coef(o, q, 0.008333333333319601);
     e = fma_coef(e, q, 0.5000000000000019);
     o = fma_coef(o, q, 0.1666666666666668);
-    e = fma_coef(e, q, 1.0);
-    o = fma_coef(o, q, 1.0);
-    return ldexp(fma(o, s, e), -(int)k);
+    return ldexp(1.0 + fma(q, fma(o, s, e), s), -(int)k);
 }
 
 // exp(-t) to FP32 accuracy for any t >= 0 given in FP64: the range reduction

@@ -8,6 +8,8 @@
 #include "okmi_internal.h"
 #include "ao_device.h"
 
+#include <type_traits>
+
 namespace {
 
 struct AoArgs {
@@ -187,7 +189,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
     // one shell for the wave's points: its rows evaluated, or zero when it is
     // out of reach (every value and derivative below the screening bound)
     auto shell = [&](const ShellRec& sh) {
-        const double d2 = __longlong_as_double(__builtin_amdgcn_readfirstlane(__double_as_longlong(box_dist2(lo, hi, sh))));
+        const double d2 = uniform(box_dist2(lo, hi, sh));
         if (d2 >= sh.rcut2) {
             if (act)
                 for (int c = 0; c < OKMI_MAX_SETS; ++c) {
@@ -230,6 +232,187 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
             for (int e = 0; e < nsh; ++e) shell(load_shell(a.wshells, cw.x + e));
         }
     }
+}
+
+// FP64 values of every shell (codes of PASS: 0 value, 1 value and first
+// derivatives, 2 and 3 value and diagonal or mixed second ones), one lane per
+// point.  The four waves of a workgroup take the same 64 points and every
+// fourth shell each (blockIdx.y: a part of the shells, where the points alone
+// would leave the chip short of waves), so that the waves in flight cover the
+// scalar load of a shell's record, which holds its first four primitives.
+// Bound by its stores: rows leave as whole 512-byte lines, non-temporal (they
+// are read back, if at all, by a later kernel).
+struct AoListArgs {
+    const ListRec* shells;      // by class, output rows, radii of OKMI_SCREEN
+    const PrimGroup* more;
+    const double* T;
+    GridDesc grid;
+    int64_t p0, np, ld, set_stride;
+    int nsh, per;               // shells; per blockIdx.y
+    int dst[4];                 // output set of the pass's AO sets, -1: not wanted
+};
+
+template <int PASS> struct AoSets { static constexpr int n = PASS == 0 ? 1 : 4; };
+
+template <int L, bool SPH, int PASS>
+__device__ __forceinline__ void ao_rows(const AoListArgs& a, double* o, bool act, double X, double Y, double Z, double S0,
+                                        double S1, double S2)
+{
+    constexpr int NS = AoSets<PASS>::n;
+    each_row<0>(RowSets<L, SPH, PASS>(X, Y, Z, S0, S1, S2), [&](int r, const double (&v)[NS]) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            if (a.dst[s] >= 0 && act) __builtin_nontemporal_store(v[s], o + a.dst[s] * a.set_stride + r * a.ld);
+    });
+}
+
+template <int L, int PASS>
+__device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& sh, double* o, bool act, double X, double Y,
+                                           double Z, double S0, double S1, double S2)
+{
+    constexpr int NS = AoSets<PASS>::n, NC = ncart(L);
+    constexpr int c1 = PASS == 1 ? 1 : PASS == 2 ? 4 : 7;
+    ShellPows<L, double> P;
+    P.init(X, Y, Z);
+    const OKMI_CONST double* T = cptr(a.T) + sh.t0;
+    auto set = [&](auto code, int s) {
+        if (a.dst[s] < 0) return;
+        double c[NC];
+        cart_all<L, decltype(code)::value, double>(P, S0, S1, S2, c);
+        for (int r = 0; r < sh.nrow; ++r) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
+            if (act) __builtin_nontemporal_store(v, o + a.dst[s] * a.set_stride + r * a.ld);
+        }
+    };
+    set(std::integral_constant<int, 0>{}, 0);
+    if constexpr (NS > 1) {
+        set(std::integral_constant<int, c1>{}, 1);
+        set(std::integral_constant<int, c1 + 1>{}, 2);
+        set(std::integral_constant<int, c1 + 2>{}, 3);
+    }
+}
+
+template <int PASS>
+__global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a, double* __restrict__ out)
+{
+    constexpr int NS = AoSets<PASS>::n;
+    constexpr bool need1 = PASS == 1 || PASS == 2, need2 = PASS >= 2;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+    const bool act = i < a.np;
+    double px, py, pz;
+    grid_point(a.grid, a.p0 + (act ? i : a.np - 1), px, py, pz);
+    double lo[3] = {px, py, pz}, hi[3] = {px, py, pz};   // the wave's bounding box
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
+            hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
+        }
+    const int end = min(a.nsh, ((int)blockIdx.y + 1) * a.per);
+    for (int s = (int)blockIdx.y * a.per + wave; s < end; s += 4) {
+        const ListRec sh = load_list(a.shells, s);
+        double d2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double d = fmax(fmax(lo[k] - sh.c[k], sh.c[k] - hi[k]), 0.0);
+            d2 = fma(d, d, d2);
+        }
+        d2 = uniform(d2);
+        double* o = out + sh.row0 * a.ld + i;
+        if (!(d2 < sh.rcut2)) {   // every value and derivative below the screening bound
+            if (act)
+                for (int q = 0; q < NS; ++q) {
+                    if (a.dst[q] < 0) continue;
+                    for (int r = 0; r < sh.nrow; ++r)
+                        __builtin_nontemporal_store(0.0, o + a.dst[q] * a.set_stride + r * a.ld);
+                }
+            continue;
+        }
+        const double X = px - sh.c[0], Y = py - sh.c[1], Z = pz - sh.c[2];
+        const double rr = X * X + Y * Y + Z * Z;
+        double S0 = 0.0, S1 = 0.0, S2 = 0.0;
+        auto prim = [&](double alpha, double d) {
+            const double de = d * gauss_f64(alpha * rr);
+            S0 += de;
+            if constexpr (need1) S1 = fma(alpha, de, S1);
+            if constexpr (need2) S2 = fma(alpha * alpha, de, S2);
+        };
+        // the primitives in reach lead (radii descend)
+        if (d2 < sh.prcut2[0]) prim(sh.alpha[0], sh.d[0]);
+        if (d2 < sh.prcut2[1]) prim(sh.alpha[1], sh.d[1]);
+        if (d2 < sh.prcut2[2]) prim(sh.alpha[2], sh.d[2]);
+        if (d2 < sh.prcut2[3]) {
+            prim(sh.alpha[3], sh.d[3]);
+            for (int q = 4; q < sh.nprim; ++q) {
+                const OKMI_CONST PrimGroup* g = cptr(a.more) + sh.more + ((q - 4) >> 2);
+                if (!(d2 < g->rcut2[q & 3])) break;
+                prim(g->alpha[q & 3], g->d[q & 3]);
+            }
+        }
+        S1 *= -2.0;
+        S2 *= 4.0;
+#define OKMI_AO_CASE(L)                                                                              \
+    case L:                                                                                          \
+        if (sh.kind == SHELL_T_GENERAL) ao_general<L, PASS>(a, sh, o, act, X, Y, Z, S0, S1, S2);     \
+        else if (L <= 3 && sh.kind == SHELL_T_SPHERICAL)                                             \
+            ao_rows<(L <= 3 ? L : 0), true, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                   \
+        else ao_rows<L, false, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                                \
+        break;
+        switch (sh.l) {
+            OKMI_AO_CASE(0) OKMI_AO_CASE(1) OKMI_AO_CASE(2) OKMI_AO_CASE(3)
+        default:
+            OKMI_AO_CASE(4)
+        }
+#undef OKMI_AO_CASE
+    }
+}
+
+// Waves that fill the chip several times over: the shells are split into parts
+// until the points give as many (small grids).
+constexpr int64_t AO_WAVES = 16384;
+
+int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const int (&first)[OKMI_MAX_SETS],
+                   double* out, int64_t ld, int64_t set_stride, hipStream_t st)
+{
+    AoListArgs a{};
+    a.shells = b->d_lshells_a;
+    a.more = b->d_lgroups_a;
+    a.T = b->d_T;
+    a.grid = g;
+    a.p0 = p0;
+    a.np = np;
+    a.ld = ld;
+    a.set_stride = set_stride;
+    a.nsh = b->nshell;
+    const int64_t blocks = (np + 63) / 64;
+    // (at least two shells per wave)
+    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>((AO_WAVES / 4 + blocks - 1) / blocks, b->nshell / 8));
+    a.per = (int)((b->nshell + parts - 1) / parts);
+    const dim3 grd((unsigned)blocks, (unsigned)((b->nshell + a.per - 1) / a.per)), blk(256);
+    bool value = first[0] >= 0;   // written by the first pass launched
+    auto pass = [&](int c1) {     // codes c1 .. c1 + 2
+        bool any = false;
+        for (int q = 0; q < 3; ++q) {
+            a.dst[1 + q] = first[c1 + q];
+            any = any || first[c1 + q] >= 0;
+        }
+        if (!any) return false;
+        a.dst[0] = value ? first[0] : -1;
+        value = false;
+        return true;
+    };
+    if (pass(1)) hipLaunchKernelGGL((k_ao_list<1>), grd, blk, 0, st, a, out);
+    if (pass(4)) hipLaunchKernelGGL((k_ao_list<2>), grd, blk, 0, st, a, out);
+    if (pass(7)) hipLaunchKernelGGL((k_ao_list<3>), grd, blk, 0, st, a, out);
+    if (value) {
+        a.dst[0] = first[0];
+        hipLaunchKernelGGL((k_ao_list<0>), grd, blk, 0, st, a, out);
+    }
+    return 0;
 }
 
 }  // namespace
@@ -284,7 +467,9 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
         width = bricks->nbk * 64;
     }
     OkmiProfScope prof("ao_eval", st);
-    for (int grp = 0; grp < 2; ++grp) {
+    const bool list = !bricks && !live && out_dtype == OKMI_F64 && shells == b->d_shells && b->d_lshells_a;
+    if (list && launch_ao_list(b, g, p0, np, first, (double*)out, ld, set_stride, st)) return 1;
+    for (int grp = 0; grp < 2 && !list; ++grp) {
         const int c0 = grp == 0 ? 0 : 4, c1 = grp == 0 ? 4 : OKMI_MAX_SETS;
         bool any = false;
         for (int c = 0; c < OKMI_MAX_SETS; ++c) {

@@ -194,17 +194,6 @@ __device__ __forceinline__ void tile_point(const FusedArgs& a, int64_t tile, int
     }
 }
 
-// value known to be equal in all lanes -> scalar register, so that the
-// compiler treats everything derived from it as wave-uniform (scalar loads
-// of the shell tables, scalar branches)
-__device__ __forceinline__ double uniform(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readfirstlane((int)b);
-    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 __device__ __forceinline__ double wave_min(double v)
 {
 #pragma unroll

@@ -142,6 +142,27 @@ __device__ __forceinline__ PrimGroup load_group(const PrimGroup* base, int i)
     return g;
 }
 
+__device__ __forceinline__ ListRec load_list(const ListRec* base, int i)
+{
+    constexpr int NW = sizeof(ListRec) / 8;
+    struct Words { uint64_t w[NW]; } v;
+    const OKMI_CONST uint64_t* src = (const OKMI_CONST uint64_t*)(cptr(base) + i);
+#pragma unroll
+    for (int k = 0; k < NW; ++k) v.w[k] = src[k];
+    return __builtin_bit_cast(ListRec, v);
+}
+
+// value known to be equal in all lanes -> scalar register, so that the
+// compiler treats everything derived from it as wave-uniform (scalar loads
+// of the shell tables, scalar branches)
+__device__ __forceinline__ double uniform(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b);
+    const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
 __device__ __forceinline__ int2 load_int2(const int2* base, int i)
 {
     const OKMI_CONST int* p = (const OKMI_CONST int*)cptr(base) + 2 * i;
