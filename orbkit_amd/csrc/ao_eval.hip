@@ -240,8 +240,11 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
 // fourth shell each (blockIdx.y: a part of the shells, where the points alone
 // would leave the chip short of waves), so that the waves in flight cover the
 // scalar load of a shell's record, which holds its first four primitives.
-// Bound by its stores: rows leave as whole 512-byte lines, non-temporal (they
-// are read back, if at all, by a later kernel).
+// Bound by its stores (3.35 GB in 608 us, 5.5 TB/s, against 6.9 of a fill).  They
+// go through L2: a row of an odd number of points begins inside a line, whose
+// two parts two waves write, and non-temporal stores sent the parts to memory one
+// by one (126,362 points x 162 rows: 68 us non-temporal, 42 through L2; rows of
+// whole lines, 400 x 4 x 261,568: 631 and 608 us).
 struct AoListArgs {
     const ListRec* shells;      // by class, output rows, radii of OKMI_SCREEN
     const PrimGroup* more;
@@ -262,7 +265,7 @@ __device__ __forceinline__ void ao_rows(const AoListArgs& a, double* o, bool act
     each_row<0>(RowSets<L, SPH, PASS>(X, Y, Z, S0, S1, S2), [&](int r, const double (&v)[NS]) {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
-            if (a.dst[s] >= 0 && act) __builtin_nontemporal_store(v[s], o + a.dst[s] * a.set_stride + r * a.ld);
+            if (a.dst[s] >= 0 && act) o[a.dst[s] * a.set_stride + r * a.ld] = v[s];
     });
 }
 
@@ -283,7 +286,7 @@ __device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& s
             double v = 0.0;
 #pragma unroll
             for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
-            if (act) __builtin_nontemporal_store(v, o + a.dst[s] * a.set_stride + r * a.ld);
+            if (act) o[a.dst[s] * a.set_stride + r * a.ld] = v;
         }
     };
     set(std::integral_constant<int, 0>{}, 0);
@@ -327,8 +330,7 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a
             if (act)
                 for (int q = 0; q < NS; ++q) {
                     if (a.dst[q] < 0) continue;
-                    for (int r = 0; r < sh.nrow; ++r)
-                        __builtin_nontemporal_store(0.0, o + a.dst[q] * a.set_stride + r * a.ld);
+                    for (int r = 0; r < sh.nrow; ++r) o[a.dst[q] * a.set_stride + r * a.ld] = 0.0;
                 }
             continue;
         }
