@@ -25,10 +25,10 @@ struct AoArgs {
     int dst[OKMI_MAX_SETS];    // output set of derivative code c, -1: not written by this launch
     // brick mode (regular grids): wave w of the launch takes brick bk0 + w
     // (4x4x4 points, z fastest) of the nbx x nby x nbz bricks and writes
-    // columns 64 w + lane; lanes of a brick outside the grid repeat its
+    // columns tile_stride w + lane (64: whole rows); lanes of a brick outside the grid repeat its
     // nearest grid point, so every column of the nbk bricks is written
     int brick;
-    int64_t bk0, nbk, nbx, nby, nbz;
+    int64_t bk0, nbk, nbx, nby, nbz, tile_stride;
     // optional live-chunk mask (AoLiveMask): the wave walks only the shells
     // of its tile's live chunks (chunk table and work-ordered shells of the
     // fused layout); null: every shell of `shells`
@@ -169,7 +169,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         iy = iy < g.ny ? iy : g.ny - 1;
         iz = iz < g.nz ? iz : g.nz - 1;
         act = wb < a.nbk;
-        i = wb * 64 + lane;
+        i = wb * a.tile_stride + lane;
         px = g.x[ix]; py = g.y[iy]; pz = g.z[iz];
     } else {
         i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -464,6 +464,7 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
         if (bricks->nbk <= 0) return 0;
         a.brick = 1;
         a.bk0 = bricks->bk0; a.nbk = bricks->nbk;
+        a.tile_stride = bricks->tile_stride;
         a.nbx = bricks->nbx; a.nby = bricks->nby; a.nbz = bricks->nbz;
         grd = dim3((unsigned)((bricks->nbk + 3) / 4));
         width = bricks->nbk * 64;

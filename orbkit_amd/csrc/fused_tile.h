@@ -95,21 +95,6 @@ struct FusedArgs {
     double* norm_part;        // FP64 kernel: per tile sum_p Phi_m(p)^2, [tile][mpad] (null: not wanted)
 };
 
-// n / d for n < 2^31 by a multiplication (all scalar instructions; a division
-// of wave-uniform integers is a dozen vector ones)
-struct FastDiv {
-    unsigned d, m, s;
-    void set(unsigned div)
-    {
-        d = div;
-        int l = 0;
-        while (((uint64_t)1 << l) < div) ++l;
-        m = l ? (unsigned)((((uint64_t)1 << (31 + l)) + div - 1) / div) : 0;
-        s = l ? l - 1 : 0;
-    }
-    __device__ __forceinline__ unsigned div(unsigned n) const { return d == 1 ? n : __umulhi(n, m) >> s; }
-};
-
 // Arguments of the FP64 kernel (fused_f64.h): the shells one by one (sorted by
 // angular momentum, row0 = C column), C and the occupations as the caller gave
 // them.

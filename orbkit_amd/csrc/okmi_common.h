@@ -183,3 +183,18 @@ __host__ __device__ constexpr int cart_exp(int l, int c, int axis)
     int v = l == 0 ? t0[c] : l == 1 ? t1[c] : l == 2 ? t2[c] : l == 3 ? t3[c] : t4[c];
     return axis == 0 ? v / 100 : axis == 1 ? (v / 10) % 10 : v % 10;
 }
+
+// n / d for n < 2^31 by a multiplication (all scalar instructions; a division
+// of wave-uniform integers is a dozen vector ones)
+struct FastDiv {
+    unsigned d, m, s;
+    void set(unsigned div)
+    {
+        d = div;
+        int l = 0;
+        while (((uint64_t)1 << l) < div) ++l;
+        m = l ? (unsigned)((((uint64_t)1 << (31 + l)) + div - 1) / div) : 0;
+        s = l ? l - 1 : 0;
+    }
+    __device__ __forceinline__ unsigned div(unsigned n) const { return d == 1 ? n : __umulhi(n, m) >> s; }
+};

@@ -73,9 +73,11 @@ int okmi_launch_ao_eval(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64
 
 // the same with explicit shell/primitive tables (e.g. the fused screening
 // radii) and, for regular grids, brick order: bricks [bk0, bk0 + nbk) of
-// nbx x nby x nbz 4x4x4 bricks, column 64 (b - bk0) + lane
+// nbx x nby x nbz 4x4x4 bricks, column 64 (b - bk0) + lane; with a tile stride
+// (one set), brick bk0 + t's 64 columns lie at t * tile_stride instead of 64 t
 struct AoBricks {
     int64_t bk0, nbk, nbx, nby, nbz;
+    int64_t tile_stride = 64;
 };
 // With the shells in the fused row order (d_ishells): per tile of 64 << shift
 // columns, bit c of mask[tile * words + c / 64] marks chunk c live; a shell

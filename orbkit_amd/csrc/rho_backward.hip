@@ -73,15 +73,14 @@ __global__ void k_transpose(const R* C, int nmo, int nao, R* CT)
     CT[k * nmo + m] = C[i];
 }
 
-// B[i][p] = 2 occ_i g(p) Phi[i][p] for p < np, 0 for np <= p < nfill
-template <typename R>
-__global__ void k_bmat(const R* Phi, const R* occ, const R* g, int nmo, int64_t np, int64_t nfill, int64_t ld, R* B)
-{
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nfill) return;
-    const R gp = p < np ? R(2) * g[p] : R(0);
-    for (int i = 0; i < nmo; ++i) B[i * ld + p] = p < np ? occ[i] * gp * Phi[i * ld + p] : R(0);
-}
+// Element (row, p) of a matrix over points at row * `row` + (p >> 6) * `tile`
+// + (p & 63): rows of `ld` points are {ld, 64}, 64-point tiles of nr whole rows
+// {64, 64 nr}.  The matrices that only these kernels touch are held in tiles: a
+// wave's work is a tile or the tiles of a range, whose rows then lie together
+// (rows of a 512,000-point chunk lie 4 MB apart, a page of its own per row).
+struct Pitch {
+    int64_t row, tile;
+};
 
 // W (M x K, row-major) packed as MFMA A operands: Wp[t][s][l] = W[16t +
 // l%16][4s + l/16] for M tile t and K step s, zero outside W, so that a
@@ -98,6 +97,38 @@ __global__ void k_pack_w(const R* W, int M, int K, R* Wp)
     const int m = 16 * t + (l & 15), k = 4 * st + (l >> 4);
     Wp[i] = (m < M && k < K) ? W[(int64_t)m * K + k] : R(0);
 }
+
+// Output scaling of a product: out[m][p] * 2 occ[m] g[p] for p < np and 0 from
+// np on (B from Phi as it leaves the accumulators; a pass of its own took 53 us
+// over 40 x 512,000 FP64 values); occ null: the product itself.
+template <typename R>
+struct ColScale {
+    typedef typename Mfma<R>::v4 V;
+    const R* occ;
+    const R* g;
+    int64_t np;
+    // the factors 2 g of points p .. p + 3 (g may start at any element)
+    __device__ __forceinline__ V load(int64_t p) const
+    {
+        V v{0, 0, 0, 0};
+        if (occ) {
+            const int64_t e = np - 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = R(2) * g[p + j < e ? p + j : e];
+        }
+        return v;
+    }
+    // row m of points p .. p + 3, left = np - p
+    __device__ __forceinline__ V apply(int m, const V& gp, int64_t left, V v) const
+    {
+        if (occ) {
+            const R o = occ[m];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = j < left ? o * gp[j] * v[j] : R(0);
+        }
+        return v;
+    }
+};
 
 // out[m][p] = sum_k W[m][k] X[k][p] for m < M and the points of [0, npad)
 // (npad a multiple of 64, <= the row strides; X rows 16-byte aligned for
@@ -119,9 +150,9 @@ __global__ void k_pack_w(const R* W, int M, int K, R* Wp)
 //           chunk (MG = 2; G = C^T B: the other rows are never read).
 template <typename R, int MG, int MODE>
 __global__ __launch_bounds__(256, 2) void k_gemm_nn(const R* __restrict__ Wp, int M, int K,
-                                                    const R* __restrict__ X, int64_t ldx, int64_t npad,
-                                                    R* __restrict__ out, int64_t ldo, const int* __restrict__ live,
-                                                    const int* __restrict__ lcount, int nchunk)
+                                                    const R* __restrict__ X, Pitch px, int64_t npad,
+                                                    R* __restrict__ out, Pitch po, const int* __restrict__ live,
+                                                    const int* __restrict__ lcount, int nchunk, ColScale<R> cs)
 {
     static_assert(MODE != 2 || MG == 2, "MODE 2 computes the two M tiles of one chunk per group");
     typedef typename Mfma<R>::v4 V;
@@ -131,7 +162,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn(const R* __restrict__ Wp, in
     const int64_t tile = (int64_t)blockIdx.x * 4 + wave;
     const int64_t p0 = tile * 64;
     if (p0 >= npad) return;
-    const R* xp = X + p0 + 4 * r;
+    const R* xp = X + tile * px.tile + 4 * r;
+    R* op = out + tile * po.tile + 4 * r;
+    const V gp = cs.load(p0 + 4 * r);
+    const int64_t left = cs.np - (p0 + 4 * r);
     const int nmt = (M + 15) / 16, nks = (K + 3) / 4;
     const int* lst = MODE ? live + tile * nchunk : nullptr;
     const int nlive = MODE ? __builtin_amdgcn_readfirstlane(lcount[tile]) : 0;
@@ -165,7 +199,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn(const R* __restrict__ Wp, in
         // load in flight.
         auto load = [&](int st, V& xv, R (&wv)[MG]) {
             const int ks = kstep(st);
-            xv = *(const V*)(xp + (int64_t)min(4 * ks + q, K - 1) * ldx);
+            xv = *(const V*)(xp + (int64_t)min(4 * ks + q, K - 1) * px.row);
 #pragma unroll
             for (int mt = 0; mt < MG; ++mt) {
                 const int t = min(g0 + mt, nmt - 1);
@@ -203,8 +237,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn(const R* __restrict__ Wp, in
             for (int i = 0; i < 4; ++i) {
                 const int m = (g0 + mt) * 16 + Mfma<R>::row(i, q);
                 if (m < M)
-                    *(V*)(out + (int64_t)m * ldo + p0 + 4 * r) =
-                        V{acc[mt][0][i], acc[mt][1][i], acc[mt][2][i], acc[mt][3][i]};
+                    *(V*)(op + (int64_t)m * po.row) =
+                        cs.apply(m, gp, left, V{acc[mt][0][i], acc[mt][1][i], acc[mt][2][i], acc[mt][3][i]});
             }
     }
     };
@@ -219,9 +253,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn(const R* __restrict__ Wp, in
 // MODE 2: the M tiles of the tile's live chunks (MG = 2).
 template <typename R, int MG, int MODE, int KS>
 __global__ __launch_bounds__(256, 2) void k_gemm_nn_xr(const R* __restrict__ Wp, int M, int K,
-                                                       const R* __restrict__ X, int64_t ldx, int64_t npad,
-                                                       R* __restrict__ out, int64_t ldo, const int* __restrict__ live,
-                                                       const int* __restrict__ lcount, int nchunk)
+                                                       const R* __restrict__ X, Pitch px, int64_t npad,
+                                                       R* __restrict__ out, Pitch po, const int* __restrict__ live,
+                                                       const int* __restrict__ lcount, int nchunk, ColScale<R> cs)
 {
     static_assert(MODE != 2 || MG == 2, "MODE 2 computes the two M tiles of one chunk per group");
     typedef typename Mfma<R>::v4 V;
@@ -230,12 +264,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn_xr(const R* __restrict__ Wp,
     const int64_t tile = (int64_t)blockIdx.x * 4 + wave;
     const int64_t p0 = tile * 64;
     if (p0 >= npad) return;
-    const R* xp = X + p0 + 4 * r;
+    const R* xp = X + tile * px.tile + 4 * r;
+    R* op = out + tile * po.tile + 4 * r;
+    const V gp = cs.load(p0 + 4 * r);
+    const int64_t left = cs.np - (p0 + 4 * r);
     const int nmt = (M + 15) / 16, nks = (K + 3) / 4;
     V xr[KS];
 #pragma unroll
     for (int st = 0; st < KS; ++st)
-        xr[st] = st < nks ? *(const V*)(xp + (int64_t)min(4 * st + q, K - 1) * ldx) : V{0, 0, 0, 0};
+        xr[st] = st < nks ? *(const V*)(xp + (int64_t)min(4 * st + q, K - 1) * px.row) : V{0, 0, 0, 0};
     const int* lst = MODE ? live + tile * nchunk : nullptr;
     const int ngroup = MODE == 2 ? __builtin_amdgcn_readfirstlane(lcount[tile]) : (nmt + MG - 1) / MG;
     // the list's first 128 entries held across the lanes, read with readlane;
@@ -289,8 +326,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn_xr(const R* __restrict__ Wp,
             for (int i = 0; i < 4; ++i) {
                 const int m = (g0 + mt) * 16 + Mfma<R>::row(i, q);
                 if (m < M)
-                    *(V*)(out + (int64_t)m * ldo + p0 + 4 * r) =
-                        V{acc[mt][0][i], acc[mt][1][i], acc[mt][2][i], acc[mt][3][i]};
+                    *(V*)(op + (int64_t)m * po.row) =
+                        cs.apply(m, gp, left, V{acc[mt][0][i], acc[mt][1][i], acc[mt][2][i], acc[mt][3][i]});
             }
     }
     };
@@ -304,23 +341,24 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nn_xr(const R* __restrict__ Wp,
 // read from HBM once; the waves of one point range run on one XCD (blocks
 // are dealt to the 8 XCDs round-robin: range s takes blocks with index
 // % 8 == s % 8), where they share that range's B rows through the XCD's L2.
+// A range is every nsplit-th tile of 64 points, rotated from one to the next
+// (tile j nsplit + (s + j phase) mod nsplit): neighbouring tiles, whose live
+// chunks are alike, go to different waves, so that the waves end together.
 // The K index of lane (r = l%16, q = l/16) in MFMA j of a 16-point step is
 // 4q + j, so that each lane reads 4 consecutive points (one vector load) per
-// row.  Rows are padded with zeros up to a multiple of 16 points (krange a
-// multiple of 16, rows aligned to 4 elements); the rows of the next step are
-// loaded while a step is multiplied.  The partials are written (no atomics)
-// and summed in FP64 in a fixed order by k_reduce_dc.  With `mask` (rows in
-// the fused order, points in 64-point tiles with live-chunk masks
-// mask[tile][nw]) the rows of a tile's dead chunks are not read: they count
-// as zero (their values are below the screening bound and were not
-// evaluated), and a step with both of the wave's chunks dead is skipped.
-constexpr int NT = 4;
+// row; the rows of the next step are loaded while a step is multiplied.  The
+// partials are written (no atomics) and summed in FP64 in a fixed order by
+// k_reduce_dc.  With `mask` (rows in the fused order, live-chunk masks
+// mask[tile][nw]) the wave, whose AO tile is one chunk, takes only the tiles
+// where that chunk is live, found 64 at a time by its lanes: the rows of dead
+// chunks were not evaluated and count as zero.
+constexpr int NT = 2;
 template <typename R, int MG>
-__global__ __launch_bounds__(64, 2) void k_gemm_tn(const R* __restrict__ B, int nmo, const R* __restrict__ A, int nao,
-                                                int64_t kend, int64_t ld, int64_t krange, int nsplit,
-                                                R* __restrict__ part, const unsigned long long* __restrict__ mask,
-                                                int nw, int nchunk)
+__global__ __launch_bounds__(64, 3) void k_gemm_tn(const R* __restrict__ B, Pitch pb, int nmo, const R* __restrict__ A,
+                                                   Pitch pa, int nao, int npt, int nsplit, R* __restrict__ part,
+                                                   const unsigned long long* __restrict__ mask, int nw)
 {
+    static_assert(NT == 2, "the AO tile is a 32-row chunk");
     typedef typename Mfma<R>::v4 V;
     const int ntile = (nao + 16 * NT - 1) / (16 * NT);
     const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -329,69 +367,80 @@ __global__ __launch_bounds__(64, 2) void k_gemm_tn(const R* __restrict__ B, int 
     const int lane = threadIdx.x;
     const int r = lane & 15, q = lane >> 4;
     const int n0 = t * (16 * NT);
-    const int64_t k0 = (int64_t)split * krange;
-    const int64_t k1 = min(kend, k0 + krange);
-    const V* ap[NT];
-    bool nrow[NT];
+    const int nj = (npt + nsplit - 1) / nsplit;
+    const int phase = (int)(((int64_t)nsplit * 159) >> 8);   // about 0.62 nsplit
+    auto tile_of = [&](int j) { return j * nsplit + (int)((unsigned)(split + j * phase) % (unsigned)nsplit); };
+    const R* ap[NT];
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-        nrow[u] = n0 + 16 * u + r < nao;
-        ap[u] = (const V*)(A + (int64_t)(nrow[u] ? n0 + 16 * u + r : 0) * ld + 4 * q);
+        // rows past nao / nmo read row 0: they only reach accumulator columns /
+        // rows that are not stored
+        const int n = n0 + 16 * u + r;
+        ap[u] = A + (n < nao ? n : 0) * pa.row + 4 * q;
     }
     R* out = part + (int64_t)split * nmo * nao;
     const int nmt = (nmo + 15) / 16;
     for (int g0 = 0; g0 < nmt; g0 += MG) {
-        const V* bp[MG];
-        bool mrow[MG];
+        const R* bp[MG];
 #pragma unroll
         for (int mt = 0; mt < MG; ++mt) {
             const int m = (g0 + mt) * 16 + r;
-            mrow[mt] = m < nmo;
-            bp[mt] = (const V*)(B + (int64_t)(mrow[mt] ? m : 0) * ld + 4 * q);
+            bp[mt] = B + (m < nmo ? m : 0) * pb.row + 4 * q;
         }
         V acc[MG][NT];
 #pragma unroll
         for (int mt = 0; mt < MG; ++mt)
 #pragma unroll
             for (int u = 0; u < NT; ++u) acc[mt][u] = V{0, 0, 0, 0};
-        // the next step's rows are loaded while this step is multiplied
-        V nb[MG], na[NT];
-        bool nany = true;
-        auto load = [&](int64_t k) {
-            bool lv[2] = {true, true};   // the wave's two 32-row chunks live in this point tile
-            if (mask) {
-                const unsigned long long* mrow = mask + (k >> 6) * nw;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int c = (n0 >> 5) + h;
-                    lv[h] = c < nchunk && ((mrow[c >> 6] >> (c & 63)) & 1);
-                }
+        int jb = -64, tl = 0;
+        unsigned long long bits = 0;
+        auto next = [&]() {   // the range's next live tile, -1: none
+            while (!bits) {
+                jb += 64;
+                if (jb >= nj) return -1;
+                const int j = jb + lane;
+                tl = tile_of(j);
+                bool lv = j < nj && tl < npt;
+                if (lv && mask) lv = (mask[(int64_t)tl * nw + (t >> 6)] >> (t & 63)) & 1;
+                bits = __builtin_amdgcn_ballot_w64(lv);
             }
-            nany = lv[0] || lv[1];
-            if (nany)
-#pragma unroll
-                for (int mt = 0; mt < MG; ++mt) nb[mt] = bp[mt][k >> 2];
-#pragma unroll
-            for (int u = 0; u < NT; ++u) na[u] = lv[u >> 1] ? ap[u][k >> 2] : V{0, 0, 0, 0};
+            const int j = __builtin_ctzll(bits);
+            bits &= bits - 1;
+            return (int)__builtin_amdgcn_readlane(tl, j);
         };
-        if (k0 < k1) load(k0);
-        for (int64_t k = k0; k < k1; k += 16) {
-            // rows past nmo / nao read row 0: they only reach accumulator
-            // rows / columns that are not stored
-            V vb[MG], va[NT];
+        V nb[MG], na[NT];
+        auto load = [&](int tile, int sub) {
+            const int64_t oa = tile * pa.tile + 16 * sub, ob = tile * pb.tile + 16 * sub;
 #pragma unroll
-            for (int mt = 0; mt < MG; ++mt) vb[mt] = nb[mt];
+            for (int mt = 0; mt < MG; ++mt) nb[mt] = *(const V*)(bp[mt] + ob);
 #pragma unroll
-            for (int u = 0; u < NT; ++u) va[u] = na[u];
-            const bool any = nany;
-            if (k + 16 < k1) load(k + 16);
-            if (!any) continue;
+            for (int u = 0; u < NT; ++u) na[u] = *(const V*)(ap[u] + oa);
+        };
+        int tile = next();
+        if (tile >= 0) load(tile, 0);
+        while (tile >= 0) {
+            int after = -1;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int sub = 0; sub < 4; ++sub) {
+                V vb[MG], va[NT];
 #pragma unroll
-                for (int mt = 0; mt < MG; ++mt)
+                for (int mt = 0; mt < MG; ++mt) vb[mt] = nb[mt];
 #pragma unroll
-                    for (int u = 0; u < NT; ++u) acc[mt][u] = Mfma<R>::mac(vb[mt][j], va[u][j], acc[mt][u]);
+                for (int u = 0; u < NT; ++u) va[u] = na[u];
+                if (sub < 3) {
+                    load(tile, sub + 1);
+                } else {
+                    after = next();
+                    load(after >= 0 ? after : tile, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int mt = 0; mt < MG; ++mt)
+#pragma unroll
+                        for (int u = 0; u < NT; ++u) acc[mt][u] = Mfma<R>::mac(vb[mt][j], va[u][j], acc[mt][u]);
+            }
+            tile = after;
         }
 #pragma unroll
         for (int mt = 0; mt < MG; ++mt)
@@ -405,24 +454,36 @@ __global__ __launch_bounds__(64, 2) void k_gemm_tn(const R* __restrict__ B, int 
     }
 }
 
-// dC[e] += sum_s part[s][e] for e < n over s = 0 .. nsplit - 1 in FP64, in
-// a fixed order: eight interleaved partial sums (s mod 8, eight independent
-// loads in flight per thread), then combined in index order
-template <typename R>
-__global__ void k_reduce_dc(const R* part, int nsplit, int64_t n, R* dC)
+// Sum over s < ns of part[s * n + c] in FP64, in a fixed order, by a block of 256
+// threads: W columns from c0, each by 256 / W threads (partial t takes s = t,
+// t + 256 / W, ...), whose sums thread (column, 0) adds in order and returns.
+// One thread per column alone waits for ns loads in turn: 50 us for 700 columns
+// x 125.
+template <int W, typename R>
+__device__ __forceinline__ double column_sum(const R* part, int ns, int64_t n, int64_t c0)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    int s = 0;
-    for (; s + 8 <= nsplit; s += 8)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] += (double)part[(int64_t)(s + j) * n + e];
-    for (int j = 0; s + j < nsplit; ++j) v[j] += (double)part[(int64_t)(s + j) * n + e];
+    constexpr int P = 256 / W;
+    __shared__ double red[P][W];
+    const int x = threadIdx.x % W, y = threadIdx.x / W;
+    double v = 0.0;
+    if (c0 + x < n)
+        for (int s = y; s < ns; s += P) v += (double)part[s * n + c0 + x];
+    red[y][x] = v;
+    __syncthreads();
     double t = 0.0;
+    if (y == 0)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) t += v[j];
-    dC[e] = (R)((double)dC[e] + t);
+        for (int p = 0; p < P; ++p) t += red[p][x];
+    return t;
+}
+
+// dC[e] += sum_s part[s][e] for e < n over s < nsplit
+template <typename R>
+__global__ __launch_bounds__(256) void k_reduce_dc(const R* part, int nsplit, int64_t n, R* dC)
+{
+    const int64_t e = (int64_t)blockIdx.x * 32 + threadIdx.x;
+    const double t = column_sum<32>(part, nsplit, n, (int64_t)blockIdx.x * 32);
+    if (threadIdx.x < 32 && e < n) dC[e] = (R)((double)dC[e] + t);
 }
 
 __device__ __forceinline__ double wave_sum(double v)
@@ -437,20 +498,20 @@ __device__ __forceinline__ double wave_sum(double v)
 // lanes of a brick outside the grid repeating its nearest grid point.
 struct BwdBricks {
     int on;
-    int64_t bk0, nbx, nby, nbz, nx, ny, nz;
+    unsigned bk0;        // bricks count below 2^31 (64 points of dL/drho each)
+    FastDiv nby, nbz;
+    int64_t nx, ny, nz;
 };
 
-// grid indices of column `col`; returns whether the point lies in the grid
-__device__ __forceinline__ bool brick_index(const BwdBricks& bm, int64_t col, int64_t& ix, int64_t& iy, int64_t& iz)
+// grid indices of lane l of the chunk's brick `tile`; returns whether the point
+// lies in the grid
+__device__ __forceinline__ bool brick_index(const BwdBricks& bm, int64_t tile, int l, int64_t& ix, int64_t& iy,
+                                            int64_t& iz)
 {
-    const int l = (int)(col & 63);
-    int64_t t = bm.bk0 + (col >> 6);
-    const int64_t bz = t % bm.nbz;
-    t /= bm.nbz;
-    const int64_t by = t % bm.nby, bx = t / bm.nby;
-    ix = 4 * bx + (l >> 4);
-    iy = 4 * by + ((l >> 2) & 3);
-    iz = 4 * bz + (l & 3);
+    const unsigned t = bm.bk0 + (unsigned)tile, u = bm.nbz.div(t), bx = bm.nby.div(u);
+    ix = 4 * (int64_t)bx + (l >> 4);
+    iy = 4 * (int64_t)(u - bx * bm.nby.d) + ((l >> 2) & 3);
+    iz = 4 * (int64_t)(t - u * bm.nbz.d) + (l & 3);
     const bool in = ix < bm.nx && iy < bm.ny && iz < bm.nz;
     ix = ix < bm.nx ? ix : bm.nx - 1;
     iy = iy < bm.ny ? iy : bm.ny - 1;
@@ -464,10 +525,11 @@ struct ShellGradArgs {
     const PrimRec* prims;
     const double* T;
     GridDesc grid;
-    int64_t p0, np, ld;
+    int64_t p0, np;
+    Pitch pg;            // of G
     int nprim_total;
     int is_normalized;
-    const R* G;          // [nao][ld]
+    const R* G;
     double* partial;     // [nrange][nprim_total + 3 nshell]
     int64_t ncol;
     // screened (whole regular grid): columns in bricks, G rows in the fused
@@ -509,11 +571,11 @@ __device__ __forceinline__ void shell_point(const ShellGradArgs<R>& a, const She
     // loaded before the primitive loop, whose exponentials then cover their
     // latency; the loads are unconditional (rows past the shell's last read
     // its last row, unused)
-    const R* Gi = a.G + (int64_t)sh.row0 * a.ld + i;
+    const R* Gi = a.G + (i >> 6) * a.pg.tile + (int64_t)sh.row0 * a.pg.row + (i & 63);
     R gv[NC];
     if (sh.kind != SHELL_T_GENERAL) {
 #pragma unroll
-        for (int k = 0; k < NC; ++k) gv[k] = Gi[(int64_t)min(k, sh.nrow - 1) * a.ld];
+        for (int k = 0; k < NC; ++k) gv[k] = Gi[(int64_t)min(k, sh.nrow - 1) * a.pg.row];
     }
     R S0 = 0, S1 = 0;
     R dw[MP];
@@ -543,7 +605,7 @@ __device__ __forceinline__ void shell_point(const ShellGradArgs<R>& a, const She
         for (int k = 0; k < NC; ++k) w[k] = gv[k] * (R)cart_norm(L, k);
     } else {
         for (int rw = 0; rw < sh.nrow; ++rw) {
-            const R g = Gi[(int64_t)rw * a.ld];
+            const R g = Gi[(int64_t)rw * a.pg.row];
 #pragma unroll
             for (int k = 0; k < NC; ++k) w[k] = fma(g, (R)Ts[rw * NC + k], w[k]);
         }
@@ -584,7 +646,7 @@ __device__ void shell_grad(const ShellGradArgs<R>& a, const ShellRec& sh, int pw
         for (int t = threadIdx.x; t < sh.nrow * ncart(L); t += blockDim.x) Ts[t] = T[t];
     }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pend = min(sh.nprim, pw0 + MP);
     const double nfac = a.is_normalized ? 0.0 : (2.0 * L + 3.0) / 4.0;
     R gr[3] = {0, 0, 0};
@@ -593,23 +655,23 @@ __device__ void shell_grad(const ShellGradArgs<R>& a, const ShellRec& sh, int pw
     for (int j = 0; j < MP; ++j) ga[j] = 0;
     const int64_t r0 = (int64_t)blockIdx.x * RANGE;
     const int64_t r1 = min(a.np, r0 + RANGE);
-    for (int64_t b = r0; b < r1; b += 256) {
-        const int64_t i = b + threadIdx.x;
+    const int chunk = sh.row0 >> 5;
+    for (int64_t b = r0 + 64 * wave; b < r1; b += 256) {
+        const int64_t i = b + lane;
         bool act = i < r1;
+        // the shell's rows of G exist where its chunk is live; the mask is the
+        // wave's, so that a dead tile costs no index arithmetic
+        if (a.mask && !((a.mask[(b >> 6) * a.nw + (chunk >> 6)] >> (chunk & 63)) & 1)) continue;
         double px, py, pz;
         if (a.bm.on) {
             int64_t ix, iy, iz;
-            act = brick_index(a.bm, act ? i : r0, ix, iy, iz) && act;
+            act = brick_index(a.bm, b >> 6, lane, ix, iy, iz) && act;
             px = a.grid.x[ix]; py = a.grid.y[iy]; pz = a.grid.z[iz];
         } else {
             grid_point(a.grid, a.p0 + (act ? i : r0), px, py, pz);
         }
         const double X = px - sh.cx, Y = py - sh.cy, Z = pz - sh.cz;
-        bool near = act && X * X + Y * Y + Z * Z < sh.rcut2;
-        if (a.mask && near) {   // the shell's rows of G exist where its chunk is live
-            const int c = sh.row0 >> 5;
-            near = (a.mask[(i >> 6) * a.nw + (c >> 6)] >> (c & 63)) & 1;
-        }
+        const bool near = act && X * X + Y * Y + Z * Z < sh.rcut2;
         if (!__builtin_amdgcn_ballot_w64(near)) continue;   // no point of this wave reaches the shell
         shell_point<L, MP, R>(a, sh, pw0, pend, px, py, pz, act ? i : r0, nfac, near, gr, ga, Ts);
     }
@@ -653,32 +715,33 @@ __global__ __launch_bounds__(256) void k_shell_grad(ShellGradArgs<R> a)
     }
 }
 
-// column sums of partial[nrange][ncol] in range order, then added to the
-// outputs: exponent columns to dalpha, shell position columns to the
-// shell's atom (shells of one atom summed in shell order by one thread)
-__global__ void k_reduce_cols(const double* partial, int nrange, int64_t ncol, double* colsum)
+// column sums of partial[nrange][ncol], then added to the outputs: exponent
+// columns to dalpha (one thread each), shell position columns to the shell's
+// atom (one wave per component: the lanes take every 64th shell, and their sums
+// are added in a fixed order)
+__global__ __launch_bounds__(256) void k_reduce_cols(const double* partial, int nrange, int64_t ncol, double* colsum)
 {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncol) return;
-    double s = 0.0;
-    for (int r = 0; r < nrange; ++r) s += partial[(int64_t)r * ncol + c];
-    colsum[c] = s;
+    const int64_t c = (int64_t)blockIdx.x * 16 + threadIdx.x;
+    const double t = column_sum<16>(partial, nrange, ncol, (int64_t)blockIdx.x * 16);
+    if (threadIdx.x < 16 && c < ncol) colsum[c] = t;
 }
 
 template <typename R>
-__global__ void k_scatter_grad(const double* colsum, const ShellRec* shells, int nshell, int nprim_total,
-                               int natoms, R* dalpha, R* dR)
+__global__ __launch_bounds__(64) void k_scatter_grad(const double* colsum, const ShellRec* shells, int nshell,
+                                                     int nprim_total, int natoms, R* dalpha, R* dR)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nprim_total) {
-        dalpha[t] = (R)((double)dalpha[t] + colsum[t]);
-    } else if (t < nprim_total + 3 * natoms) {
-        const int a = (t - nprim_total) / 3, d = (t - nprim_total) % 3;
+    const int lane = threadIdx.x;
+    if ((int)blockIdx.x < 3 * natoms) {
+        const int o = blockIdx.x, a = o / 3, d = o % 3;
         double s = 0.0;
-        for (int sh = 0; sh < nshell; ++sh)
-            if (load_shell(shells, sh).atom == a) s += colsum[nprim_total + 3 * sh + d];
-        dR[3 * a + d] = (R)((double)dR[3 * a + d] + s);
+        for (int sh = lane; sh < nshell; sh += 64)
+            if (shells[sh].atom == a) s += colsum[nprim_total + 3 * sh + d];
+        s = wave_sum(s);
+        if (lane == 0) dR[o] = (R)((double)dR[o] + s);
+        return;
     }
+    const int t = ((int)blockIdx.x - 3 * natoms) * 64 + lane;
+    if (t < nprim_total) dalpha[t] = (R)((double)dalpha[t] + colsum[t]);
 }
 
 // zero-filled padding of a [rows][ld] buffer's columns [c0, c1) (fill kernel,
@@ -722,13 +785,14 @@ __global__ void k_fill_zero(R* x, int64_t n)
     if (i < n) x[i] = R(0);
 }
 
-// rows[0 .. nrows) of X [.][ld] zeroed over columns [0, ncol)
+// rows[0 .. nrows) of X zeroed over columns [0, ncol)
 template <typename R>
-__global__ void k_zero_rows_r(R* X, int64_t ld, const int* rows, int nrows, int64_t ncol)
+__global__ void k_zero_rows_r(R* X, Pitch p, const int* rows, int nrows, int64_t ncol)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)nrows * ncol) return;
-    X[(int64_t)rows[i / ncol] * ld + i % ncol] = R(0);
+    const int64_t c = i % ncol;
+    X[rows[i / ncol] * p.row + (c >> 6) * p.tile + (c & 63)] = R(0);
 }
 
 // dL/drho of each brick column (0 for lanes outside the grid)
@@ -738,7 +802,7 @@ __global__ void k_gather_bricks(const R* g, BwdBricks bm, int64_t n, R* out)
     const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= n) return;
     int64_t ix, iy, iz;
-    const bool in = brick_index(bm, col, ix, iy, iz);
+    const bool in = brick_index(bm, col >> 6, (int)(col & 63), ix, iy, iz);
     out[col] = in ? g[(ix * bm.ny + iy) * bm.nz + iz] : R(0);
 }
 
@@ -750,7 +814,7 @@ struct BwdLayout {
     int64_t ncol = 0;
     int nsplit_max = 0;   // point ranges of the dL/dC contraction
     int krows = 0;        // rows of A and G: the AO count, or the fused rows of the screened path if more
-    size_t ct = 0, wc = 0, wct = 0, a = 0, phi = 0, bm = 0, g = 0, part = 0, cols = 0, dcp = 0, total = 0;   // bytes
+    size_t ct = 0, wc = 0, wct = 0, a = 0, bm = 0, g = 0, part = 0, cols = 0, dcp = 0, total = 0;   // bytes
     size_t cp = 0, dca = 0, gb = 0, live = 0, lcount = 0, mask = 0;   // screened path
 };
 
@@ -784,7 +848,6 @@ BwdLayout bwd_layout(const OkmiBasis* b, int nmo, int64_t chunk, size_t es)
     L.wc = o; o += pad256(packed_w_elems(nmo, L.krows) * es);     // C packed (Phi = C A)
     L.wct = o; o += pad256(packed_w_elems(L.krows, nmo) * es);    // C^T packed (G = C^T B)
     L.a = o; o += pad256(K * L.chunk * es);
-    L.phi = o; o += pad256((size_t)nmo * L.chunk * es);
     L.bm = o; o += pad256((size_t)nmo * L.chunk * es);
     L.g = o; o += pad256(K * L.chunk * es);
     L.part = o; o += pad256((size_t)L.nrange * L.ncol * sizeof(double));
@@ -815,16 +878,15 @@ size_t ws_bytes_of(const OkmiBasis* b, int nmo, int64_t chunk, size_t es)
 // so that the groups divide the tiles as evenly as possible.  mode 1 / 2:
 // the screened forms of k_gemm_nn (live-chunk lists per 64-point tile).
 template <typename R>
-void launch_gemm_nn(const R* Wp, int M, int K, const R* X, int64_t ldx, int64_t npad, R* out, int64_t ldo,
-                    hipStream_t st, int mode = 0, const int* live = nullptr, const int* lcount = nullptr,
-                    int nchunk = 0)
+void launch_gemm_nn(const R* Wp, int M, int K, const R* X, Pitch px, int64_t npad, R* out, Pitch po,
+                    hipStream_t st, const ColScale<R>& cs, int mode, const int* live, const int* lcount, int nchunk)
 {
     const dim3 grd((unsigned)((npad + 255) / 256)), blk(256);
     const int nks = (K + 3) / 4;
     if (nks <= 16) {   // short K (the MO count): X rows held in registers
 #define OKMI_GXR(MG, MODE, KS) \
-    hipLaunchKernelGGL((k_gemm_nn_xr<R, MG, MODE, KS>), grd, blk, 0, st, Wp, M, K, X, ldx, npad, out, ldo, live, lcount, \
-                       nchunk)
+    hipLaunchKernelGGL((k_gemm_nn_xr<R, MG, MODE, KS>), grd, blk, 0, st, Wp, M, K, X, px, npad, out, po, live, lcount, \
+                       nchunk, cs)
 #define OKMI_GXR_KS(MG, MODE)                      \
     do {                                           \
         if (nks <= 4) OKMI_GXR(MG, MODE, 4);       \
@@ -839,7 +901,7 @@ void launch_gemm_nn(const R* Wp, int M, int K, const R* X, int64_t ldx, int64_t 
         if (mode != 1) return;
     }
 #define OKMI_GNN(MG, MODE) \
-    hipLaunchKernelGGL((k_gemm_nn<R, MG, MODE>), grd, blk, 0, st, Wp, M, K, X, ldx, npad, out, ldo, live, lcount, nchunk)
+    hipLaunchKernelGGL((k_gemm_nn<R, MG, MODE>), grd, blk, 0, st, Wp, M, K, X, px, npad, out, po, live, lcount, nchunk, cs)
     if (mode == 2) {
         OKMI_GNN(2, 2);
         return;
@@ -874,8 +936,25 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     constexpr size_t es = sizeof(R);
     const char* name = es == 8 ? "rho_backward" : "rho_backward_f32";
     if (np <= 0 || nmo <= 0) return 0;
-    // largest chunk (a multiple of 64 points, at most np rounded up) whose layout fits
-    int64_t lo = 64, hi = (np + 63) & ~(int64_t)63;
+    // Screened form for a whole regular grid: points in 4x4x4 bricks, AO rows
+    // in the fused order of the basis (32-row chunks), and per 64-point tile
+    // only the chunks with a shell in reach (the bound of the fused kernels)
+    // are evaluated (A), contracted (Phi = C A, dL/dC = B A^T) and produced
+    // (G = C^T B); the shell gradients read G where the shell's chunk is live.
+    const bool scr = g.regular && p0 == 0 && np == g.nx * g.ny * g.nz && b->nchunk > 0 && b->d_ishells &&
+                     b->nkpad > 0;
+    BwdBricks bm{};
+    int64_t total = np;
+    if (scr) {
+        const int64_t nbx = (g.nx + 3) / 4, nby = (g.ny + 3) / 4, nbz = (g.nz + 3) / 4;
+        bm.on = 1;
+        bm.nby.set((unsigned)nby);
+        bm.nbz.set((unsigned)nbz);
+        bm.nx = g.nx; bm.ny = g.ny; bm.nz = g.nz;
+        total = nbx * nby * nbz * 64;
+    }
+    // largest chunk (a multiple of 64 points, at most all of them) whose layout fits
+    int64_t lo = 64, hi = (total + 63) & ~(int64_t)63;
     if (!ws || ws_bytes_of(b, nmo, lo, es) > ws_bytes) {
         okmi_set_error("%s: workspace of %zu bytes is too small (need at least %zu)", name, ws_bytes,
                        ws_bytes_of(b, nmo, lo, es));
@@ -909,19 +988,11 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     R* WC = (R*)(w + Lo.wc);
     R* WCT = (R*)(w + Lo.wct);
     R* A = (R*)(w + Lo.a);
-    R* Phi = (R*)(w + Lo.phi);
     R* B = (R*)(w + Lo.bm);
     R* G = (R*)(w + Lo.g);
     double* part = (double*)(w + Lo.part);
     double* cols = (double*)(w + Lo.cols);
     R* dcp = (R*)(w + Lo.dcp);
-    // Screened form for a whole regular grid: points in 4x4x4 bricks, AO rows
-    // in the fused order of the basis (32-row chunks), and per 64-point tile
-    // only the chunks with a shell in reach (the bound of the fused kernels)
-    // are evaluated (A), contracted (Phi = C A, dL/dC = B A^T) and produced
-    // (G = C^T B); the shell gradients read G where the shell's chunk is live.
-    const bool scr = g.regular && p0 == 0 && np == g.nx * g.ny * g.nz && b->nchunk > 0 && b->d_ishells &&
-                     b->nkpad > 0 && b->nkpad <= Lo.krows;
     const int K = scr ? b->nkpad : b->nao;   // rows of A and G
     // the FP32 backward screens with the bound of the paths ending in FP32
     const bool split = es == 4;
@@ -933,14 +1004,9 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     int* lcount = (int*)(w + Lo.lcount);
     unsigned long long* lmask = (unsigned long long*)(w + Lo.mask);
     const int nw = scr ? live_mask_words(b) : 0;
-    BwdBricks bm{};
-    int64_t total = np;
-    if (scr) {
-        bm.on = 1;
-        bm.nbx = (g.nx + 3) / 4; bm.nby = (g.ny + 3) / 4; bm.nbz = (g.nz + 3) / 4;
-        bm.nx = g.nx; bm.ny = g.ny; bm.nz = g.nz;
-        total = bm.nbx * bm.nby * bm.nbz * 64;
-    }
+    // A of the unscreened form is written by rows
+    const Pitch pa = scr ? Pitch{64, (int64_t)K * 64} : Pitch{chunk, 64};
+    const Pitch pb{64, (int64_t)nmo * 64}, pg{64, (int64_t)K * 64};
     OkmiProfScope prof(name, st);
     const R* Cw = d_c;   // C in the row order of A
     if (scr) {
@@ -951,7 +1017,7 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
         // rows no shell writes (padding of the chunks) are zero in A for good
         if (b->npadrows > 0)
             hipLaunchKernelGGL(k_zero_rows_r<R>, dim3((unsigned)(((int64_t)b->npadrows * chunk + 255) / 256)),
-                               dim3(256), 0, st, A, chunk, (const int*)b->d_padrows, b->npadrows, chunk);
+                               dim3(256), 0, st, A, pa, (const int*)b->d_padrows, b->npadrows, chunk);
         Cw = Cp;
     }
     hipLaunchKernelGGL(k_transpose<R>, dim3((unsigned)(((int64_t)nmo * K + 255) / 256)), dim3(256), 0, st, Cw, nmo,
@@ -963,17 +1029,16 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
     const int set0 = 0;
     for (int64_t c0 = 0; c0 < total; c0 += chunk) {
         const int64_t n = total - c0 < chunk ? total - c0 : chunk;
-        const int64_t n16 = (n + 15) & ~(int64_t)15;
         const int64_t n64 = (n + 63) & ~(int64_t)63;
         int rc;
         if (scr) {
-            bm.bk0 = c0 / 64;
-            rc = okmi_launch_live_chunks(b, g, 1, bm.bk0, 0, n, 64, live, lcount, st, lmask, split);
+            bm.bk0 = (unsigned)(c0 / 64);
+            rc = okmi_launch_live_chunks(b, g, 1, c0 / 64, 0, n, 64, live, lcount, st, lmask, split);
             if (rc) return rc;
-            const AoBricks bk{bm.bk0, n / 64, bm.nbx, bm.nby, bm.nbz};
+            const AoBricks bk{c0 / 64, n / 64, (g.nx + 3) / 4, (g.ny + 3) / 4, (g.nz + 3) / 4, pa.tile};
             const AoLiveMask am{lmask, nw, 0, split ? b->d_wshells_s : nullptr};
             rc = okmi_launch_ao_eval_ex(b, split ? b->d_ishells_s : b->d_ishells, split ? b->d_fprims_s : b->d_fprims,
-                                        g, 0, n, &bk, &set0, 1, es == 8 ? OKMI_F64 : OKMI_F32, A, chunk, 0, st, &am);
+                                        g, 0, n, &bk, &set0, 1, es == 8 ? OKMI_F64 : OKMI_F32, A, pa.row, 0, st, &am);
             if (rc) return rc;
             hipLaunchKernelGGL(k_gather_bricks<R>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d_grad, bm, n,
                                gb);
@@ -981,54 +1046,51 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
         } else {
             rc = okmi_launch_ao_eval(b, g, p0 + c0, n, &set0, 1, es == 8 ? OKMI_F64 : OKMI_F32, A, chunk, 0, st);
             if (rc) return rc;
-            if (n16 > n)
-                hipLaunchKernelGGL(k_zero_cols<R>, dim3((unsigned)((b->nao * (n16 - n) + 255) / 256)), dim3(256), 0,
-                                   st, A, b->nao, chunk, n, n16);
+            if (n64 > n)
+                hipLaunchKernelGGL(k_zero_cols<R>, dim3((unsigned)((b->nao * (n64 - n) + 255) / 256)), dim3(256), 0,
+                                   st, A, b->nao, chunk, n, n64);
             dg = d_grad + c0;
         }
         {
             OkmiProfScope p1(es == 8 ? "gemm_nn" : "gemm_nn_f32", st);
-            launch_gemm_nn<R>(WC, nmo, K, A, chunk, n64, Phi, chunk, st, scr ? 1 : 0, live, lcount, b->nchunk);
+            launch_gemm_nn<R>(WC, nmo, K, A, pa, n64, B, pb, st, ColScale<R>{d_occ, dg, n}, scr ? 1 : 0, live,
+                              lcount, b->nchunk);
         }
-        hipLaunchKernelGGL(k_bmat<R>, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, Phi, d_occ, dg, nmo, n,
-                           n16, chunk, B);
-        // point ranges: about 2048 waves over the chip, at least 256 points
-        // per range, at most the partial buffer's ranges
+        // point ranges: about 3072 waves over the chip (three per SIMD, what the
+        // registers allow), at least 256 points per range, at most the partial
+        // buffer's ranges
         const int64_t tiles = (K + 16 * NT - 1) / (16 * NT);
-        int64_t nsplit = std::max<int64_t>(1, std::min<int64_t>({(2048 + tiles - 1) / tiles, n16 / 256,
-                                                                 (int64_t)Lo.nsplit_max}));
-        int64_t krange = ((n16 + nsplit - 1) / nsplit + 15) & ~(int64_t)15;
-        if (scr) krange = (krange + 63) & ~(int64_t)63;   // whole 64-point tiles per range
-        nsplit = (n16 + krange - 1) / krange;
+        const int64_t nsplit = std::max<int64_t>(1, std::min<int64_t>({(3072 + tiles - 1) / tiles, n64 / 256,
+                                                                       (int64_t)Lo.nsplit_max}));
         // blocks: (range group of 8, AO tile, XCD); range = group * 8 + XCD
         const unsigned nblk = (unsigned)(((nsplit + 7) / 8) * tiles * 8);
         const int nmt = (nmo + 15) / 16;
         const unsigned long long* tn_mask = scr ? lmask : nullptr;
-        const int nchunk_tn = b->nchunk;
         {
             OkmiProfScope p2(es == 8 ? "gemm_tn" : "gemm_tn_f32", st);
             if (nmt == 1)
-                hipLaunchKernelGGL((k_gemm_tn<R, 1>), dim3(nblk), dim3(64), 0, st, B, nmo, A, K, n16, chunk,
-                                   krange, (int)nsplit, dcp, tn_mask, nw, nchunk_tn);
+                hipLaunchKernelGGL((k_gemm_tn<R, 1>), dim3(nblk), dim3(64), 0, st, B, pb, nmo, A, pa, K,
+                                   (int)(n64 / 64), (int)nsplit, dcp, tn_mask, nw);
             else if (nmt == 2)
-                hipLaunchKernelGGL((k_gemm_tn<R, 2>), dim3(nblk), dim3(64), 0, st, B, nmo, A, K, n16, chunk,
-                                   krange, (int)nsplit, dcp, tn_mask, nw, nchunk_tn);
+                hipLaunchKernelGGL((k_gemm_tn<R, 2>), dim3(nblk), dim3(64), 0, st, B, pb, nmo, A, pa, K,
+                                   (int)(n64 / 64), (int)nsplit, dcp, tn_mask, nw);
             else
-                hipLaunchKernelGGL((k_gemm_tn<R, 3>), dim3(nblk), dim3(64), 0, st, B, nmo, A, K, n16, chunk,
-                                   krange, (int)nsplit, dcp, tn_mask, nw, nchunk_tn);
+                hipLaunchKernelGGL((k_gemm_tn<R, 3>), dim3(nblk), dim3(64), 0, st, B, pb, nmo, A, pa, K,
+                                   (int)(n64 / 64), (int)nsplit, dcp, tn_mask, nw);
         }
         const int64_t ndc = (int64_t)nmo * K;
-        hipLaunchKernelGGL(k_reduce_dc<R>, dim3((unsigned)((ndc + 255) / 256)), dim3(256), 0, st, dcp, (int)nsplit,
+        hipLaunchKernelGGL(k_reduce_dc<R>, dim3((unsigned)((ndc + 31) / 32)), dim3(256), 0, st, dcp, (int)nsplit,
                            ndc, scr ? dCa : d_dc);
         {
             OkmiProfScope p1(es == 8 ? "gemm_nn" : "gemm_nn_f32", st);
-            launch_gemm_nn<R>(WCT, K, nmo, B, chunk, n64, G, chunk, st, scr ? 2 : 0, live, lcount, b->nchunk);
+            launch_gemm_nn<R>(WCT, K, nmo, B, pb, n64, G, pg, st, ColScale<R>{}, scr ? 2 : 0, live, lcount,
+                              b->nchunk);
         }
         ShellGradArgs<R> sa{};
         sa.shells = scr ? (split ? b->d_ishells_s : b->d_ishells) : b->d_shells;
         sa.prims = scr ? (split ? b->d_fprims_s : b->d_fprims) : b->d_prims;
         sa.T = b->d_T; sa.grid = g;
-        sa.p0 = p0 + c0; sa.np = n; sa.ld = chunk; sa.nprim_total = b->nprim; sa.is_normalized = b->is_normalized;
+        sa.p0 = p0 + c0; sa.np = n; sa.pg = pg; sa.nprim_total = b->nprim; sa.is_normalized = b->is_normalized;
         sa.G = G; sa.partial = part; sa.ncol = Lo.ncol;
         sa.bm = bm;
         sa.mask = scr ? lmask : nullptr;
@@ -1044,9 +1106,9 @@ int launch_backward(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t n
                                    dim3((unsigned)nrange, (unsigned)b->nshell, (unsigned)((maxp + MAXP - 1) / MAXP)),
                                    dim3(256), 0, st, sa);
         }
-        hipLaunchKernelGGL(k_reduce_cols, dim3((unsigned)((Lo.ncol + 255) / 256)), dim3(256), 0, st, part, nrange,
+        hipLaunchKernelGGL(k_reduce_cols, dim3((unsigned)((Lo.ncol + 15) / 16)), dim3(256), 0, st, part, nrange,
                            Lo.ncol, cols);
-        hipLaunchKernelGGL(k_scatter_grad<R>, dim3((unsigned)((b->nprim + 3 * b->natoms + 255) / 256)), dim3(256), 0,
+        hipLaunchKernelGGL(k_scatter_grad<R>, dim3((unsigned)(3 * b->natoms + (b->nprim + 63) / 64)), dim3(64), 0,
                            st, cols, b->d_shells, b->nshell, b->nprim, b->natoms, d_dalpha, d_dr);
     }
     if (scr) {
