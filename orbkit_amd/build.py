@@ -15,7 +15,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), 'include')
 
 # (the slow ones first)
 SOURCES = ['fused_f64_p1.hip', 'mo_fused_f64.hip', 'fused_f64_general.hip', 'fused_f64_p4.hip', 'fused_f64_p0.hip',
-           'fused_f64_p23.hip', 'rho_fused.hip', 'rho_big.hip', 'rho_backward.hip', 'rho_gemm_m1.hip', 'rho_gemm_m0.hip',
+           'fused_f64_p23.hip', 'rho_fused.hip', 'rho_big.hip', 'rho_big_split.hip', 'rho_backward.hip', 'rho_gemm_m1.hip', 'rho_gemm_m0.hip',
            'abi.cpp', 'ao_eval.hip', 'rho_gemm.hip', 'rho_fused_f64.hip', 'electrons.hip', 'extras.hip', 'cube.cpp',
            'detci.hip']
 

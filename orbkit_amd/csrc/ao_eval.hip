@@ -33,7 +33,7 @@ struct AoArgs {
     // of its tile's live chunks (chunk table and work-ordered shells of the
     // fused layout); null: every shell of `shells`
     const unsigned long long* live_mask;
-    int mask_words, mask_shift;
+    int mask_words, mask_shift, mask_quads;
     const int2* chunks;        // per chunk: first work entry, shells | used rows << 16
     const ShellRec* wshells;   // work order, internal rows, fused radii, PrimRec primitives
 };
@@ -175,6 +175,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
         act = i < a.np;
         grid_point(a.grid, a.p0 + (act ? i : 0), px, py, pz);
+        i = (i >> 6) * a.tile_stride + (i & 63);
     }
     // bounding box of the wave's points (inactive lanes repeat point 0,
     // which only enlarges the box)
@@ -188,14 +189,17 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         }
     // one shell for the wave's points: its rows evaluated, or zero when it is
     // out of reach (every value and derivative below the screening bound)
-    auto shell = [&](const ShellRec& sh) {
+    // (quads: the live quads of its chunk, whose rows alone are read)
+    auto shell = [&](const ShellRec& sh, unsigned quads) {
         const double d2 = uniform(box_dist2(lo, hi, sh));
         if (d2 >= sh.rcut2) {
             if (act)
                 for (int c = 0; c < OKMI_MAX_SETS; ++c) {
                     if (a.dst[c] < 0) continue;
                     OutT* o = out + a.dst[c] * a.set_stride + (int64_t)sh.row0 * a.ld + i;
-                    for (int r = 0; r < sh.nrow; ++r) __builtin_nontemporal_store((OutT)0, &o[(int64_t)r * a.ld]);
+                    for (int r = 0; r < sh.nrow; ++r)
+                        if (quads >> (((sh.row0 + r) & 31) >> 2) & 1)
+                            __builtin_nontemporal_store((OutT)0, &o[(int64_t)r * a.ld]);
                 }
             return;
         }
@@ -208,7 +212,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         }
     };
     if (!a.live_mask) {
-        for (int s = 0; s < a.nshell; ++s) shell(load_shell(a.shells, s));
+        for (int s = 0; s < a.nshell; ++s) shell(load_shell(a.shells, s), 0xff);
         return;
     }
     // the shells of the live chunks of this wave's tile; the rows of the
@@ -225,11 +229,19 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         unsigned long long m = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(m0 >> 32)) << 32) |
                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)m0);
         while (m) {
-            const int c = 64 * w + __builtin_ctzll(m);
-            m &= m - 1;
+            const int bit = __builtin_ctzll(m);
+            int c = 64 * w + bit;
+            unsigned quads = 0xff;
+            if (a.mask_quads) {
+                c >>= 3;
+                quads = (unsigned)(m >> (bit & ~7)) & 0xff;
+                m &= ~(0xffull << (bit & ~7));
+            } else {
+                m &= m - 1;
+            }
             const int2 cw = load_int2(a.chunks, c);
             const int nsh = cw.y & 0xffff;
-            for (int e = 0; e < nsh; ++e) shell(load_shell(a.wshells, cw.x + e));
+            for (int e = 0; e < nsh; ++e) shell(load_shell(a.wshells, cw.x + e), quads);
         }
     }
 }
@@ -436,6 +448,7 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
         a.live_mask = live->mask;
         a.mask_words = live->words;
         a.mask_shift = live->shift;
+        a.mask_quads = live->quads;
         a.chunks = b->d_chunks;
         a.wshells = live->wshells ? live->wshells : b->d_wshells;
     }
@@ -448,6 +461,7 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
     a.ld = ld;
     a.set_stride = set_stride;
     a.nshell = b->nshell;
+    a.tile_stride = live ? live->tile_stride : 64;
     // each code's first set; the groups write those, repeats are copies
     int first[OKMI_MAX_SETS];
     for (int c = 0; c < OKMI_MAX_SETS; ++c) first[c] = -1;

@@ -88,6 +88,11 @@ struct AoLiveMask {
     int words;
     int shift;
     const ShellRec* wshells;   // work-order shells of the screening bound in use (null: d_wshells)
+    // quads: the masks mark quads (bit q: rows 4 q .. 4 q + 3); a chunk is live
+    // if one of its eight is, and a shell out of reach writes zeros only to the
+    // rows of live quads
+    bool quads = false;
+    int64_t tile_stride = 64;  // range order: column c at tile_stride (c / 64) + c % 64
 };
 int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const PrimRec* prims, const GridDesc& g,
                            int64_t p0, int64_t np, const AoBricks* bricks, const int* drv, int ndrv, int out_dtype,
@@ -138,6 +143,9 @@ int okmi_launch_permute_c(const double* C, int nmo, int nao, int64_t kpad, const
 // zero rows rows[0 .. nrows) of S sets [S][set_stride] (row stride ld) over columns [0, ncol)
 int okmi_launch_zero_rows(double* a, int S, int64_t set_stride, int64_t ld, const int* rows, int nrows, int64_t ncol,
                           hipStream_t st);
+
+int okmi_launch_zero_rows_f32(float* a, int S, int64_t set_stride, int64_t ld, const int* rows, int nrows, int64_t ncol,
+                              hipStream_t st);
 
 // codes whose AO sets a density request needs: 0, the requested codes and
 // the first derivatives entering second-derivative product terms

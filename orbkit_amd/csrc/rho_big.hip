@@ -16,8 +16,7 @@
 // S is 1 (rho), 4 (+ first derivatives), 7 (+ diagonal second derivatives)
 // or 10 (+ mixed second derivatives); a request is served by the smallest S
 // holding its codes and their product terms.
-#include "okmi_internal.h"
-#include "split_mfma.h"
+#include "rho_big.h"
 
 namespace {
 
@@ -75,15 +74,6 @@ struct BigLds {
     static constexpr int STAGE = AO_FLOATS * 4 + C_BYTES;          // bytes per buffer
     static constexpr int TOTAL = 2 * STAGE;
 };
-
-// XCD-aware block order: hardware places block b on XCD b % 8; blocks that
-// share a point tile (its MO tiles) are given consecutive logical indices on
-// one XCD so its L2 serves the AO tile to all of them.
-__device__ __forceinline__ int64_t logical_block(int64_t b, int64_t nb)
-{
-    const int64_t xcd = b & 7, j = b >> 3, per = nb >> 3, rem = nb & 7;
-    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + j;
-}
 
 // LONG: live lists may exceed 128 entries (more than 128 chunks of 32 rows),
 // and their tail is read from memory
@@ -325,57 +315,6 @@ __global__ __launch_bounds__(64 * BigCfg<S>::NW, 1) void k_rho_big(BigArgs a)
     }
 }
 
-__global__ void k_pad_occ_big(const double* occ, int nmo, int mpad, double* out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < mpad) out[i] = i < nmo ? occ[i] : 0.0;
-}
-
-struct OutCodes {
-    int n;
-    int c[16];
-};
-
-struct BrickMap {
-    int on;
-    int64_t bk0, nbx, nby, nbz, nx, ny, nz;
-};
-
-// rho[p] = sum_mt partial[mt][0][col]; delta[r][p] = sum_mt partial[mt][c_r][col]
-// (code 0: 2 rho, orbkit/core.py:299-300 with drv None).  Column col is point
-// p = col (range order) or, in brick order, the grid point of lane col % 64
-// of brick bk0 + col / 64 (columns outside the grid are dropped).
-__global__ void k_reduce_big(const double* partial, int nmt, int S, int64_t ld, int64_t np, OutCodes oc,
-                             double* rho, double* delta, int64_t ld_delta, BrickMap bm)
-{
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= np) return;
-    int64_t p = col;
-    if (bm.on) {
-        const int lane = (int)(col & 63);
-        int64_t t = bm.bk0 + (col >> 6);
-        const int64_t bz = t % bm.nbz;
-        t /= bm.nbz;
-        const int64_t by = t % bm.nby, bx = t / bm.nby;
-        const int64_t ix = 4 * bx + (lane >> 4), iy = 4 * by + ((lane >> 2) & 3), iz = 4 * bz + (lane & 3);
-        if (ix >= bm.nx || iy >= bm.ny || iz >= bm.nz) return;
-        p = (ix * bm.ny + iy) * bm.nz + iz;
-    }
-    double r = 0.0;
-    for (int m = 0; m < nmt; ++m) r += partial[(int64_t)m * S * ld + col];
-    rho[p] = r;
-    for (int j = 0; j < oc.n; ++j) {
-        const int c = oc.c[j];
-        double v = 0.0;
-        if (c == 0) {
-            v = 2.0 * r;
-        } else {
-            for (int m = 0; m < nmt; ++m) v += partial[((int64_t)m * S + c) * ld + col];
-        }
-        delta[j * ld_delta + p] = v;
-    }
-}
-
 // Live chunks of each point tile of NP columns: one wave per tile forms the
 // tile's bounding box from its points (brick order: the grid points of the
 // bricks' lanes; range order: points p0 + column), then tests every 32-row
@@ -397,48 +336,12 @@ struct LiveArgs {
     int words;
 };
 
-__device__ __forceinline__ double wave_reduce(double v, bool take_min)
-{
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const double u = __shfl_xor(v, o);
-        v = take_min ? fmin(v, u) : fmax(v, u);
-    }
-    return v;
-}
-
 __global__ __launch_bounds__(64) void k_big_live(LiveArgs a)
 {
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x;
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int j = lane; j < a.np; j += 64) {
-        const int64_t col = t * a.np + j;
-        if (col >= a.n) continue;
-        double q[3];
-        if (a.bm.on) {
-            const int l = (int)(col & 63);
-            int64_t b = a.bm.bk0 + (col >> 6);
-            const int64_t bz = b % a.bm.nbz;
-            b /= a.bm.nbz;
-            const int64_t by = b % a.bm.nby, bx = b / a.bm.nby;
-            const int64_t ix = 4 * bx + (l >> 4), iy = 4 * by + ((l >> 2) & 3), iz = 4 * bz + (l & 3);
-            if (ix >= a.bm.nx || iy >= a.bm.ny || iz >= a.bm.nz) continue;
-            q[0] = a.grid.x[ix]; q[1] = a.grid.y[iy]; q[2] = a.grid.z[iz];
-        } else {
-            grid_point(a.grid, a.p0 + col, q[0], q[1], q[2]);
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            lo[d] = fmin(lo[d], q[d]);
-            hi[d] = fmax(hi[d], q[d]);
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        lo[d] = wave_reduce(lo[d], true);
-        hi[d] = wave_reduce(hi[d], false);
-    }
+    double lo[3], hi[3];
+    columns_box(a.grid, a.bm, a.p0, a.n, t * a.np, a.np, lane, lo, hi);
     int base = 0;
     for (int c0 = 0; c0 < a.nchunk; c0 += 64) {
         const int c = c0 + lane;
@@ -499,24 +402,15 @@ int launch_big_s(const BigArgs& a, hipStream_t st)
     return a.nchunk > 128 ? launch_big_l<PREC, S, true>(a, st) : launch_big_l<PREC, S, false>(a, st);
 }
 
+// (the split precisions come here for 7 and 10 sets only)
 template <int PREC>
 int launch_big(const BigArgs& a, int S, hipStream_t st)
 {
-    switch (S) {
-    case 1: return launch_big_s<PREC, 1>(a, st);
-    case 4: return launch_big_s<PREC, 4>(a, st);
-    case 7: return launch_big_s<PREC, 7>(a, st);
-    default: return launch_big_s<PREC, 10>(a, st);
+    if constexpr (PREC == OKMI_PREC_F32) {
+        if (S == 1) return launch_big_s<PREC, 1>(a, st);
+        if (S == 4) return launch_big_s<PREC, 4>(a, st);
     }
-}
-
-inline size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-int big_sets(const int* drv_out, int nout)
-{
-    int mx = 0;
-    for (int r = 0; r < nout; ++r) mx = std::max(mx, drv_out[r]);
-    return mx == 0 ? 1 : mx <= 3 ? 4 : mx <= 6 ? 7 : 10;
+    return S == 7 ? launch_big_s<PREC, 7>(a, st) : launch_big_s<PREC, 10>(a, st);
 }
 
 struct BigLayout {
@@ -572,6 +466,16 @@ int okmi_launch_zero_rows(double* a, int S, int64_t set_stride, int64_t ld, cons
     return 0;
 }
 
+int okmi_launch_zero_rows_f32(float* a, int S, int64_t set_stride, int64_t ld, const int* rows, int nrows, int64_t ncol,
+                              hipStream_t st)
+{
+    const int64_t nz = (int64_t)S * nrows * ncol;
+    if (nz <= 0) return 0;
+    hipLaunchKernelGGL(k_zero_rows<float>, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, st, a, S, set_stride, ld,
+                       rows, nrows, ncol);
+    return 0;
+}
+
 size_t okmi_big_ws_bytes(const OkmiBasis* b, int nmo, int prec, int S, int64_t np)
 {
     const BigLayout L = big_layout(b, nmo, prec, S);
@@ -601,6 +505,9 @@ int okmi_launch_rho_big(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np,
     const BigLayout L = big_layout(b, nmo, prec, S);
     int rc0 = okmi_prepare_fused(b);   // output-row shells and primitives with the fused radii
     if (rc0) return rc0;
+    if (prec != OKMI_PREC_F32 && S <= 4)
+        return okmi_launch_rho_big_split(b, g, p0, np, d_c, d_occ, nmo, prec, S, drv_out, nout, rho, delta, ld_delta, ws,
+                                         ws_bytes, st);
     if (!ws || ws_bytes < L.fixed + L.per_point * 128) {
         okmi_set_error("rho_big: workspace of %zu bytes is too small (need at least %zu)", ws_bytes,
                        L.fixed + L.per_point * 128);
@@ -644,11 +551,7 @@ int okmi_launch_rho_big(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np,
     // padding rows of the AO buffer zeroed once (no shell writes them)
     hipLaunchKernelGGL(k_prep_c, dim3((unsigned)((L.mpad * L.kpad + 255) / 256)), dim3(256), 0, st, d_c, nmo, b->nao,
                        prec, L.mpad, L.kpad, (const int*)b->d_colmap, cpl);
-    if (b->npadrows > 0) {
-        const int64_t nz = (int64_t)S * b->npadrows * chunk;
-        hipLaunchKernelGGL(k_zero_rows<float>, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, st, ao, S,
-                           (int64_t)L.kpad * chunk, chunk, (const int*)b->d_padrows, b->npadrows, chunk);
-    }
+    okmi_launch_zero_rows_f32(ao, S, (int64_t)L.kpad * chunk, chunk, (const int*)b->d_padrows, b->npadrows, chunk, st);
     hipLaunchKernelGGL(k_pad_occ_big, dim3((unsigned)((L.mpad + 255) / 256)), dim3(256), 0, st, d_occ, nmo,
                        (int)L.mpad, occp);
     int codes[10];
