@@ -370,6 +370,8 @@ extern "C" int okmi_basis_destroy(okmi_basis* b)
     if (b->d_lgroups) (void)hipFree(b->d_lgroups);
     if (b->d_lshells_a) (void)hipFree(b->d_lshells_a);
     if (b->d_lgroups_a) (void)hipFree(b->d_lgroups_a);
+    for (void* p : {(void*)b->d_wlist, (void*)b->d_wlist_groups, (void*)b->d_wlist_s, (void*)b->d_wlist_groups_s})
+        if (p) (void)hipFree(p);
     delete[] b->h_shells;
     delete[] b->h_prims;
     delete[] b->h_T;

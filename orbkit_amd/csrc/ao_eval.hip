@@ -33,7 +33,7 @@ struct AoArgs {
     // of its tile's live chunks (chunk table and work-ordered shells of the
     // fused layout); null: every shell of `shells`
     const unsigned long long* live_mask;
-    int mask_words, mask_shift, mask_quads;
+    int mask_words, mask_shift;
     const int2* chunks;        // per chunk: first work entry, shells | used rows << 16
     const ShellRec* wshells;   // work order, internal rows, fused radii, PrimRec primitives
 };
@@ -175,7 +175,6 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
         act = i < a.np;
         grid_point(a.grid, a.p0 + (act ? i : 0), px, py, pz);
-        i = (i >> 6) * a.tile_stride + (i & 63);
     }
     // bounding box of the wave's points (inactive lanes repeat point 0,
     // which only enlarges the box)
@@ -189,17 +188,14 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         }
     // one shell for the wave's points: its rows evaluated, or zero when it is
     // out of reach (every value and derivative below the screening bound)
-    // (quads: the live quads of its chunk, whose rows alone are read)
-    auto shell = [&](const ShellRec& sh, unsigned quads) {
+    auto shell = [&](const ShellRec& sh) {
         const double d2 = uniform(box_dist2(lo, hi, sh));
         if (d2 >= sh.rcut2) {
             if (act)
                 for (int c = 0; c < OKMI_MAX_SETS; ++c) {
                     if (a.dst[c] < 0) continue;
                     OutT* o = out + a.dst[c] * a.set_stride + (int64_t)sh.row0 * a.ld + i;
-                    for (int r = 0; r < sh.nrow; ++r)
-                        if (quads >> (((sh.row0 + r) & 31) >> 2) & 1)
-                            __builtin_nontemporal_store((OutT)0, &o[(int64_t)r * a.ld]);
+                    for (int r = 0; r < sh.nrow; ++r) __builtin_nontemporal_store((OutT)0, &o[(int64_t)r * a.ld]);
                 }
             return;
         }
@@ -212,7 +208,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         }
     };
     if (!a.live_mask) {
-        for (int s = 0; s < a.nshell; ++s) shell(load_shell(a.shells, s), 0xff);
+        for (int s = 0; s < a.nshell; ++s) shell(load_shell(a.shells, s));
         return;
     }
     // the shells of the live chunks of this wave's tile; the rows of the
@@ -229,19 +225,11 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
         unsigned long long m = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(m0 >> 32)) << 32) |
                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)m0);
         while (m) {
-            const int bit = __builtin_ctzll(m);
-            int c = 64 * w + bit;
-            unsigned quads = 0xff;
-            if (a.mask_quads) {
-                c >>= 3;
-                quads = (unsigned)(m >> (bit & ~7)) & 0xff;
-                m &= ~(0xffull << (bit & ~7));
-            } else {
-                m &= m - 1;
-            }
+            const int c = 64 * w + __builtin_ctzll(m);
+            m &= m - 1;
             const int2 cw = load_int2(a.chunks, c);
             const int nsh = cw.y & 0xffff;
-            for (int e = 0; e < nsh; ++e) shell(load_shell(a.wshells, cw.x + e), quads);
+            for (int e = 0; e < nsh; ++e) shell(load_shell(a.wshells, cw.x + e));
         }
     }
 }
@@ -269,20 +257,20 @@ struct AoListArgs {
 
 template <int PASS> struct AoSets { static constexpr int n = PASS == 0 ? 1 : 4; };
 
-template <int L, bool SPH, int PASS>
-__device__ __forceinline__ void ao_rows(const AoListArgs& a, double* o, bool act, double X, double Y, double Z, double S0,
+template <int L, bool SPH, int PASS, typename OutT>
+__device__ __forceinline__ void ao_rows(const AoListArgs& a, OutT* o, bool act, double X, double Y, double Z, double S0,
                                         double S1, double S2)
 {
     constexpr int NS = AoSets<PASS>::n;
     each_row<0>(RowSets<L, SPH, PASS>(X, Y, Z, S0, S1, S2), [&](int r, const double (&v)[NS]) {
 #pragma unroll
         for (int s = 0; s < NS; ++s)
-            if (a.dst[s] >= 0 && act) o[a.dst[s] * a.set_stride + r * a.ld] = v[s];
+            if (a.dst[s] >= 0 && act) o[a.dst[s] * a.set_stride + r * a.ld] = (OutT)v[s];
     });
 }
 
-template <int L, int PASS>
-__device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& sh, double* o, bool act, double X, double Y,
+template <int L, int PASS, typename OutT>
+__device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& sh, OutT* o, bool act, double X, double Y,
                                            double Z, double S0, double S1, double S2)
 {
     constexpr int NS = AoSets<PASS>::n, NC = ncart(L);
@@ -298,7 +286,7 @@ __device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& s
             double v = 0.0;
 #pragma unroll
             for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
-            if (act) o[a.dst[s] * a.set_stride + r * a.ld] = v;
+            if (act) o[a.dst[s] * a.set_stride + r * a.ld] = (OutT)v;
         }
     };
     set(std::integral_constant<int, 0>{}, 0);
@@ -309,11 +297,67 @@ __device__ __forceinline__ void ao_general(const AoListArgs& a, const ListRec& s
     }
 }
 
+// squared distance from a record's centre to the box (wave-uniform)
+__device__ __forceinline__ double list_dist2(const double (&lo)[3], const double (&hi)[3], const ListRec& sh)
+{
+    double d2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double d = fmax(fmax(lo[k] - sh.c[k], sh.c[k] - hi[k]), 0.0);
+        d2 = fma(d, d, d2);
+    }
+    return uniform(d2);
+}
+
+// the rows of one shell in reach (squared distance d2 to the wave's box) at
+// the lane's point, its first row's place at o
+template <int PASS, typename OutT>
+__device__ __forceinline__ void list_shell(const AoListArgs& a, const ListRec& sh, double d2, double px, double py, double pz,
+                                           OutT* o, bool act)
+{
+    constexpr bool need1 = PASS == 1 || PASS == 2, need2 = PASS >= 2;
+    const double X = px - sh.c[0], Y = py - sh.c[1], Z = pz - sh.c[2];
+    const double rr = X * X + Y * Y + Z * Z;
+    double S0 = 0.0, S1 = 0.0, S2 = 0.0;
+    auto prim = [&](double alpha, double d) {
+        const double de = d * gauss_out<OutT>(alpha * rr);
+        S0 += de;
+        if constexpr (need1) S1 = fma(alpha, de, S1);
+        if constexpr (need2) S2 = fma(alpha * alpha, de, S2);
+    };
+    // the primitives in reach lead (radii descend)
+    if (d2 < sh.prcut2[0]) prim(sh.alpha[0], sh.d[0]);
+    if (d2 < sh.prcut2[1]) prim(sh.alpha[1], sh.d[1]);
+    if (d2 < sh.prcut2[2]) prim(sh.alpha[2], sh.d[2]);
+    if (d2 < sh.prcut2[3]) {
+        prim(sh.alpha[3], sh.d[3]);
+        for (int q = 4; q < sh.nprim; ++q) {
+            const OKMI_CONST PrimGroup* g = cptr(a.more) + sh.more + ((q - 4) >> 2);
+            if (!(d2 < g->rcut2[q & 3])) break;
+            prim(g->alpha[q & 3], g->d[q & 3]);
+        }
+    }
+    S1 *= -2.0;
+    S2 *= 4.0;
+#define OKMI_AO_CASE(L)                                                                              \
+    case L:                                                                                          \
+        if (sh.kind == SHELL_T_GENERAL) ao_general<L, PASS>(a, sh, o, act, X, Y, Z, S0, S1, S2);     \
+        else if (L <= 3 && sh.kind == SHELL_T_SPHERICAL)                                             \
+            ao_rows<(L <= 3 ? L : 0), true, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                   \
+        else ao_rows<L, false, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                                \
+        break;
+    switch (sh.l) {
+        OKMI_AO_CASE(0) OKMI_AO_CASE(1) OKMI_AO_CASE(2) OKMI_AO_CASE(3)
+    default:
+        OKMI_AO_CASE(4)
+    }
+#undef OKMI_AO_CASE
+}
+
 template <int PASS>
 __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a, double* __restrict__ out)
 {
     constexpr int NS = AoSets<PASS>::n;
-    constexpr bool need1 = PASS == 1 || PASS == 2, need2 = PASS >= 2;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t i = (int64_t)blockIdx.x * 64 + lane;
     const bool act = i < a.np;
@@ -330,13 +374,7 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a
     const int end = min(a.nsh, ((int)blockIdx.y + 1) * a.per);
     for (int s = (int)blockIdx.y * a.per + wave; s < end; s += 4) {
         const ListRec sh = load_list(a.shells, s);
-        double d2 = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const double d = fmax(fmax(lo[k] - sh.c[k], sh.c[k] - hi[k]), 0.0);
-            d2 = fma(d, d, d2);
-        }
-        d2 = uniform(d2);
+        const double d2 = list_dist2(lo, hi, sh);
         double* o = out + sh.row0 * a.ld + i;
         if (!(d2 < sh.rcut2)) {   // every value and derivative below the screening bound
             if (act)
@@ -346,42 +384,94 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a
                 }
             continue;
         }
-        const double X = px - sh.c[0], Y = py - sh.c[1], Z = pz - sh.c[2];
-        const double rr = X * X + Y * Y + Z * Z;
-        double S0 = 0.0, S1 = 0.0, S2 = 0.0;
-        auto prim = [&](double alpha, double d) {
-            const double de = d * gauss_f64(alpha * rr);
-            S0 += de;
-            if constexpr (need1) S1 = fma(alpha, de, S1);
-            if constexpr (need2) S2 = fma(alpha * alpha, de, S2);
-        };
-        // the primitives in reach lead (radii descend)
-        if (d2 < sh.prcut2[0]) prim(sh.alpha[0], sh.d[0]);
-        if (d2 < sh.prcut2[1]) prim(sh.alpha[1], sh.d[1]);
-        if (d2 < sh.prcut2[2]) prim(sh.alpha[2], sh.d[2]);
-        if (d2 < sh.prcut2[3]) {
-            prim(sh.alpha[3], sh.d[3]);
-            for (int q = 4; q < sh.nprim; ++q) {
-                const OKMI_CONST PrimGroup* g = cptr(a.more) + sh.more + ((q - 4) >> 2);
-                if (!(d2 < g->rcut2[q & 3])) break;
-                prim(g->alpha[q & 3], g->d[q & 3]);
+        list_shell<PASS>(a, sh, d2, px, py, pz, o, act);
+    }
+}
+
+// Values and first derivatives (PASS 0, 1) of the shells in a tile's live chunks
+// (AoLiveMask), the AO sets of the staged contractions.  The four waves of a
+// workgroup take the same 64 points and every fourth of those shells: with one
+// wave per tile and one scalar load per primitive (each waited for in turn), a
+// pass of 3,277 tiles left the chip a single, latency-bound round of waves.
+// Per pass of 209,664 points x 4 FP32 sets (2,950 AOs): 393 -> 212 us; 512,000
+// points x 1 set (400 AOs): FP64 211 -> 141 us, FP32 152 -> 73 us.
+struct AoLiveArgs {
+    AoListArgs l;               // shells: work order, internal rows
+    const int2* chunks;         // per chunk: first shell, shells | used rows << 16
+    const unsigned long long* mask;
+    int words, shift, quads;    // as AoLiveMask
+    int brick;                  // as AoArgs
+    int64_t bk0, nbx, nby, nbz, tile_stride;
+};
+
+template <int PASS, typename OutT>
+__global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_live(AoLiveArgs a, OutT* __restrict__ out)
+{
+    constexpr int NS = AoSets<PASS>::n;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tile = blockIdx.x;
+    bool act = true;
+    double px, py, pz;
+    if (a.brick) {   // lanes outside the grid repeat its nearest point
+        const GridDesc& g = a.l.grid;
+        unsigned t = (unsigned)(a.bk0 + tile);   // (2^32 bricks would be 2 TB of densities)
+        const unsigned nbz = (unsigned)a.nbz, nby = (unsigned)a.nby;
+        const int64_t bz = t % nbz;
+        t /= nbz;
+        const int64_t by = t % nby, bx = t / nby;
+        const int64_t ix = min(4 * bx + (lane >> 4), g.nx - 1), iy = min(4 * by + ((lane >> 2) & 3), g.ny - 1);
+        const int64_t iz = min(4 * bz + (lane & 3), g.nz - 1);
+        px = g.x[ix]; py = g.y[iy]; pz = g.z[iz];
+    } else {   // (lanes past the end repeat the first point)
+        const int64_t i = tile * 64 + lane;
+        act = i < a.l.np;
+        grid_point(a.l.grid, a.l.p0 + (act ? i : 0), px, py, pz);
+    }
+    double lo[3] = {px, py, pz}, hi[3] = {px, py, pz};
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
+            hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
+        }
+    OutT* base = out + tile * a.tile_stride + lane;
+    const unsigned long long* mrow = a.mask + (tile >> a.shift) * a.words;
+    int skip = wave;   // shells until this wave's next one
+    for (int w = 0; w < a.words; ++w) {
+        const unsigned long long m0 = mrow[w];
+        unsigned long long m = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(m0 >> 32)) << 32) |
+                               (unsigned)__builtin_amdgcn_readfirstlane((unsigned)m0);
+        while (m) {
+            const int bit = __builtin_ctzll(m);
+            int c = 64 * w + bit;
+            unsigned quads = 0xff;   // the chunk's quads that are read
+            if (a.quads) {
+                c >>= 3;
+                quads = (unsigned)(m >> (bit & ~7)) & 0xff;
+                m &= ~(0xffull << (bit & ~7));
+            } else {
+                m &= m - 1;
             }
+            const int2 cw = load_int2(a.chunks, c);
+            const int nsh = cw.y & 0xffff;
+            for (; skip < nsh; skip += 4) {
+                const ListRec sh = load_list(a.l.shells, cw.x + skip);
+                const double d2 = list_dist2(lo, hi, sh);
+                OutT* o = base + sh.row0 * a.l.ld;
+                if (d2 < sh.rcut2) {
+                    list_shell<PASS>(a.l, sh, d2, px, py, pz, o, act);
+                } else if (act) {   // out of the wave's reach: zero rows
+                    for (int q = 0; q < NS; ++q) {
+                        if (a.l.dst[q] < 0) continue;
+                        for (int r = 0; r < sh.nrow; ++r)
+                            if (quads >> (((sh.row0 + r) & 31) >> 2) & 1)
+                                o[a.l.dst[q] * a.l.set_stride + r * a.l.ld] = (OutT)0;
+                    }
+                }
+            }
+            skip -= nsh;
         }
-        S1 *= -2.0;
-        S2 *= 4.0;
-#define OKMI_AO_CASE(L)                                                                              \
-    case L:                                                                                          \
-        if (sh.kind == SHELL_T_GENERAL) ao_general<L, PASS>(a, sh, o, act, X, Y, Z, S0, S1, S2);     \
-        else if (L <= 3 && sh.kind == SHELL_T_SPHERICAL)                                             \
-            ao_rows<(L <= 3 ? L : 0), true, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                   \
-        else ao_rows<L, false, PASS>(a, o, act, X, Y, Z, S0, S1, S2);                                \
-        break;
-        switch (sh.l) {
-            OKMI_AO_CASE(0) OKMI_AO_CASE(1) OKMI_AO_CASE(2) OKMI_AO_CASE(3)
-        default:
-            OKMI_AO_CASE(4)
-        }
-#undef OKMI_AO_CASE
     }
 }
 
@@ -448,7 +538,6 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
         a.live_mask = live->mask;
         a.mask_words = live->words;
         a.mask_shift = live->shift;
-        a.mask_quads = live->quads;
         a.chunks = b->d_chunks;
         a.wshells = live->wshells ? live->wshells : b->d_wshells;
     }
@@ -486,7 +575,29 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
     OkmiProfScope prof("ao_eval", st);
     const bool list = !bricks && !live && out_dtype == OKMI_F64 && shells == b->d_shells && b->d_lshells_a;
     if (list && launch_ao_list(b, g, p0, np, first, (double*)out, ld, set_stride, st)) return 1;
-    for (int grp = 0; grp < 2 && !list; ++grp) {
+    // values and first derivatives of live chunks (second derivatives: k_ao_eval's group 1)
+    if (live) {
+        AoLiveArgs w{};
+        const bool split = live->wshells && live->wshells == b->d_wshells_s;
+        w.l.shells = split ? b->d_wlist_s : b->d_wlist;
+        w.l.more = split ? b->d_wlist_groups_s : b->d_wlist_groups;
+        w.l.T = b->d_T;
+        w.l.grid = g; w.l.p0 = p0; w.l.np = np; w.l.ld = ld; w.l.set_stride = set_stride;
+        for (int c = 0; c < 4; ++c) w.l.dst[c] = first[c];
+        w.chunks = b->d_chunks;
+        w.mask = live->mask; w.words = live->words; w.shift = live->shift; w.quads = live->quads;
+        w.brick = a.brick; w.bk0 = a.bk0; w.nbx = a.nbx; w.nby = a.nby; w.nbz = a.nbz; w.tile_stride = a.tile_stride;
+        const dim3 tiles((unsigned)(bricks ? bricks->nbk : (np + 63) / 64));
+        const bool first_deriv = first[1] >= 0 || first[2] >= 0 || first[3] >= 0;
+        if (out_dtype == OKMI_F64) {
+            if (first_deriv) hipLaunchKernelGGL((k_ao_live<1, double>), tiles, blk, 0, st, w, (double*)out);
+            else if (first[0] >= 0) hipLaunchKernelGGL((k_ao_live<0, double>), tiles, blk, 0, st, w, (double*)out);
+        } else {
+            if (first_deriv) hipLaunchKernelGGL((k_ao_live<1, float>), tiles, blk, 0, st, w, (float*)out);
+            else if (first[0] >= 0) hipLaunchKernelGGL((k_ao_live<0, float>), tiles, blk, 0, st, w, (float*)out);
+        }
+    }
+    for (int grp = live ? 1 : 0; grp < 2 && !list; ++grp) {
         const int c0 = grp == 0 ? 0 : 4, c1 = grp == 0 ? 4 : OKMI_MAX_SETS;
         bool any = false;
         for (int c = 0; c < OKMI_MAX_SETS; ++c) {

@@ -53,6 +53,12 @@ struct OkmiBasis {
     PrimGroup* d_lgroups = nullptr;
     ListRec* d_lshells_a = nullptr;   // the same with the radii of OKMI_SCREEN (MO values)
     PrimGroup* d_lgroups_a = nullptr;
+    // the same records in work order with internal rows, for AO sets of the
+    // live chunks only (radii of OKMI_SCREEN_FUSED and OKMI_SCREEN_SPLIT)
+    ListRec* d_wlist = nullptr;
+    PrimGroup* d_wlist_groups = nullptr;
+    ListRec* d_wlist_s = nullptr;
+    PrimGroup* d_wlist_groups_s = nullptr;
     bool standard = false;   // every shell l <= 3 with real spherical or Cartesian rows
     int nchunk = 0;
     int nkpad = 0;
@@ -90,7 +96,7 @@ struct AoLiveMask {
     const ShellRec* wshells;   // work-order shells of the screening bound in use (null: d_wshells)
     // quads: the masks mark quads (bit q: rows 4 q .. 4 q + 3); a chunk is live
     // if one of its eight is, and a shell out of reach writes zeros only to the
-    // rows of live quads
+    // rows of live quads (codes 0 .. 3)
     bool quads = false;
     int64_t tile_stride = 64;  // range order: column c at tile_stride (c / 64) + c % 64
 };

@@ -1,7 +1,7 @@
 // Density for many MOs (more than the fused kernel keeps in registers).
 // Replaces slice_rho's density branch (orbkit/core.py:179-308) for large
 // NMO: per chunk of points
-//   1. k_ao_eval writes the AO sets of codes 0..S-1 in FP32 (FP64
+//   1. k_ao_live (codes 0..3) and k_ao_eval write the AO sets of codes 0..S-1 in FP32 (FP64
 //      evaluation rounded once), rows coalesced: ao[s][k][p];
 //   2. k_rho_big contracts them with C on the matrix cores.  A workgroup owns
 //      128 MOs x NP points x all S sets; the K loop (AO rows, 32 per step)

@@ -5,7 +5,7 @@
 //   1. k_live_quads lists, per tile of NP points, the 32-row chunks of the fused
 //      row order with a shell in reach, and which of their quads (four
 //      consecutive rows) hold a row of such a shell;
-//   2. k_ao_eval writes the AO sets in FP32 in tiles of 64 points,
+//   2. k_ao_live writes the AO sets in FP32 in tiles of 64 points,
 //      ao[tile of 64][set][row][64], rows of dead quads left unwritten;
 //   3. k_rho_split contracts the listed chunks with C, one K step of the bf16
 //      MFMA each, and reduces its MOs to density terms;

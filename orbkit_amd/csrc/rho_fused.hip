@@ -228,14 +228,15 @@ int prepare_fused_tables(OkmiBasis* b)
     bool standard = true;
     for (int j = 0; j < b->nshell; ++j)
         standard = standard && b->h_shells[j].l <= 3 && b->h_shells[j].kind != SHELL_T_GENERAL;
-    auto list_tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ListRec>& ls,
-                           std::vector<PrimGroup>& more) {
-        ls.resize(b->nshell);
-        for (int j = 0; j < b->nshell; ++j) {
-            const ShellRec& hs = b->h_shells[by_l[j]];
+    auto list_tables = [&](const std::vector<int>& take, bool internal_rows, const std::vector<double>& frc2,
+                           const std::vector<double>& fprc2, std::vector<ListRec>& ls, std::vector<PrimGroup>& more) {
+        ls.resize(take.size());
+        for (size_t j = 0; j < take.size(); ++j) {
+            const int i = take[j];
+            const ShellRec& hs = b->h_shells[i];
             ListRec& r = ls[j];
-            r = ListRec{{hs.cx, hs.cy, hs.cz}, frc2[by_l[j]], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)more.size(),
-                        hs.row0, hs.nrow, hs.t0, hs.l | kind_of(hs) << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
+            r = ListRec{{hs.cx, hs.cy, hs.cz}, frc2[i], {}, {}, {}, hs.l, hs.kind, hs.nprim, (int)more.size(),
+                        internal_rows ? krow[i] : hs.row0, hs.nrow, hs.t0, hs.l | kind_of(hs) << 3 | (hs.kind == SHELL_T_GENERAL ? hs.nrow << 5 : 0)};
             const std::vector<int> order = sorted_prims(hs, fprc2);
             const PrimGroup first = prim_group(order, 0, fprc2);
             for (int k = 0; k < 4; ++k) {
@@ -246,13 +247,15 @@ int prepare_fused_tables(OkmiBasis* b)
             for (int q = 4; q < hs.nprim; q += 4) more.push_back(prim_group(order, q, fprc2));
         }
     };
-    std::vector<ListRec> ls, ls_a;
-    std::vector<PrimGroup> lgroups, lgroups_a;
-    list_tables(b->h_frcut2, b->h_fprcut2, ls, lgroups);
+    std::vector<ListRec> ls, ls_a, ws, ws_s;
+    std::vector<PrimGroup> lgroups, lgroups_a, wgroups, wgroups_s;
+    list_tables(by_l, false, b->h_frcut2, b->h_fprcut2, ls, lgroups);
+    list_tables(work, true, b->h_frcut2, b->h_fprcut2, ws, wgroups);
+    list_tables(work, true, b->h_frcut2s, b->h_fprcut2s, ws_s, wgroups_s);
     std::vector<double> arc2(b->nshell), aprc2(b->nprim);   // radii of OKMI_SCREEN
     for (int i = 0; i < b->nshell; ++i) arc2[i] = b->h_shells[i].rcut2;
     for (int i = 0; i < b->nprim; ++i) aprc2[i] = b->h_prims[i].rcut2;
-    list_tables(arc2, aprc2, ls_a, lgroups_a);
+    list_tables(by_l, false, arc2, aprc2, ls_a, lgroups_a);
     std::vector<ShellRec> os(b->h_shells, b->h_shells + b->nshell);
     for (int i = 0; i < b->nshell; ++i) os[i].rcut2 = b->h_frcut2[i];
     std::vector<int> padrows;
@@ -276,6 +279,10 @@ int prepare_fused_tables(OkmiBasis* b)
     if (!rc) rc = upload(&b->d_lgroups, lgroups, "rho_fused: their primitive groups");
     if (!rc) rc = upload(&b->d_lshells_a, ls_a, "mo_fused: shells by class");
     if (!rc) rc = upload(&b->d_lgroups_a, lgroups_a, "mo_fused: their primitive groups");
+    if (!rc) rc = upload(&b->d_wlist, ws, "ao_eval: work-order shells");
+    if (!rc) rc = upload(&b->d_wlist_groups, wgroups, "ao_eval: their primitive groups");
+    if (!rc) rc = upload(&b->d_wlist_s, ws_s, "ao_eval: work-order shells (FP32 bound)");
+    if (!rc) rc = upload(&b->d_wlist_groups_s, wgroups_s, "ao_eval: their primitive groups (FP32 bound)");
     if (rc) return rc;
     b->standard = standard;
     b->nchunk = nchunk;
