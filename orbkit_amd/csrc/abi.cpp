@@ -354,24 +354,7 @@ extern "C" int okmi_basis_destroy(okmi_basis* b)
     if (b->d_shells) (void)hipFree(b->d_shells);
     if (b->d_prims) (void)hipFree(b->d_prims);
     if (b->d_T) (void)hipFree(b->d_T);
-    if (b->d_chunks) (void)hipFree(b->d_chunks);
-    if (b->d_fshells) (void)hipFree(b->d_fshells);
-    if (b->d_fprims) (void)hipFree(b->d_fprims);
-    if (b->d_fgroups) (void)hipFree(b->d_fgroups);
-    if (b->d_oshells) (void)hipFree(b->d_oshells);
-    if (b->d_ishells) (void)hipFree(b->d_ishells);
-    if (b->d_wshells) (void)hipFree(b->d_wshells);
-    for (void* p : {(void*)b->d_fshells_s, (void*)b->d_ishells_s, (void*)b->d_wshells_s, (void*)b->d_fprims_s,
-                    (void*)b->d_fgroups_s})
-        if (p) (void)hipFree(p);
-    if (b->d_padrows) (void)hipFree(b->d_padrows);
-    if (b->d_colmap) (void)hipFree(b->d_colmap);
-    if (b->d_lshells) (void)hipFree(b->d_lshells);
-    if (b->d_lgroups) (void)hipFree(b->d_lgroups);
-    if (b->d_lshells_a) (void)hipFree(b->d_lshells_a);
-    if (b->d_lgroups_a) (void)hipFree(b->d_lgroups_a);
-    for (void* p : {(void*)b->d_wlist, (void*)b->d_wlist_groups, (void*)b->d_wlist_s, (void*)b->d_wlist_groups_s})
-        if (p) (void)hipFree(p);
+    if (b->d_tables) (void)hipFree(b->d_tables);
     delete[] b->h_shells;
     delete[] b->h_prims;
     delete[] b->h_T;

@@ -29,9 +29,9 @@ struct OkmiBasis {
     // own row order: each shell's rows lie inside one 32-row chunk (zero rows
     // pad the chunks), colmap maps internal rows to output rows (-1: pad),
     // and screening radii for the bound OKMI_SCREEN_FUSED.
+    void* d_tables = nullptr;   // the device allocation that the pointers below point into
     int2* d_chunks = nullptr;   // per chunk: first work entry, shells | used rows << 16
     ShellRec* d_fshells = nullptr;   // row0 = internal row, rcut2 = fused radius
-    ShellRec* d_oshells = nullptr;   // output rows, rcut2 = fused radius
     ShellRec* d_ishells = nullptr;   // internal rows (prim0 into d_fprims), rcut2 = fused radius
     ShellRec* d_wshells = nullptr;   // the same in work order (entry j of a chunk's list is record j)
     int* d_padrows = nullptr;        // internal rows that hold no AO (chunk padding)
@@ -53,8 +53,7 @@ struct OkmiBasis {
     PrimGroup* d_lgroups = nullptr;
     ListRec* d_lshells_a = nullptr;   // the same with the radii of OKMI_SCREEN (MO values)
     PrimGroup* d_lgroups_a = nullptr;
-    // the same records in work order with internal rows, for AO sets of the
-    // live chunks only (radii of OKMI_SCREEN_FUSED and OKMI_SCREEN_SPLIT)
+    // the same records in work order with internal rows (radii of OKMI_SCREEN_FUSED and OKMI_SCREEN_SPLIT)
     ListRec* d_wlist = nullptr;
     PrimGroup* d_wlist_groups = nullptr;
     ListRec* d_wlist_s = nullptr;
@@ -105,8 +104,7 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
                            void* out, int64_t ld, int64_t set_stride, hipStream_t st,
                            const AoLiveMask* live = nullptr);
 
-// fused-path tables (internal row order, fused screening radii) and the
-// output-row shell table with the fused radii (d_oshells); built once
+// fused-path tables (internal row order, fused screening radii); built once
 int okmi_prepare_fused(OkmiBasis* b);
 
 // MO values Phi_s = C A_s for NS sets stored [set][mo][point] (FP64 MFMA)

@@ -503,7 +503,7 @@ int okmi_launch_rho_big(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np,
         }
     const int S = big_sets(drv_out, nout);
     const BigLayout L = big_layout(b, nmo, prec, S);
-    int rc0 = okmi_prepare_fused(b);   // output-row shells and primitives with the fused radii
+    int rc0 = okmi_prepare_fused(b);
     if (rc0) return rc0;
     if (prec != OKMI_PREC_F32 && S <= 4)
         return okmi_launch_rho_big_split(b, g, p0, np, d_c, d_occ, nmo, prec, S, drv_out, nout, rho, delta, ld_delta, ws,

@@ -5,6 +5,8 @@
 // instances are compiled in rho_fused_f64.hip.
 #include "fused_tile.h"
 
+#include <cstring>
+
 namespace {
 
 using namespace okmi_fused;
@@ -56,6 +58,33 @@ int upload(T** d, const std::vector<T>& h, const char* what)
     if (e != hipSuccess) return okmi_hip_fail(e, what);
     return 0;
 }
+
+// Host tables gathered into one device allocation (256-byte aligned parts)
+struct TableUpload {
+    std::vector<char> host;
+    std::vector<std::pair<void**, size_t>> parts;   // pointer to set, its offset
+
+    template <typename T>
+    void add(T** d, const std::vector<T>& h)
+    {
+        const size_t at = align256(host.size());
+        host.resize(at + std::max<size_t>(1, sizeof(T) * h.size()));
+        if (!h.empty()) std::memcpy(host.data() + at, h.data(), sizeof(T) * h.size());
+        parts.push_back({(void**)d, at});
+    }
+    int run(void** base, const char* what)
+    {
+        hipError_t e = hipMalloc(base, host.size());
+        if (e != hipSuccess) {
+            *base = nullptr;
+            return okmi_hip_fail(e, what);
+        }
+        e = hipMemcpy(*base, host.data(), host.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) return okmi_hip_fail(e, what);
+        for (auto& p : parts) *p.first = (char*)*base + p.second;
+        return 0;
+    }
+};
 
 // Internal row layout of the fused kernels: every 32-row chunk holds whole
 // shells, packed from its first row.  A tile skips the contraction of every
@@ -256,33 +285,33 @@ int prepare_fused_tables(OkmiBasis* b)
     for (int i = 0; i < b->nshell; ++i) arc2[i] = b->h_shells[i].rcut2;
     for (int i = 0; i < b->nprim; ++i) aprc2[i] = b->h_prims[i].rcut2;
     list_tables(by_l, false, arc2, aprc2, ls_a, lgroups_a);
-    std::vector<ShellRec> os(b->h_shells, b->h_shells + b->nshell);
-    for (int i = 0; i < b->nshell; ++i) os[i].rcut2 = b->h_frcut2[i];
     std::vector<int> padrows;
     for (int r = 0; r < nkpad; ++r)
         if (colmap[r] < 0) padrows.push_back(r);
-    int rc = upload(&b->d_chunks, ch, "rho_fused: chunk map");
-    if (!rc) rc = upload(&b->d_fshells, fs, "rho_fused: shells");
-    if (!rc) rc = upload(&b->d_fprims, fp, "rho_fused: primitives");
-    if (!rc) rc = upload(&b->d_fgroups, groups, "rho_fused: primitive groups");
-    if (!rc) rc = upload(&b->d_oshells, os, "rho_fused: output-row shells");
-    if (!rc) rc = upload(&b->d_ishells, is, "rho_fused: internal-row shells");
-    if (!rc) rc = upload(&b->d_wshells, wsh, "rho_fused: work-order shells");
-    if (!rc) rc = upload(&b->d_padrows, padrows, "rho_fused: padding rows");
-    if (!rc) rc = upload(&b->d_colmap, colmap, "rho_fused: row map");
-    if (!rc) rc = upload(&b->d_fshells_s, fs_s, "rho_fused: shells (FP32 bound)");
-    if (!rc) rc = upload(&b->d_fgroups_s, groups_s, "rho_fused: primitive groups (FP32 bound)");
-    if (!rc) rc = upload(&b->d_ishells_s, is_s, "rho_fused: internal-row shells (FP32 bound)");
-    if (!rc) rc = upload(&b->d_wshells_s, wsh_s, "rho_fused: work-order shells (FP32 bound)");
-    if (!rc) rc = upload(&b->d_fprims_s, fp_s, "rho_fused: primitives (FP32 bound)");
-    if (!rc) rc = upload(&b->d_lshells, ls, "rho_fused: shells by class");
-    if (!rc) rc = upload(&b->d_lgroups, lgroups, "rho_fused: their primitive groups");
-    if (!rc) rc = upload(&b->d_lshells_a, ls_a, "mo_fused: shells by class");
-    if (!rc) rc = upload(&b->d_lgroups_a, lgroups_a, "mo_fused: their primitive groups");
-    if (!rc) rc = upload(&b->d_wlist, ws, "ao_eval: work-order shells");
-    if (!rc) rc = upload(&b->d_wlist_groups, wgroups, "ao_eval: their primitive groups");
-    if (!rc) rc = upload(&b->d_wlist_s, ws_s, "ao_eval: work-order shells (FP32 bound)");
-    if (!rc) rc = upload(&b->d_wlist_groups_s, wgroups_s, "ao_eval: their primitive groups (FP32 bound)");
+    // one allocation and one copy for all of them
+    TableUpload up;
+    up.add(&b->d_chunks, ch);
+    up.add(&b->d_fshells, fs);
+    up.add(&b->d_fprims, fp);
+    up.add(&b->d_fgroups, groups);
+    up.add(&b->d_fgroups_s, groups_s);
+    up.add(&b->d_ishells, is);
+    up.add(&b->d_wshells, wsh);
+    up.add(&b->d_padrows, padrows);
+    up.add(&b->d_colmap, colmap);
+    up.add(&b->d_fshells_s, fs_s);
+    up.add(&b->d_ishells_s, is_s);
+    up.add(&b->d_wshells_s, wsh_s);
+    up.add(&b->d_fprims_s, fp_s);
+    up.add(&b->d_lshells, ls);
+    up.add(&b->d_lgroups, lgroups);
+    up.add(&b->d_lshells_a, ls_a);
+    up.add(&b->d_lgroups_a, lgroups_a);
+    up.add(&b->d_wlist, ws);
+    up.add(&b->d_wlist_groups, wgroups);
+    up.add(&b->d_wlist_s, ws_s);
+    up.add(&b->d_wlist_groups_s, wgroups_s);
+    const int rc = up.run(&b->d_tables, "rho_fused: tables");
     if (rc) return rc;
     b->standard = standard;
     b->nchunk = nchunk;
