@@ -232,7 +232,8 @@ def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
       dom = ('rho_fused_f64', 'k_rho_fused', 'f64', 1)
     elif nmo > 64:
       names = ['ao_eval', 'rho_big']
-      dom = ('rho_big', 'k_rho_big', 'f32' if path == 'f32' else 'bf16', PRODUCTS[path])
+      big = 'k_rho_big' if path == 'f32' or max(codes, default=0) > 3 else 'k_rho_split'
+      dom = ('rho_big', big, 'f32' if path == 'f32' else 'bf16', PRODUCTS[path])
     else:
       names = ['rho_fused']
       dom = ('rho_fused', 'k_rho_fused', 'f32' if path == 'f32' else 'bf16', PRODUCTS[path])
