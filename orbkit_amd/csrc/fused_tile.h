@@ -1,8 +1,7 @@
 // Tile body of the fused density kernels: AO evaluation -> LDS -> MFMA
 // contraction with the MO coefficients -> density terms, in one launch.  MOs
-// never leave registers.  Shared by the single-molecule kernels (split and
-// FP32 precisions in rho_fused.hip, FP64 in rho_fused_f64.hip) and the batch
-// kernel.
+// never leave registers.  Shared by the single-molecule and batch kernels of the
+// FP32 and split precisions (rho_fused.hip); FP64 has its own (fused_f64.h).
 //
 // A workgroup of four waves owns a tile of 64 grid points: a 4x4x4 brick of a
 // regular grid (compact in space) or 64 consecutive points of a vector grid.
@@ -10,19 +9,16 @@
 // For each chunk the four waves take the chunk's shells one at a time from a
 // shared counter, costliest first (lane = point), and evaluate them in FP64
 // (coordinates, exponentials, polynomials, the Cartesian-to-spherical map),
-// storing each value in LDS [row][point]: rounded once to FP32 for the
-// reduced precisions, in FP64 (with the full-accuracy exponential) for the
-// FP64 contraction.  Reduced precisions use one buffer and three workgroups
+// storing each value in LDS [row][point], rounded once to FP32: one buffer and three workgroups
 // per CU for rho / rho + grad rho with l <= 3, with the chunk's C columns
-// shared through LDS, else double buffering with one barrier per chunk; FP64
-// uses one 64 KB buffer and two workgroups per CU (see FusedPlan).  Each wave
+// shared through LDS, else double buffering with one barrier per chunk (see
+// FusedPlan).  Each wave
 // then multiplies the rows of its 16-point column with the matching 32
 // columns of C:
-//   F64     v_mfma_f64_16x16x4_f64, C and AO in FP64, FP64 accumulation
 //   F32     v_mfma_f32_16x16x4_f32, C and AO in FP32
 //   BF16X3  v_mfma_f32_16x16x32_bf16 on (hi, lo) splits, 3 products
 //   BF16X6  (hi, mid, lo) splits, 6 products (terms below 2^-24 dropped)
-// accumulating in FP32 except F64.  The epilogue forms the density terms in
+// accumulating in FP32.  The epilogue forms the density terms in
 // FP64.
 //
 // Screening: a shell whose screening radius (every value and derivative
@@ -64,12 +60,7 @@ template <int PREC> struct Tile {
     using Acc = f4;
     static constexpr int LD = 65;
 };
-template <> struct Tile<OKMI_PREC_F64> {
-    using T = double;
-    using Acc = d4;
-    static constexpr int LD = 64;
-};
-template <typename T> constexpr int tile_ld() { return std::is_same<T, double>::value ? 64 : 65; }
+template <typename T> constexpr int tile_ld() { return 65; }
 
 struct FusedArgs {
     const ShellRec* shells;   // in work order: per chunk its shells, costliest first
@@ -342,20 +333,12 @@ template <int PREC, int MT>
 struct COperand {
     Split<PREC> ca[MT];
     float cf[MT][KC / 4];
-    double cd[PREC == OKMI_PREC_F64 ? MT : 1][KC / 4];
 };
 
 template <int PREC, int MT>
 __device__ __forceinline__ void load_c(const FusedArgs& a, int k0, int g, int n16, COperand<PREC, MT>& c)
 {
-    if constexpr (PREC == OKMI_PREC_F64) {
-        const double* C = (const double*)a.C;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int ks = 0; ks < KC / 4; ++ks)
-                c.cd[mt][ks] = C[(int64_t)(mt * 16 + n16) * a.kpad + k0 + 4 * ks + g];
-    } else if constexpr (PREC == OKMI_PREC_F32) {
+    if constexpr (PREC == OKMI_PREC_F32) {
         // K step ks of lane group g takes chunk row 8 g + ks (the same in
         // contract), so a lane's 8 values are contiguous: two 16-byte loads
         const float* C = (const float*)a.C;
@@ -501,15 +484,7 @@ __device__ __forceinline__ void contract(const typename Tile<PREC>::T* L, int co
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const typename Tile<PREC>::T* src = L + s * KC * LD + col * 16 + n16;
-        if constexpr (PREC == OKMI_PREC_F64) {
-#pragma unroll
-            for (int ks = 0; ks < KC / 4; ++ks) {
-                const double b = src[(4 * ks + g) * LD];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    if (mt < nmt) acc[mt][s] = __builtin_amdgcn_mfma_f64_16x16x4f64(c.cd[mt][ks], b, acc[mt][s], 0, 0, 0);
-            }
-        } else if constexpr (PREC == OKMI_PREC_F32) {
+        if constexpr (PREC == OKMI_PREC_F32) {
 #pragma unroll
             for (int ks = 0; ks < KC / 4; ++ks) {
                 const float b = src[(8 * g + ks) * LD];   // chunk row 8 g + ks, as load_c
@@ -532,8 +507,7 @@ __device__ __forceinline__ void contract(const typename Tile<PREC>::T* L, int co
 
 // Density terms of the 16-point column `col` of the tile from its MO values:
 // item i of the lane holds Phi[m][tile point 16 col + n16] with
-// m = 16 mt + 4 g + i (FP32 accumulator layout) or m = 16 mt + 4 i + g
-// (v_mfma_f64_16x16x4f64 leaves D[4 i + lane / 16][lane % 16] in item i).
+// m = 16 mt + 4 g + i.
 template <int PREC, int PASS, int MT>
 __device__ __forceinline__ void epilogue(const FusedArgs& a, int64_t tile, int col, int lane,
                                          const typename Tile<PREC>::Acc (&acc)[MT][PassCodes<PASS>::n])
@@ -549,7 +523,7 @@ __device__ __forceinline__ void epilogue(const FusedArgs& a, int64_t tile, int c
     for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const double w = a.occ[mt * 16 + (PREC == OKMI_PREC_F64 ? 4 * i + g : 4 * g + i)];
+            const double w = a.occ[mt * 16 + 4 * g + i];
             const double f0 = acc[mt][0][i];
             if constexpr (PASS <= 1) r0 += w * (f0 * f0);
             if constexpr (NS > 1) {
@@ -689,19 +663,17 @@ __device__ __forceinline__ int next_live(const FusedArgs& a, const unsigned long
 // which needs a few more registers) fit in 168 VGPRs without spilling (33 KB
 // AO tile plus up to 11.5 KB of C stage) and run at 3 waves/SIMD; the others
 // keep two buffers (66.5 KB, 2 waves/SIMD), where holding C through the
-// evaluation hides its latency.  FP64 always has one buffer (64 KB for four
-// AO sets) and two workgroups per CU.  FP64 and FP32 load their C operand
-// into registers before the evaluation and hold it through it (hold_c).
+// evaluation hides its latency.  FP32 loads its C operand into registers
+// before the evaluation and may hold it through it (hold_c).
 template <int PREC, int PASS, int LM, int MT, bool BATCH> struct FusedPlan {
-    static constexpr bool f64 = PREC == OKMI_PREC_F64;
-    static constexpr bool single = f64 || (PASS <= 1 && LM <= 3 && MT <= (BATCH ? 2 : 3));
+    static constexpr bool single = PASS <= 1 && LM <= 3 && MT <= (BATCH ? 2 : 3);
     static constexpr int buffers = single ? 1 : 2;
-    static constexpr int occupancy = f64 ? 2 : single ? 3 : 2;
-    static constexpr bool c_early = f64 ? MT <= 3 : PASS <= 1 ? MT <= 3 : MT <= 2;
-    // one-buffer schedule, C in registers (FP64, FP32): loaded before the
+    static constexpr int occupancy = single ? 3 : 2;
+    static constexpr bool c_early = PASS <= 1 ? MT <= 3 : MT <= 2;
+    // one-buffer schedule, C in registers (FP32): loaded before the
     // evaluation and held through it, its latency hidden there (FP32 with 3
     // MO tiles and four AO sets would exceed the 168-VGPR budget)
-    static constexpr bool hold_c = c_early && (f64 || (PREC == OKMI_PREC_F32 && (PASS == 0 || MT <= 2)));
+    static constexpr bool hold_c = c_early && PREC == OKMI_PREC_F32 && (PASS == 0 || MT <= 2);
 };
 
 // One tile of 64 points by four waves that all evaluate and all contract:
@@ -819,7 +791,7 @@ int launch_mt(const FusedArgs& a, int mt, hipStream_t st)
         return 1;
     }
     dim3 blk(256), grd((unsigned)ntile);
-    OkmiProfScope prof(PREC == OKMI_PREC_F64 ? "rho_fused_f64" : "rho_fused", st);
+    OkmiProfScope prof("rho_fused", st);
     switch (mt) {
     case 1: hipLaunchKernelGGL((k_rho_fused<PREC, PASS, 1, LM>), grd, blk, 0, st, a); return 0;
     case 2: hipLaunchKernelGGL((k_rho_fused<PREC, PASS, 2, LM>), grd, blk, 0, st, a); return 0;
