@@ -131,9 +131,9 @@ template <int NT, int NR> struct CWhere {
         rs = a.ct ? 8 * a.ct_ld : 8;
         const int last = (a.ct ? mp : a.nmo) - 1;
         mt = n16 * ms;
-        mtl = NR == 0 ? min(n16, last - 16 * (NT - 1)) * ms : mt;
+        mtl = NR == 0 ? last_tile_mo(n16, last, NT) * ms : mt;
         mr = (n16 & 3) * ms;
-        mrl = min(n16 & 3, last - 16 * NT - 4 * (NR - 1)) * ms;
+        mrl = last_group_mo(n16 & 3, last, NT, NR) * ms;
     }
     __device__ __forceinline__ void shell(unsigned row0)
     {

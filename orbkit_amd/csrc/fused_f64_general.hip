@@ -10,7 +10,7 @@ int launch_f64_general(const F64Args& a, int pass, hipStream_t st)
     case 1: return launch_f64_units<1, false, false, 4, 8, 12, 16>(a, st);
     case 2: return launch_f64_units<2, false, false, 4, 8, 12, 16>(a, st);
     case 3: return launch_f64_units<3, false, false, 4, 8, 12, 16>(a, st);
-    default: return launch_f64_units<4, false, false, 4, 8, 10>(a, st);
+    default: return launch_f64_units<4, false, false, 4, 8, 9, 10>(a, st);
     }
 }
 

@@ -38,6 +38,7 @@
 #pragma once
 #include "okmi_internal.h"
 #include "ao_device.h"
+#include "c_place.h"
 #include "split_mfma.h"
 
 #include <type_traits>
@@ -818,16 +819,7 @@ int launch_pass(const FusedArgs& a, int pass, int mt, int lm, hipStream_t st)
     }
 }
 
-// Launches of the FP64 kernel (fused_f64.h; instances compiled in several
-// files).  Groups of 4 MOs that a pass has an instance for, from the groups
-// asked for: every count for rho and rho with first derivatives of standard
-// bases (l <= 3, real spherical or Cartesian rows), and up to 10 for the pass of
-// seven AO sets; multiples of 4 for the others; MO values: every second count.
-inline int f64_units(int u, int pass, bool standard, bool mo)
-{
-    if (!standard || pass == 2 || pass == 3) return pass == 4 && u > 8 ? 10 : (u + 3) & ~3;
-    return mo && u > 2 ? (u + 1) & ~1 : u;
-}
+// Launches of the FP64 kernel (fused_f64.h; instances compiled in several files)
 int launch_f64_p0(const F64Args& a, hipStream_t st);   // standard bases
 int launch_f64_p1(const F64Args& a, hipStream_t st);
 int launch_f64_p4(const F64Args& a, hipStream_t st);
