@@ -32,4 +32,12 @@ __host__ __device__ inline int last_group_mo(int n4, int last, int NT, int NR)
     return n4 < most ? n4 : most > 0 ? most : 0;
 }
 
+// Row of a shell of N rows that place w = 0 .. W - 1 gives to the K step of rows
+// R .. R + W - 1 (the W lane groups of split_rows); places past the last row
+// repeat it
+template <int W> __host__ __device__ constexpr int split_row(int R, int w, int N)
+{
+    return R + W <= N ? R + w : R + w < N ? R + w : N - 1;
+}
+
 }  // namespace okmi_fused

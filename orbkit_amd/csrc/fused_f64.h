@@ -197,7 +197,8 @@ __device__ __forceinline__ void take(bool on, const double (&t)[NS], double (&v)
 // Rows of one (W = 4) or two (W = 2) standard shells left over at the end of
 // their class, each held by W lane groups: group w of a shell's W (lane's w)
 // gives row R + w to the K step, so the shell takes 1 / W of the K steps that a
-// quad with empty places would.  `row`: the shell's first C row; c: row w.
+// quad with empty places would.  `row`: the shell's first C row; c: row
+// split_row(0, w).
 template <int PASS, int W, int L, bool SPH, int R, int NT, int NR, int NS>
 __device__ __forceinline__ void split_rows(const RowSets<L, SPH, PASS>& rows, CWhere<NT, NR>& cw, unsigned row, int w,
                                            const COps<NT, NR>& c, MoAcc<NT, NR, NS>& acc)
@@ -206,8 +207,7 @@ __device__ __forceinline__ void split_rows(const RowSets<L, SPH, PASS>& rows, CW
     if constexpr (R < N) {
         COps<NT, NR> next;
         if constexpr (R + W < N) {
-            // (places past the last row repeat it)
-            cw.shell(row + R + W + (R + 2 * W <= N ? w : min(w, N - 1 - R - W)));
+            cw.shell(row + split_row<W>(R + W, w, N));
             cw.load(0, next);
         }
         double v[NS], t[NS];
@@ -414,7 +414,8 @@ __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* en
         const int live = W > 1 || mine ? rowlive >> LIST_ROW_BITS : 0;
         s += n;
         const unsigned row = rowlive & LIST_ROW_MASK;
-        cw.shell(row + w);
+        if constexpr (W > 1) cw.shell(row + split_row<W>(0, w, shell_rows<L, KIND == SHELL_T_SPHERICAL>()));
+        else cw.shell(row);
         COps<M::NT, M::NR> c;
         cw.load(0, c);
         const double X = px - e->c[0], Y = py - e->c[1], Z = pz - e->c[2];
