@@ -106,7 +106,11 @@ struct Plan {
     // MOs of a launch of the first pass, and width of C^T (the last group's
     // padding included)
     int64_t mp(int pass) const { return 4 * (int64_t)f64_units(u, pass, standard, false); }
-    int64_t mpt() const { return (groups - 1) * 4 * (int64_t)u + std::max(mp(first()), p2 || p3 ? mp(3) : 0); }
+    int64_t mpt() const
+    {
+        const int64_t more = (p2 && !p4) || p3 ? mp(3) : 0;   // the passes after the first
+        return (groups - 1) * 4 * (int64_t)u + std::max(mp(first()), more);
+    }
     size_t c_bytes(const OkmiBasis* b, int nmo) const
     {
         const size_t n = align256(8 * (size_t)b->nao * mpt());
