@@ -487,8 +487,6 @@ int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np
     a.more = b->d_lgroups_a;
     a.T = b->d_T;
     a.grid = g;
-    a.p0 = p0;
-    a.np = np;
     a.ld = ld;
     a.set_stride = set_stride;
     a.nsh = b->nshell;
@@ -496,7 +494,15 @@ int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np
     // (at least two shells per wave)
     const int64_t parts = std::max<int64_t>(1, std::min<int64_t>((AO_WAVES / 4 + blocks - 1) / blocks, b->nshell / 8));
     a.per = (int)((b->nshell + parts - 1) / parts);
-    const dim3 grd((unsigned)blocks, (unsigned)((b->nshell + a.per - 1) / a.per)), blk(256);
+    const dim3 blk(256);
+    auto launch = [&](auto pass) {
+        for (int64_t t = 0; t < blocks; t += OKMI_MAX_BLOCKS) {
+            a.p0 = p0 + 64 * t;
+            a.np = std::min(np - 64 * t, 64 * OKMI_MAX_BLOCKS);
+            const dim3 grd((unsigned)((a.np + 63) / 64), (unsigned)((b->nshell + a.per - 1) / a.per));
+            hipLaunchKernelGGL((k_ao_list<decltype(pass)::value>), grd, blk, 0, st, a, out + 64 * t);
+        }
+    };
     bool value = first[0] >= 0;   // written by the first pass launched
     auto pass = [&](int c1) {     // codes c1 .. c1 + 2
         bool any = false;
@@ -509,12 +515,12 @@ int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np
         value = false;
         return true;
     };
-    if (pass(1)) hipLaunchKernelGGL((k_ao_list<1>), grd, blk, 0, st, a, out);
-    if (pass(4)) hipLaunchKernelGGL((k_ao_list<2>), grd, blk, 0, st, a, out);
-    if (pass(7)) hipLaunchKernelGGL((k_ao_list<3>), grd, blk, 0, st, a, out);
+    if (pass(1)) launch(std::integral_constant<int, 1>{});
+    if (pass(4)) launch(std::integral_constant<int, 2>{});
+    if (pass(7)) launch(std::integral_constant<int, 3>{});
     if (value) {
         a.dst[0] = first[0];
-        hipLaunchKernelGGL((k_ao_list<0>), grd, blk, 0, st, a, out);
+        launch(std::integral_constant<int, 0>{});
     }
     return 0;
 }

@@ -474,7 +474,8 @@ __global__ __launch_bounds__(256, (MoSplit<PASS, U, STD>::OCC)) void k_fused_f64
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n16 = lane & 15;
-    const TileWhere W(a, blockIdx.x);
+    const unsigned tile = a.tile0 + blockIdx.x;
+    const TileWhere W(a, tile);
     double px, py, pz;
     W.point(a, lane, px, py, pz);   // lane l of every wave: point l of the tile, for its box
     double qx, qy, qz;
@@ -530,22 +531,26 @@ __global__ __launch_bounds__(256, (MoSplit<PASS, U, STD>::OCC)) void k_fused_f64
             if (a.norm_part) {   // uniform: every thread takes the branch or none
                 int64_t p;
                 const bool act = W.index(a, wave * 16 + n16, p);
-                tile_norms<PASS, U, STD>(a, blockIdx.x, wave, lane, act, norms, acc);
+                tile_norms<PASS, U, STD>(a, tile, wave, lane, act, norms, acc);
             }
         }
     }
 }
 
 template <int PASS, bool STD, int U, bool MO>
-int launch_f64_one(const F64Args& a, hipStream_t st)
+int launch_f64_one(F64Args a, hipStream_t st)
 {
     if (a.ntile >= ((int64_t)1 << 31)) {   // one workgroup per tile; brick indices are 32-bit
         okmi_set_error("rho_fused: %lld tiles of 64 points (at most 2^31 - 1 per call)", (long long)a.ntile);
         return 1;
     }
-    if (a.ntile == 0) return 0;
     OkmiProfScope prof(MO ? "mo_fused_f64" : "rho_fused_f64", st);
-    hipLaunchKernelGGL((k_fused_f64<PASS, U, STD, MO>), dim3((unsigned)a.ntile), dim3(256), 0, st, a);
+    // (a launch holds fewer than 2^32 threads)
+    for (int64_t t = 0; t < a.ntile; t += OKMI_MAX_BLOCKS) {
+        a.tile0 = (unsigned)t;
+        const unsigned n = (unsigned)std::min(a.ntile - t, OKMI_MAX_BLOCKS);
+        hipLaunchKernelGGL((k_fused_f64<PASS, U, STD, MO>), dim3(n), dim3(256), 0, st, a);
+    }
     return 0;
 }
 

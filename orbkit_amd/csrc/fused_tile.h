@@ -113,6 +113,7 @@ struct F64Args {
     int term_row[10];
     int brick;                // regular grid in bricks of 4x4x4 points (p0 = 0, all points)
     int64_t ntile;            // tiles of 64 points
+    unsigned tile0;           // first one of the launch
     FastDiv dz, dy;           // bricks per axis
     double* norm_part;        // per tile sum_p Phi_m(p)^2, [tile][groups of 4 MOs x 4] (null: not wanted)
 

@@ -6,6 +6,10 @@
 #define OKMI_MAX_L 4          // s..g, the range orbkit's tables cover
 #define OKMI_MAX_SETS 10      // derivative codes 0..9
 
+// Workgroups of 256 threads in a launch that may have a workgroup per 64 points:
+// a launch holds fewer than 2^32 threads, which 2^30 points would reach.
+constexpr int64_t OKMI_MAX_BLOCKS = (int64_t)1 << 23;
+
 // One contracted shell as the kernels see it (wave-uniform record, read
 // through the scalar cache).  Cartesian components are always evaluated in
 // the canonical (molden) order of orbkit/tools.py:117-135; the per-shell
