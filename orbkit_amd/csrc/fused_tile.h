@@ -101,7 +101,7 @@ struct F64Args {
     GridDesc grid;
     int64_t p0, np;
     const double* C;          // [nmo][nao]
-    const double* ct;         // C^T, rows ct_ld doubles apart, this launch's MOs zero padded to 4; null: C is read as it is
+    const double* ct;         // C^T of this launch's MOs, rows ct_ld doubles apart, zero padded; null: C is read as it is
     int ct_ld;
     int add;                  // 1: the launch adds its MOs' terms to the outputs
     const double* occ;        // [nmo]

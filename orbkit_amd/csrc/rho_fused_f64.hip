@@ -51,20 +51,25 @@ using namespace okmi_fused;
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// C [nmo][nao] -> [nao][mpad], zero padded: one 32 x 32 block per workgroup of
-// 256 threads, through LDS
-__global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, int nao, int mpad, double* out)
+// C [nmo][nao] -> [group][nao][width], group g its MOs from `step` g on, zero
+// padded: one 32 x 32 block per workgroup of 256 threads, through LDS.  (A matrix
+// per group: rows of at most 64 MOs, which the kernel's 32-bit offsets reach for
+// any basis; rows of all MOs passed 4 GiB at 25,000 AOs x 21,500 MOs.)
+__global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, int nao, int step, int width, double* out)
 {
     __shared__ double t[32][33];
-    const int r0 = 32 * blockIdx.x, m0 = 32 * blockIdx.y;
+    const int r0 = 32 * blockIdx.x, m0 = 32 * blockIdx.y, g0 = step * blockIdx.z;
+    const int have = min(step, nmo - g0);
+    C += (int64_t)g0 * nao;
+    out += (int64_t)blockIdx.z * nao * width;
     for (int i = threadIdx.x; i < 1024; i += 256) {
         const int m = m0 + i / 32, r = r0 + i % 32;
-        t[i / 32][i % 32] = m < nmo && r < nao ? C[(int64_t)m * nao + r] : 0.0;
+        t[i / 32][i % 32] = m < have && r < nao ? C[(int64_t)m * nao + r] : 0.0;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 1024; i += 256) {
         const int r = r0 + i / 32, m = m0 + i % 32;
-        if (r < nao && m < mpad) out[(int64_t)r * mpad + m] = t[i % 32][i / 32];
+        if (r < nao && m < width) out[(int64_t)r * width + m] = t[i % 32][i / 32];
     }
 }
 
@@ -103,17 +108,12 @@ struct Plan {
         u = ((nmo + groups - 1) / groups + 3) / 4;
     }
     int first() const { return p4 ? 4 : p1 ? 1 : 0; }
-    // MOs of a launch of the first pass, and width of C^T (the last group's
-    // padding included)
+    // MOs of a launch of a pass, and of a group's C^T (the padding of every pass)
     int64_t mp(int pass) const { return 4 * (int64_t)f64_units(u, pass, standard, false); }
-    int64_t mpt() const
-    {
-        const int64_t more = (p2 && !p4) || p3 ? mp(3) : 0;   // the passes after the first
-        return (groups - 1) * 4 * (int64_t)u + std::max(mp(first()), more);
-    }
+    int64_t width() const { return std::max(mp(first()), (p2 && !p4) || p3 ? mp(3) : 0); }
     size_t c_bytes(const OkmiBasis* b, int nmo) const
     {
-        const size_t n = align256(8 * (size_t)b->nao * mpt());
+        const size_t n = align256(8 * (size_t)b->nao * groups * width());
         return nmo <= 64 ? std::max(n, okmi_fused_c_bytes(b, nmo, OKMI_PREC_F64)) : n;
     }
     size_t slack(bool norms) const { return 256 + (norms ? 256 + (size_t)mp(first()) * 8 : 0); }
@@ -134,10 +134,11 @@ F64Args basis_args(const OkmiBasis* b, const GridDesc& g, int nmo, const double*
     return f;
 }
 
-void transpose_c(const OkmiBasis* b, const double* d_c, int nmo, int64_t mpt, double* out, hipStream_t st)
+void transpose_c(const OkmiBasis* b, const double* d_c, int nmo, int groups, int step, int64_t width, double* out,
+                 hipStream_t st)
 {
-    hipLaunchKernelGGL(k_transpose_c, dim3((unsigned)((b->nao + 31) / 32), (unsigned)((mpt + 31) / 32)), dim3(256), 0, st,
-                       d_c, nmo, b->nao, (int)mpt, out);
+    hipLaunchKernelGGL(k_transpose_c, dim3((unsigned)((b->nao + 31) / 32), (unsigned)((width + 31) / 32), (unsigned)groups),
+                       dim3(256), 0, st, d_c, nmo, b->nao, step, (int)width, out);
 }
 
 }  // namespace
@@ -187,8 +188,8 @@ int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0,
     f.np = std::min(np, chunk);
     f.set_bricks(brick);
     if (pl.groups > 1 || f.ntile * (1 + (pl.p2 && !pl.p4) + pl.p3) >= TRANSPOSE_TILES) {
-        transpose_c(b, d_c, nmo, pl.mpt(), ct, st);
-        f.ct_ld = (int)pl.mpt();
+        transpose_c(b, d_c, nmo, pl.groups, (int)step, pl.width(), ct, st);
+        f.ct_ld = (int)pl.width();
     }
     if (pl.direct) {
         f.ld_term = ld_delta;
@@ -212,7 +213,7 @@ int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0,
             f.nmo = std::min<int>(nmo - m0, (int)step);
             f.C = d_c + (int64_t)m0 * b->nao;
             f.occ = d_occ + m0;
-            if (f.ct_ld) f.ct = ct + m0;
+            if (f.ct_ld) f.ct = ct + (int64_t)gr * b->nao * f.ct_ld;
             f.norm_part = norm_part;   // read by the first pass (rho) only
             int r = launch_rho_f64(f, pl.u, pl.first(), b->standard, st);
             if (!r && pl.p2 && !pl.p4) r = launch_rho_f64(f, pl.u, 2, b->standard, st);
@@ -239,12 +240,12 @@ int okmi_launch_mo_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, 
 {
     const int groups = (nmo + 63) / 64, u = ((nmo + groups - 1) / groups + 3) / 4, step = 4 * u;
     double* ct = (double*)(((uintptr_t)ws + 255) & ~(uintptr_t)255);
-    const int64_t mpt = (groups - 1) * step + 64;   // (the widest instance's padding included)
-    transpose_c(b, d_c, nmo, mpt, ct, st);
+    const int64_t width = 4 * (int64_t)f64_units(u, 3, b->standard, true);   // (the widest instance's)
+    transpose_c(b, d_c, nmo, groups, step, width, ct, st);
     F64Args f = basis_args(b, g, nmo, d_c);
     f.shells = b->d_lshells_a;
     f.more = b->d_lgroups_a;
-    f.ct_ld = (int)mpt;
+    f.ct_ld = (int)width;
     f.p0 = p0;
     f.np = np;
     f.set_bricks(g.regular && p0 == 0 && np == g.nx * g.ny * g.nz);
@@ -265,7 +266,7 @@ int okmi_launch_mo_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, 
             const int m0 = gr * step;
             if (m0 >= nmo) break;
             f.nmo = std::min(nmo - m0, step);
-            f.ct = ct + m0;
+            f.ct = ct + (int64_t)gr * b->nao * width;
             f.term = d_mo + (int64_t)m0 * ld_mo;
             f.units = f64_units(u, pass, b->standard, true);
             const int r = launch_mo_f64(f, pass, b->standard, st);
