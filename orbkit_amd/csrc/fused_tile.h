@@ -241,9 +241,11 @@ __device__ __forceinline__ void prim_sums(const PrimGroup& pg, double rr, double
 
 // Rows of a shell of one pass into the LDS tile from its first row's place,
 // AO sets SS elements apart (rounded once to T).  SETS (values alone): rows from
-// the Cartesian values, set by set (the same values bit for bit).  Taken for FP32
-// with four MO tiles: 65.5 -> 55.4 us for 62 MOs, 380 AOs, 88,689 points;
-// bf16x6 with 40 MOs 44.4 -> 45.0 us, FP32 with 40 56.2 -> 56.7.
+// the Cartesian values, set by set (the same values bit for bit).  Taken with four
+// MO tiles except for bf16x6 (FP32, 62 MOs, 380 AOs, 88,689 points: 65.5 -> 55.4
+// us; bf16x3, 60 MOs, 240 AOs, 362,810 points: 106 -> 101) and for bases with l =
+// 4 (12 atoms x [s,s,p,d,g], 8 MOs, 48^3 points, bf16x6: 43 -> 39 us); bf16x6
+// with 40 MOs takes 44.4 from the monomials and 45.0 so, FP32 with 40 56.2 and 56.7.
 template <int L, int PASS, int SS, bool SETS, typename T>
 __device__ __forceinline__ void shell_rows_to(const FusedArgs& a, const ShellRec& sh, double X, double Y, double Z,
                                               double S0, double S1, double S2, T* dst)
@@ -663,14 +665,16 @@ __device__ __forceinline__ int next_live(const FusedArgs& a, const unsigned long
 // Whether an instance uses one LDS buffer and three workgroups per CU: rho
 // and rho + grad rho with l <= 3 and up to 48 MOs (32 in the batch kernel,
 // which needs a few more registers) fit in 168 VGPRs without spilling (33 KB
-// AO tile plus up to 11.5 KB of C stage) and run at 3 waves/SIMD; the others
-// keep two buffers (66.5 KB, 2 waves/SIMD), where holding C through the
+// AO tile plus up to 11.5 KB of C stage) and run at 3 waves/SIMD, rho + grad rho
+// of up to 16 MOs at 4 (128 VGPRs; with the 129 to 131 that it takes unbounded 5
+// atoms, 10 MOs, 70 x 71 x 73 points take 85 instead of 74 us in bf16x6, 87
+// instead of 76 in FP32); the others keep two buffers (66.5 KB, 2 waves/SIMD), where holding C through the
 // evaluation hides its latency.  FP32 loads its C operand into registers
 // before the evaluation and may hold it through it (hold_c).
 template <int PREC, int PASS, int LM, int MT, bool BATCH> struct FusedPlan {
     static constexpr bool single = PASS <= 1 && LM <= 3 && MT <= (BATCH ? 2 : 3);
     static constexpr int buffers = single ? 1 : 2;
-    static constexpr int occupancy = single ? 3 : 2;
+    static constexpr int occupancy = single ? (PASS == 1 && MT == 1 && !BATCH ? 4 : 3) : 2;
     static constexpr bool c_early = PASS <= 1 ? MT <= 3 : MT <= 2;
     // one-buffer schedule, C in registers (FP32): loaded before the
     // evaluation and held through it, its latency hidden there (FP32 with 3
@@ -690,7 +694,7 @@ __device__ __forceinline__ void rho_tile(const FusedArgs& a, int64_t tile, typen
 {
     using P = FusedPlan<PREC, PASS, LM, MT, BATCH>;
     using Acc = typename Tile<PREC>::Acc;
-    constexpr bool SETS = PREC == OKMI_PREC_F32 && PASS == 0 && MT == 4;   // (shell_rows_to)
+    constexpr bool SETS = PASS == 0 && (LM == 4 || (MT == 4 && PREC != OKMI_PREC_BF16X6));   // (shell_rows_to)
     constexpr int NS = PassCodes<PASS>::n;
     constexpr int BUF = FusedLds<PREC, PASS>::BUF;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
