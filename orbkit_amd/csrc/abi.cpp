@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -228,6 +229,7 @@ extern "C" int okmi_basis_create(int ncont, const int* ncart_per_cont, const int
     *out = nullptr;
     std::vector<ShellRec> shells(ncont);
     std::vector<PrimRec> prims;
+    std::map<std::string, int> blocks;   // by content: offset in T
     std::vector<double> T, craw, frc2, fprc2, frc2s, fprc2s;
     std::vector<int> pl;
     const double pref = std::pow(2.0 / M_PI, 0.75);
@@ -282,9 +284,13 @@ extern "C" int okmi_basis_create(int ncont, const int* ncart_per_cont, const int
         ShellRec& s = shells[c];
         s.cx = geo[3 * at]; s.cy = geo[3 * at + 1]; s.cz = geo[3 * at + 2];
         s.l = l; s.nprim = np; s.prim0 = prow; s.row0 = orow; s.nrow = nrow;
-        s.t0 = (int)T.size(); s.atom = at;
+        s.atom = at;
         s.kind = shell_kind(l, nrow, blk.data(), nout_per_cont != nullptr);
-        T.insert(T.end(), blk.begin(), blk.end());
+        // equal blocks are held once (the kernels that take several shells at a
+        // time read a shared one through scalar loads)
+        const auto held = blocks.emplace(std::string((const char*)blk.data(), 8 * blk.size()), (int)T.size());
+        s.t0 = held.first->second;
+        if (held.second) T.insert(T.end(), blk.begin(), blk.end());
         std::vector<double> al(np), dd(np);
         for (int p = 0; p < np; ++p) {
             const double a = prim_coeffs[2 * (prow + p)], cc = prim_coeffs[2 * (prow + p) + 1];

@@ -234,24 +234,27 @@ __device__ __forceinline__ void split_rows(const RowSets<L, SPH, PASS>& rows, CW
     }
 }
 
-// Rows of four shells with general row maps (nrow each): set by set, the
-// Cartesian values through each lane's transform block
+// Rows of the shells with one general row map (T: nrow rows, through scalar
+// loads): set by set, the Cartesian values through the map
 template <int PASS, int L, int S, int NT, int NR, int NS>
-__device__ __forceinline__ void quad_general(const double* T, int nrow, const ShellPows<L, double>& P, double S0, double S1,
-                                             double S2, const CWhere<NT, NR>& cw, MoAcc<NT, NR, NS>& acc)
+__device__ __forceinline__ void quad_general(const OKMI_CONST double* T, int nrow, const ShellPows<L, double>& P, double S0,
+                                             double S1, double S2, const CWhere<NT, NR>& cw, MoAcc<NT, NR, NS>& acc)
 {
     if constexpr (S < NS) {
         constexpr int NC = ncart(L);
         double c[NC];
         cart_all<L, PassCodes<PASS>::c[S], double>(P, S0, S1, S2, c);
+        COps<NT, NR> co, next;
+        cw.load(0, co);
         for (int r = 0; r < nrow; ++r) {
-            COps<NT, NR> co;
-            cw.load(r, co);
+            cw.load(min(r + 1, nrow - 1), next);
             double v = 0.0;
 #pragma unroll
             for (int k = 0; k < NC; ++k) v = fma(T[r * NC + k], c[k], v);
             mma_set(acc, co, S, v);
+            co = next;
         }
+        __builtin_amdgcn_sched_barrier(0);
         quad_general<PASS, L, S + 1>(T, nrow, P, S0, S1, S2, cw, acc);
     }
 }
@@ -402,7 +405,12 @@ __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* en
         const unsigned idcls = ent[at].idcls, cls = __builtin_amdgcn_readfirstlane(idcls >> LIST_ID_BITS);
         const unsigned kind = cls >> 3 & 3;
         if ((cls & 7) != L || kind != KIND) return;
-        const bool mine = s + g < cnt && idcls >> LIST_ID_BITS == cls;
+        bool mine = s + g < cnt && idcls >> LIST_ID_BITS == cls;
+        int t0 = 0;   // general row maps: shells with the same one
+        if constexpr (KIND == SHELL_T_GENERAL) {
+            t0 = __builtin_amdgcn_readfirstlane(ent[at].t0);
+            mine = mine && ent[at].t0 == t0;
+        }
         const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(mine)) >> 4;
         if (W == 1 ? split && n < 3 : n != 4 / W) return;
         const int w = g & (W - 1);
@@ -450,7 +458,7 @@ __device__ __forceinline__ void class_loop(const F64Args& a, const LiveShell* en
         if constexpr (KIND == SHELL_T_GENERAL) {
             ShellPows<L, double> P;
             P.init(X, Y, Z);
-            quad_general<PASS, L, 0>(a.T + a.shells[base + (e->idcls & LIST_ID_MASK)].t0, (int)(cls >> 5), P, S0, S1, S2, cw, acc);
+            quad_general<PASS, L, 0>(cptr(a.T) + t0, (int)(cls >> 5), P, S0, S1, S2, cw, acc);
         } else {
             const RowSets<L, KIND == SHELL_T_SPHERICAL, PASS> rows(X, Y, Z, S0, S1, S2);
             constexpr bool SPH = KIND == SHELL_T_SPHERICAL;

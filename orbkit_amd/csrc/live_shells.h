@@ -13,12 +13,13 @@ namespace okmi_fused {
 
 // One list entry: the shell (relative to the list's base index) and its class,
 // its first AO row (C column) and its live primitives among the first four,
-// its squared distance to the tile's box, and what its evaluation reads (from
-// LDS, where a load of the shell's record would be waited for).
+// its squared distance to the tile's box, and what its evaluation reads (its
+// place in the table of row maps among them; from LDS, where a load of the shell's record would be waited for).
 struct alignas(16) LiveShell {
     unsigned idcls, rowlive;
     double d2;
     double alpha[4], d[4], c[3];
+    int t0;
 };
 constexpr int LIST_ID_BITS = 18, LIST_ROW_BITS = 29;
 constexpr unsigned LIST_ID_MASK = (1u << LIST_ID_BITS) - 1, LIST_ROW_MASK = (1u << LIST_ROW_BITS) - 1;
@@ -78,6 +79,7 @@ __device__ __forceinline__ int append_live(const ListRec* shells, int nsh, int t
             e.d[q] = sh.d[q];
         }
         e.d2 = d2;
+        e.t0 = sh.t0;
         e.idcls = (unsigned)(i - base) | (unsigned)sh.cls << LIST_ID_BITS;
         e.rowlive = (unsigned)sh.row0 | (unsigned)live << LIST_ROW_BITS;
     }

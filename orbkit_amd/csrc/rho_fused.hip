@@ -241,7 +241,7 @@ int prepare_fused_tables(OkmiBasis* b)
     tables(b->h_frcut2, b->h_fprcut2, fs, groups, is, wsh, fp);
     tables(b->h_frcut2s, b->h_fprcut2s, fs_s, groups_s, is_s, wsh_s, fp_s);
     // by class (angular momentum, kind of row map; real spherical s and p rows
-    // are the Cartesian ones), then by primitives
+    // are the Cartesian ones), general ones by row map, then by primitives
     auto kind_of = [](const ShellRec& sh) {
         return sh.l <= 1 && sh.kind == SHELL_T_SPHERICAL ? (int)SHELL_T_CARTESIAN : sh.kind;
     };
@@ -252,6 +252,7 @@ int prepare_fused_tables(OkmiBasis* b)
         if (p.l != q.l) return p.l > q.l;
         if (kind_of(p) != kind_of(q)) return kind_of(p) > kind_of(q);
         if (p.nrow != q.nrow) return p.nrow > q.nrow;
+        if (p.kind == SHELL_T_GENERAL && p.t0 != q.t0) return p.t0 < q.t0;
         return p.nprim > q.nprim;
     });
     bool standard = true;
