@@ -636,9 +636,10 @@ extern "C" int okmi_rho(const okmi_basis* b, const okmi_grid* g, int64_t p0, int
                                      d_delta, ld_delta, d_mo_norm, d_ws, ws_bytes, (hipStream_t)stream);
     // More: the same kernel over groups of MOs, each evaluating the shells in
     // reach again (a quarter of a group's matrix time) instead of passing the AO
-    // sets through memory, when the workspace holds its copy of C.  (Workspaces
-    // that the staged path refuses stay refused.)
-    if (nmo > 64 && b->max_nrow <= 32 && b->nkpad > 0 && d_ws && staged_fits(b, g, p0, np, nmo, nsets, ws_bytes) &&
+    // sets through memory, when the workspace holds its copy of C and the points
+    // fill its launches.  (Workspaces that the staged path refuses stay refused.)
+    if (nmo > 64 && b->max_nrow <= 32 && b->nkpad > 0 && d_ws &&
+        okmi_rho_f64_fused_pays(b, to_desc(g), p0, np, nmo, drv_out, nout) && staged_fits(b, g, p0, np, nmo, nsets, ws_bytes) &&
         ws_bytes >= okmi_rho_f64_fused_min_bytes(b, nmo, drv_out, nout, d_mo_norm != nullptr))
         return okmi_launch_rho_f64_fused(b, to_desc(g), p0, np, d_c, d_occ, nmo, drv_out, nout, d_rho, d_delta, ld_delta,
                                          d_mo_norm, d_ws, ws_bytes, (hipStream_t)stream);

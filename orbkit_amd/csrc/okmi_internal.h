@@ -171,6 +171,8 @@ void okmi_launch_gather(const double* rho, const double* term, const double* ter
                         int n, double* out, int64_t ld_out, int64_t np, hipStream_t st);
 // FP64 fused density, any number of MOs (more than 64 in several launches over
 // groups of MOs); its workspace: at least the bytes for 64 points
+bool okmi_rho_f64_fused_pays(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, int nmo, const int* drv_out,
+                             int nout);
 size_t okmi_rho_f64_fused_min_bytes(const OkmiBasis* b, int nmo, const int* drv_out, int nout, bool norms);
 int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const double* d_c,
                               const double* d_occ, int nmo, const int* drv_out, int nout, double* rho, double* delta,

@@ -143,6 +143,24 @@ void transpose_c(const OkmiBasis* b, const double* d_c, int nmo, int groups, int
 
 }  // namespace
 
+// More than 64 MOs: the groups follow one another in the fused kernel and share
+// a launch in the staged one, so a few tiles leave the fused one's launches short
+// of work, the more groups there are the longer.  Fused / staged time over 20 to
+// 200 atoms at 1 to 64 and at 216 tiles: rho, with and without first derivatives,
+// 2 groups 0.5 to 1.2 and 0.3 to 0.6, 4 groups 0.9 to 2.4 and 0.5 to 0.8, 32 groups
+// 1.0 to 4.2 and 0.7; diagonal second derivatives, 5 groups 0.6 to 1.1 and 0.2 to
+// 0.5, 20 groups 1.1 to 2.2 and 0.4 to 0.7; mixed ones up to 1.3 and up to 0.4.
+bool okmi_rho_f64_fused_pays(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, int nmo, const int* drv_out,
+                             int nout)
+{
+    const Plan pl(b, nmo, drv_out, nout);
+    F64Args f{};
+    f.grid = g;
+    f.np = np;
+    f.set_bricks(g.regular && p0 == 0 && np == g.nx * g.ny * g.nz);
+    return f.ntile >= 128 || pl.p3 || pl.groups < (pl.p4 ? 10 : 4);
+}
+
 size_t okmi_rho_f64_fused_min_bytes(const OkmiBasis* b, int nmo, const int* drv_out, int nout, bool norms)
 {
     const Plan pl(b, nmo, drv_out, nout);

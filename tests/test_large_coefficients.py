@@ -7,7 +7,7 @@ import numpy
 import pytest
 
 pytestmark = pytest.mark.gpu
-NAO, NMO, POINTS = 24000, 22600, 70
+NAO, NMO, POINTS = 24000, 22600, 8200   # (128 tiles: the fused kernel)
 
 
 def test_more_than_4_gib_of_coefficients():
