@@ -73,10 +73,24 @@ __global__ __launch_bounds__(256) void k_transpose_c(const double* C, int nmo, i
     }
 }
 
-// Tiles from which C is transposed first: reading the caller's C costs a tile
-// about 8 ns more than whole lines of C^T, the transposition and its launch
-// about 3 us.
-constexpr int64_t TRANSPOSE_TILES = 512;
+// Whether C is transposed first, for `tiles` tiles over all passes and u groups of
+// 4 MOs.  The transposition and its launch take about 3 us.  From 512 tiles on
+// reading the caller's C costs more: a tile about 8 ns over whole lines of C^T.
+// Rho alone has little work between the loads of its K steps, 64 lines per 16 MOs
+// where C^T has 8, the more so where a row of C is whole lines of 128 bytes, which
+// share the sets of the vector cache: with more tiles than CUs it pays from 17
+// MOs and 160 AOs on (20 atoms, 400 AOs, 40 MOs, 20,000 points: 94 us in place, 50
+// from C^T; rows of other lengths from about 360 AOs on), with fewer where two or
+// three groups of 4 MOs add loads of their own (400 AOs, 8,192 points, 28 MOs: 52
+// and 44; 56 MOs: 62 and 44; 32 MOs: 36 and 40; 440 AOs, 60 MOs: 60 and 50).
+bool transposed(int64_t tiles, int u, int nao, bool rho_alone)
+{
+    if (tiles >= 512) return true;
+    const bool lines = nao % 16 == 0;
+    if (!rho_alone || u < 5 || nao < (lines ? 160 : 360)) return false;
+    if (tiles > 256) return true;
+    return lines ? u >= 7 && u % 4 >= 2 : u >= 11 && u % 4 == 3;
+}
 
 // Per point: up to 20 term rows; with MO norms one row of per-tile norms per
 // 64 points (at most 64 MOs a launch)
@@ -205,7 +219,7 @@ int okmi_launch_rho_f64_fused(const OkmiBasis* b, const GridDesc& g, int64_t p0,
     f.need_mask = pl.need;
     f.np = std::min(np, chunk);
     f.set_bricks(brick);
-    if (pl.groups > 1 || f.ntile * (1 + (pl.p2 && !pl.p4) + pl.p3) >= TRANSPOSE_TILES) {
+    if (pl.groups > 1 || transposed(f.ntile * (1 + (pl.p2 && !pl.p4) + pl.p3), pl.u, b->nao, pl.first() == 0)) {
         transpose_c(b, d_c, nmo, pl.groups, (int)step, pl.width(), ct, st);
         f.ct_ld = (int)pl.width();
     }
