@@ -505,14 +505,14 @@ int okmi_launch_rho_big(OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np,
     const BigLayout L = big_layout(b, nmo, prec, S);
     int rc0 = okmi_prepare_fused(b);
     if (rc0) return rc0;
-    if (prec != OKMI_PREC_F32 && S <= 4)
-        return okmi_launch_rho_big_split(b, g, p0, np, d_c, d_occ, nmo, prec, S, drv_out, nout, rho, delta, ld_delta, ws,
-                                         ws_bytes, st);
     if (!ws || ws_bytes < L.fixed + L.per_point * 128) {
         okmi_set_error("rho_big: workspace of %zu bytes is too small (need at least %zu)", ws_bytes,
                        L.fixed + L.per_point * 128);
         return 1;
     }
+    if (prec != OKMI_PREC_F32 && S <= 4)   // (which takes less)
+        return okmi_launch_rho_big_split(b, g, p0, np, d_c, d_occ, nmo, prec, S, drv_out, nout, rho, delta, ld_delta, ws,
+                                         ws_bytes, st);
     // a whole regular grid is processed in 4x4x4 bricks (compact point sets
     // for screening, 64-column runs per brick); otherwise in range order
     BrickMap bm{};

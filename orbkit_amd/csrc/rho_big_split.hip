@@ -318,7 +318,7 @@ int okmi_launch_rho_big_split(OkmiBasis* b, const GridDesc& g, int64_t p0, int64
     const size_t fixed = cbytes + obytes + 255;
     const size_t per_point = (size_t)S * kpad * 4 + (size_t)nb * S * 8;
     const size_t per_tile = (size_t)words * 8 + 4 + (size_t)nchunk * 4;
-    if (!ws || ws_bytes < fixed + per_point * 64 + per_tile) {
+    if (ws_bytes < fixed + per_point * 64 + per_tile) {   // (the caller's bound is above it)
         okmi_set_error("rho_big: workspace of %zu bytes is too small (need at least %zu)", ws_bytes,
                        fixed + per_point * 64 + per_tile);
         return 1;

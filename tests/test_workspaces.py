@@ -48,3 +48,32 @@ def test_least_f64_workspace(nmo, drv):
                                      core._stream()), 'okmi_rho_fused')
     assert rel_err(rho.cpu().numpy(), want[0]) <= 1e-12
     assert rel_err(delta.cpu().numpy(), want[1]) <= 1e-12
+
+
+@pytest.mark.parametrize('codes', [[], [1, 2, 3]])
+def test_least_many_mo_workspace(codes):
+  '''More than 64 MOs in split bf16: the least workspace holds C padded to whole
+  groups of 128 MOs and 128 points, one byte less is refused.'''
+  import re
+  import torch
+  from orbkit_amd import core
+  from orbkit_amd.basis import device_basis
+  from orbkit_amd.fused import FusedPlan
+  from test_f64_edges import _molecule
+  qc = _molecule(6, 'sspdf', True, 130)
+  basis = device_basis(qc.geo_spec, qc.ao_spec)
+  dg = core.DeviceGrid(*numpy.random.default_rng(3).uniform(-5, 5, (3, 300)), regular=False)
+  plan = FusedPlan(basis, dg, qc.mo_spec.get_coeffs(), qc.mo_spec.get_occ(), codes, 'bf16x6')
+  plan.launch()
+  whole = plan.result()
+  plan.ws = plan.ws[:1]
+  with pytest.raises(RuntimeError, match='too small') as e:
+    plan.launch()
+  need = int(re.search(r'need at least (\d+)', str(e.value)).group(1))
+  assert need >= 6 * 256 * basis.nao + 128 * 4 * max(1, len(codes) + 1) * basis.nao
+  plan.ws = torch.empty((need - 1) // 8, dtype=torch.float64, device='cuda')
+  with pytest.raises(RuntimeError, match='too small'):
+    plan.launch()
+  plan.ws = torch.empty(-(-need // 8), dtype=torch.float64, device='cuda')
+  plan.launch()
+  assert all(numpy.array_equal(a, b) for a, b in zip(plan.result(), whole))
