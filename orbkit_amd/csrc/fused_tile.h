@@ -9,20 +9,19 @@
 // For each chunk the four waves take the chunk's shells one at a time from a
 // shared counter, costliest first (lane = point), and evaluate them in FP64
 // (coordinates, exponentials, polynomials, the Cartesian-to-spherical map),
-// storing each value in LDS [row][point], rounded once to FP32: one buffer and three workgroups
-// per CU for rho / rho + grad rho with l <= 3, with the chunk's C columns
-// shared through LDS, else double buffering with one barrier per chunk (see
-// FusedPlan).  Each wave
-// then multiplies the rows of its 16-point column with the matching 32
-// columns of C:
+// storing each value in LDS [row][point], rounded once to FP32: one buffer and
+// three or four workgroups per CU for rho / rho + grad rho with l <= 3, with the
+// chunk's C columns shared through LDS, else double buffering with one barrier
+// per chunk (see FusedPlan).  Each wave then multiplies the rows of its 16-point
+// column with the matching 32 columns of C:
 //   F32     v_mfma_f32_16x16x4_f32, C and AO in FP32
 //   BF16X3  v_mfma_f32_16x16x32_bf16 on (hi, lo) splits, 3 products
 //   BF16X6  (hi, mid, lo) splits, 6 products (terms below 2^-24 dropped)
 // accumulating in FP32.  The epilogue forms the density terms in
 // FP64.
 //
-// Screening: a shell whose screening radius (every value and derivative
-// below 1e-40 beyond it) does not reach the tile's bounding box is not
+// Screening: a shell whose screening radius (every value and derivative below
+// OKMI_SCREEN_SPLIT beyond it) does not reach the tile's bounding box is not
 // evaluated (its rows are zero); a chunk with no such shell is skipped,
 // contraction included.
 //
@@ -52,10 +51,8 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int KC = 32;        // AO rows per chunk
 constexpr int PTS = 64;       // points per wave
 
-// LDS AO tile of a precision: element type and row stride.  FP32 rows are
-// padded to 65 floats (conflict-free 16-lane column reads); FP64 rows are
-// 64 doubles, whose reads by the FP64 MFMA operand layout (4 rows x 16
-// points) are not the limit next to the 64-cycle FP64 MFMAs they feed.
+// LDS AO tile of a precision: element type and row stride (rows of 64 points
+// padded to 65 floats: conflict-free 16-lane column reads)
 template <int PREC> struct Tile {
     using T = float;
     using Acc = f4;
@@ -84,7 +81,6 @@ struct FusedArgs {
     int tlx, tly, tlz;        // brick extents 2^tlx x 2^tly x 2^tlz (tlx + tly + tlz = 6)
     int mt_live;              // MO tiles of 16 holding a real MO (0: all MT of the instance)
     int64_t nbx, nby, nbz;    // bricks per axis
-    double* norm_part;        // FP64 kernel: per tile sum_p Phi_m(p)^2, [tile][mpad] (null: not wanted)
 };
 
 // Arguments of the FP64 kernel (fused_f64.h): the shells one by one (sorted by
@@ -203,8 +199,7 @@ struct Box {
 };
 
 // output rows of one shell and AO set from its canonical Cartesian values
-// through its general transform block, into the LDS tile (element type T:
-// rounded once to FP32, or FP64)
+// through its general transform block, into the LDS tile (rounded once to E)
 template <int L, typename E>
 __device__ __forceinline__ void store_rows(const FusedArgs& a, const ShellRec& sh, const double* c, E* dst)
 {
@@ -222,15 +217,14 @@ __device__ __forceinline__ void store_rows(const FusedArgs& a, const ShellRec& s
 // radial sums of the first N primitives of a group:
 // S0 += sum d e, S1 += sum alpha d e, S2 += sum alpha^2 d e, e = exp(-alpha r^2)
 // (the caller applies the powers of two of -2 alpha and 4 alpha^2)
-// (EXACT: the full-accuracy FP64 exponential, else the one accurate to
-// 2.6e-9 for values that end in FP32)
-template <int N, bool need1, bool need2, bool EXACT>
+// (the exponential accurate to 2.6e-9: the values end in FP32)
+template <int N, bool need1, bool need2>
 __device__ __forceinline__ void prim_sums(const PrimGroup& pg, double rr, double& S0, double& S1, double& S2)
 {
     double de[N];
 #pragma unroll
     for (int j = 0; j < N; ++j)
-        de[j] = pg.d[j] * (EXACT ? gauss_f64(pg.alpha[j] * rr) : gauss_f64_fast(pg.alpha[j] * rr));
+        de[j] = pg.d[j] * gauss_f64_fast(pg.alpha[j] * rr);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         S0 += de[j];
@@ -296,10 +290,8 @@ template <int L, int PASS, int SS, bool SETS, typename T>
 __device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const ShellRec& sh, double d2, double px, double py,
                                                  double pz, int k0, T* lds, int lane)
 {
-    constexpr bool EXACT = std::is_same<T, double>::value;
     constexpr int LD = tile_ld<T>();
-    constexpr int NS = PassCodes<PASS>::n;
-    constexpr bool need1 = PASS == 1 || PASS == 2 || PASS == 4;
+    constexpr bool need1 = PASS == 1 || PASS == 2;
     constexpr bool need2 = PASS >= 2;
     const double X = px - sh.cx, Y = py - sh.cy, Z = pz - sh.cz;
     const double rr = X * X + Y * Y + Z * Z;
@@ -314,10 +306,10 @@ __device__ __forceinline__ void eval_shell_chunk(const FusedArgs& a, const Shell
 #pragma unroll
         for (int j = 0; j < 4; ++j) nl += d2 < pg.rcut2[j];   // wave-uniform
         switch (nl) {
-        case 4: prim_sums<4, need1, need2, EXACT>(pg, rr, S0, S1, S2); break;
-        case 3: prim_sums<3, need1, need2, EXACT>(pg, rr, S0, S1, S2); break;
-        case 2: prim_sums<2, need1, need2, EXACT>(pg, rr, S0, S1, S2); break;
-        case 1: prim_sums<1, need1, need2, EXACT>(pg, rr, S0, S1, S2); break;
+        case 4: prim_sums<4, need1, need2>(pg, rr, S0, S1, S2); break;
+        case 3: prim_sums<3, need1, need2>(pg, rr, S0, S1, S2); break;
+        case 2: prim_sums<2, need1, need2>(pg, rr, S0, S1, S2); break;
+        case 1: prim_sums<1, need1, need2>(pg, rr, S0, S1, S2); break;
         default: break;
         }
         if (nl < 4) break;
@@ -662,7 +654,7 @@ __device__ __forceinline__ int next_live(const FusedArgs& a, const unsigned long
     return a.nchunk;
 }
 
-// Whether an instance uses one LDS buffer and three workgroups per CU: rho
+// Whether an instance uses one LDS buffer and three or more workgroups per CU: rho
 // and rho + grad rho with l <= 3 and up to 48 MOs (32 in the batch kernel,
 // which needs a few more registers) fit in 168 VGPRs without spilling (33 KB
 // AO tile plus up to 11.5 KB of C stage) and run at 3 waves/SIMD, rho + grad rho

@@ -37,14 +37,13 @@ struct OkmiBasis {
     int* d_padrows = nullptr;        // internal rows that hold no AO (chunk padding)
     int npadrows = 0;
     PrimRec* d_fprims = nullptr;     // rcut2 = fused radius
-    PrimGroup* d_fgroups = nullptr;  // fused-kernel primitives, groups of 4 per shell in work order
     // the same tables with the radii of the bound OKMI_SCREEN_SPLIT (the
     // paths whose AO values end in FP32; same chunks, rows and work order)
     ShellRec* d_fshells_s = nullptr;
     ShellRec* d_ishells_s = nullptr;
     ShellRec* d_wshells_s = nullptr;
     PrimRec* d_fprims_s = nullptr;
-    PrimGroup* d_fgroups_s = nullptr;
+    PrimGroup* d_fgroups_s = nullptr;   // reduced-precision fused kernel: primitives in groups of 4 per shell, work order
     int* d_colmap = nullptr;         // [nkpad]
     // the FP64 kernels that list the shells in reach of a tile: shells by
     // angular momentum (highest first) with output rows, and the primitives

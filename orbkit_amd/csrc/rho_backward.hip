@@ -8,7 +8,7 @@
 //
 //   A        AO values (okmi_launch_ao_eval)
 //   Phi      = C A                                  (k_gemm_nn, MFMA)
-//   B_ir     = 2 occ_i g_r Phi_ir                   (k_bmat)
+//   B_ir     = 2 occ_i g_r Phi_ir                   (as Phi leaves k_gemm_nn: ColScale)
 //   dL/dC   += B A^T                                (k_gemm_tn, MFMA, split over points,
 //                                                    partials summed in a fixed order)
 //   G        = C^T B   (= dL/dA)                    (k_gemm_nn with C^T)

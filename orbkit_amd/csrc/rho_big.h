@@ -1,6 +1,6 @@
-// Pieces of the many-MO density shared by the contraction with 32-row chunk
-// lists (rho_big.hip) and the split-bf16 contraction with lists of four rows
-// (rho_big_split.hip).
+// Pieces of the many-MO density shared by the contraction of whole 32-row chunks
+// (rho_big.hip) and the split-bf16 one, which leaves out a chunk's dead quads of
+// rows (rho_big_split.hip).
 #pragma once
 #include "okmi_internal.h"
 #include "split_mfma.h"

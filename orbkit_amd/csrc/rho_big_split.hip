@@ -52,7 +52,7 @@ struct SplitArgs {
     int64_t kpad;
     int64_t sub;             // tiles of 64 in ao
     int64_t np;              // points in this chunk
-    const void* C;           // [quad][plane][mpad][4] bf16
+    const void* C;           // [octet of rows][plane][mpad][8] bf16
     int64_t mpad;            // MOs in whole tiles of 16
     const double* occ;       // [mpad], zero padded
     double* partial;         // [nb][S][ld]

@@ -1,8 +1,8 @@
 // Fused density kernel (AO evaluation -> LDS -> MFMA contraction -> density
 // terms) for the FP32 and bf16-split precisions, the gather of orbkit's output
 // rows, the host-side tables and launch sequence for every precision, and
-// the many-molecule batch kernel.  The tile body is in fused_tile.h; the FP64
-// instances are compiled in rho_fused_f64.hip.
+// the many-molecule batch kernel.  The tile body is in fused_tile.h; FP64 has a
+// kernel of its own (fused_f64.h, launched by rho_fused_f64.hip).
 #include "fused_tile.h"
 
 #include <cstring>
@@ -209,18 +209,18 @@ int prepare_fused_tables(OkmiBasis* b)
         return pg;
     };
     auto tables = [&](const std::vector<double>& frc2, const std::vector<double>& fprc2, std::vector<ShellRec>& fs,
-                      std::vector<PrimGroup>& groups, std::vector<ShellRec>& is, std::vector<ShellRec>& wsh,
+                      std::vector<PrimGroup>* groups, std::vector<ShellRec>& is, std::vector<ShellRec>& wsh,
                       std::vector<PrimRec>& fp) {
         fs.assign(work.size(), ShellRec{});
-        groups.clear();
         for (size_t j = 0; j < work.size(); ++j) {
             const int i = work[j];
             fs[j] = b->h_shells[i];
             fs[j].row0 = krow[i];
             fs[j].rcut2 = frc2[i];
-            fs[j].prim0 = (int)groups.size();
+            if (!groups) continue;
+            fs[j].prim0 = (int)groups->size();
             const std::vector<int> order = sorted_prims(b->h_shells[i], fprc2);
-            for (int q = 0; q < b->h_shells[i].nprim; q += 4) groups.push_back(prim_group(order, q, fprc2));
+            for (int q = 0; q < b->h_shells[i].nprim; q += 4) groups->push_back(prim_group(order, q, fprc2));
         }
         // the same shells writing their internal rows (the many-MO and
         // staged paths stage the AO sets in the fused row order), also in
@@ -236,10 +236,10 @@ int prepare_fused_tables(OkmiBasis* b)
         for (int i = 0; i < b->nprim; ++i) fp[i].rcut2 = fprc2[i];
     };
     std::vector<ShellRec> fs, is, wsh, fs_s, is_s, wsh_s;
-    std::vector<PrimGroup> groups, groups_s;
+    std::vector<PrimGroup> groups_s;
     std::vector<PrimRec> fp, fp_s;
-    tables(b->h_frcut2, b->h_fprcut2, fs, groups, is, wsh, fp);
-    tables(b->h_frcut2s, b->h_fprcut2s, fs_s, groups_s, is_s, wsh_s, fp_s);
+    tables(b->h_frcut2, b->h_fprcut2, fs, nullptr, is, wsh, fp);
+    tables(b->h_frcut2s, b->h_fprcut2s, fs_s, &groups_s, is_s, wsh_s, fp_s);
     // by class (angular momentum, kind of row map; real spherical s and p rows
     // are the Cartesian ones), general ones by row map, then by primitives
     auto kind_of = [](const ShellRec& sh) {
@@ -294,7 +294,6 @@ int prepare_fused_tables(OkmiBasis* b)
     up.add(&b->d_chunks, ch);
     up.add(&b->d_fshells, fs);
     up.add(&b->d_fprims, fp);
-    up.add(&b->d_fgroups, groups);
     up.add(&b->d_fgroups_s, groups_s);
     up.add(&b->d_ishells, is);
     up.add(&b->d_wshells, wsh);
@@ -711,9 +710,8 @@ int okmi_batch_build(int nmol, OkmiBasis* const* bases, const GridDesc* grids, c
         const OkmiBasis* bs = bases[m];
         const GridDesc& g = grids[m];
         FusedArgs a{};
-        const bool split = B->prec != OKMI_PREC_F64;   // the screening bound of the arithmetic
-        a.shells = split ? bs->d_fshells_s : bs->d_fshells;
-        a.groups = split ? bs->d_fgroups_s : bs->d_fgroups;
+        a.shells = bs->d_fshells_s;
+        a.groups = bs->d_fgroups_s;
         a.T = bs->d_T;
         a.chunks = bs->d_chunks;
         a.grid = g; a.p0 = 0; a.np = npts[m];
