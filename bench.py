@@ -183,17 +183,22 @@ def timed(step, args, L, names, sync):
 
 # ---------------------------------------------------------------- workloads
 
-def screened_rows(L, basis, axes, precision='f64'):
-  """Sum over the grid's 4x4x4 bricks of (AO rows of the chunks the kernels
-  contract there) x (points in the brick): okmi_fused_live_rows, with the
-  screening radii of the precision ('f64', or one whose AO values end in
-  FP32)."""
+def screened_rows(L, basis, axes, path):
+  """Sum over the grid's 4x4x4 bricks of (AO rows the kernel of this path
+  contracts there) x (points in the brick): the rows of the shells in reach for
+  the fused FP64 kernel (okmi_fused_shell_rows), of the 32-row chunks with such a
+  shell for the others (okmi_fused_live_rows, with the screening radii of the
+  staged FP64 path or of the precisions whose AO values end in FP32)."""
   from orbkit_amd import _native
   ax = [numpy.ascontiguousarray(a, dtype=numpy.float64) for a in axes]
   P = lambda a: a.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
   out = ctypes.c_double()
-  _native.check(L.okmi_fused_live_rows(basis.handle, P(ax[0]), len(ax[0]), P(ax[1]), len(ax[1]), P(ax[2]), len(ax[2]),
-                                       _native.PREC[precision], ctypes.byref(out)), 'okmi_fused_live_rows')
+  grid = (basis.handle, P(ax[0]), len(ax[0]), P(ax[1]), len(ax[1]), P(ax[2]), len(ax[2]))
+  if path == 'f64':
+    _native.check(L.okmi_fused_shell_rows(*grid, ctypes.byref(out)), 'okmi_fused_shell_rows')
+  else:
+    prec = _native.PREC['f64' if path == 'f64_staged' else path]
+    _native.check(L.okmi_fused_live_rows(*grid, prec, ctypes.byref(out)), 'okmi_fused_live_rows')
   return out.value
 
 
@@ -229,7 +234,7 @@ def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
     step, result = plan.launch, plan.result
     if path == 'f64':
       names = ['rho_fused_f64']
-      dom = ('rho_fused_f64', 'k_rho_fused', 'f64', 1)
+      dom = ('rho_fused_f64', 'k_fused_f64', 'f64', 1)
     elif nmo > 64:
       names = ['ao_eval', 'rho_big']
       big = 'k_rho_big' if path == 'f32' or max(codes, default=0) > 3 else 'k_rho_split'
@@ -245,21 +250,23 @@ def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
   peak = PEAK_TFLOPS[dom[2]] / dom[3]
   roof = {'bound': 'mfma', 'achieved': achieved, 'peak': peak, 'unit': 'TFLOP/s', 'frac': achieved / peak,
           'traffic': measured_traffic(dom[1], args.workload, 'f64' if path == 'f64_staged' else path),
-          'kernel': dom[1] + ('<f64>' if path == 'f64' else ''),
+          'kernel': dom[1],
           'kernel_ms_per_step': t_launch * 1e3, 'launches_per_step': cnt / args.steps,
           'algorithmic_flop_per_step': flops}
   if dom[3] > 1:
     roof.update(executed_tflops=achieved * dom[3], mfma_dtype=dom[2], products=dom[3])
   if axes is not None:
-    # the screened contraction (every path: fused, many-MO and staged): per
-    # brick only the AO chunks with a shell in reach (the work the kernel
-    # does besides MO-tile padding)
-    sflops = 2.0 * nmo * nsets * screened_rows(L, basis, axes, 'f64' if path == 'f64_staged' else path)
+    # the screened contraction: per brick only what is in reach (the work the
+    # kernel does besides padding of MOs and of K steps, and the AO evaluation)
+    screen = 'f64_staged' if path == 'f64' and nmo > 64 else path
+    sflops = 2.0 * nmo * nsets * screened_rows(L, basis, axes, screen)
     roof['screened'] = {'flop_per_step': sflops, 'achieved': sflops / t_launch / 1e12,
                         'frac': sflops / t_launch / 1e12 / peak, 'share_of_algorithmic': sflops / flops,
-                        'note': 'algorithmic flops count every AO at every point; the kernel skips the AO chunks '
-                                'whose shells do not reach a brick (values below 1e-24), so frac (algorithmic) can '
-                                'exceed 1 and screened.frac is the hardware utilisation'}
+                        'note': 'algorithmic flops count every AO at every point; the kernel contracts only the %s '
+                                'whose screening radius reaches a brick, so frac (algorithmic) can exceed 1; '
+                                'screened.frac is the share of the matrix peak that this contraction takes, the AO '
+                                'evaluation (FP64 vector instructions) not counted'
+                                % ('shells' if screen == 'f64' else 'AO chunks with a shell')}
   roof['other_kernels_ms_per_step'] = {k: v[1] / args.steps for k, v in times.items() if k != dom[0]}
   return {'value': npts * args.steps / dt, 'ms_per_step': dt / args.steps * 1e3, 'roofline': roof}, result
 

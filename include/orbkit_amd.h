@@ -81,6 +81,8 @@ int okmi_basis_nao(const okmi_basis* b);
  * Replaces c_lcreator (orbkit/c_grid-based.h:3-5) over all contractions as
  * done by cy_core.aocreator (orbkit/cy_core.pyx:49-78), plus the row
  * renormalisation and cartesian2spherical of ao_creator (orbkit/core.py:98-102).
+ * Where every value and derivative of a shell is below 1e-40 at 64 consecutive
+ * points, its rows are exactly 0 there.
  */
 int okmi_ao_eval(const okmi_basis* b, const okmi_grid* g, int64_t p0, int64_t np,
                  const int* drv, int ndrv, int out_dtype, void* d_out, int64_t ld, void* stream);
@@ -96,9 +98,9 @@ int okmi_mocreator(const double* d_ao, int nao, int64_t npts, int64_t ld_ao,
 /*
  * Workspace bytes okmi_rho / okmi_mo_eval need to process `chunk` points per
  * pass with `nsets` AO derivative sets (FP64 AO staging, with the density's
- * live-chunk lists).  The staged density (okmi_rho_staged, okmi_rho beyond
- * 64 MOs) also keeps a copy of C in its row order: nmo x (nao rounded up to
- * whole 32-row chunks) doubles more.
+ * live-chunk lists).  A density of okmi_rho_staged, and of okmi_rho beyond 64
+ * MOs, needs room for a copy of C in the staged row order besides: nmo x (nao
+ * rounded up to whole 32-row chunks) doubles more.
  */
 size_t okmi_workspace_bytes(const okmi_basis* b, int nsets, int64_t chunk);
 
@@ -106,6 +108,11 @@ size_t okmi_workspace_bytes(const okmi_basis* b, int nsets, int64_t chunk);
  * MOs (and their derivatives) on points [p0, p0+np), FP64:
  *   d_mo[j][i][p] = derivative drv[j] of MO i at point p0+p, row stride ld_mo.
  * Replaces slice_rho's calc_mo branch (orbkit/core.py:250-263).
+ * One kernel evaluates and contracts the shells in reach of 64 points (AO terms
+ * below 1e-40 are left out) where the workspace also holds the transpose of C,
+ * nao x (nmo rounded up to 64, and 4) doubles, no code is asked for twice and no
+ * shell has more than 32 rows; otherwise AO sets in passes of the workspace's
+ * size and a product with every AO.
  */
 int okmi_mo_eval(const okmi_basis* b, const okmi_grid* g, int64_t p0, int64_t np,
                  const int* drv, int ndrv, const double* d_c, int nmo,
@@ -122,9 +129,13 @@ int okmi_mo_eval(const okmi_basis* b, const okmi_grid* g, int64_t p0, int64_t np
  * Replaces slice_rho's density branch (orbkit/core.py:179-308).
  * Up to 64 MOs, and when the workspace holds at least
  * okmi_rho_fused_workspace_bytes(b, nmo, OKMI_PREC_F64, 64) bytes, it runs
- * the fused FP64 kernel (AO values in FP64 in LDS, FP64 MFMA; points in
- * passes as large as the workspace allows); otherwise okmi_rho_staged.  The
- * basis's fused-kernel tables are built on first use.
+ * the fused FP64 kernel (the AO values of the shells in reach of 64 points,
+ * terms below 1e-24 left out, go from the registers that hold them into the FP64
+ * MFMAs; points in passes as large as the workspace allows).  More MOs run in
+ * groups of up to 64 through the same kernel when the workspace holds what
+ * okmi_rho_staged needs and the transpose of C, unless the points are few for
+ * the groups (fewer than 128 tiles of 64 points and four groups or more).
+ * Otherwise okmi_rho_staged.
  */
 int okmi_rho(const okmi_basis* b, const okmi_grid* g, int64_t p0, int64_t np,
              const double* d_c, const double* d_occ, int nmo,
@@ -183,7 +194,9 @@ size_t okmi_rho_fused_workspace_bytes(const okmi_basis* b, int nmo, int precisio
  * are handled in one fused launch per pass (MOs never written to memory);
  * with more MOs the AO sets of each chunk of points are staged in HBM
  * (FP32) and contracted by an MFMA GEMM whose epilogue forms the density
- * terms of 128 MOs at a time (same precisions).  Outputs as okmi_rho.
+ * terms of 128 MOs at a time (up to 80 for the bf16 splits without second
+ * derivatives; same precisions).  OKMI_PREC_F64 (up to 64 MOs) is okmi_rho's
+ * fused kernel.  Outputs as okmi_rho.
  * Replaces slice_rho's density branch (orbkit/core.py:179-308) with the
  * reduced-precision contraction; okmi_rho is the FP64 form.
  */
@@ -356,19 +369,28 @@ int okmi_profile_enable(int on);
 int okmi_profile_query(const char* kernel, int* count, double* total_ms);
 
 /*
- * Work measure for measurement tools: the fused kernels (and the many-MO and
- * staged paths) contract, for each 4x4x4 brick of a regular grid, only the
- * 32-row AO chunks with a shell whose screening radius reaches the brick.
+ * Work measure for measurement tools: the reduced-precision fused kernel (and
+ * the many-MO and staged paths) contract, for each 4x4x4 brick of a regular grid,
+ * only the 32-row AO chunks with a shell whose screening radius reaches the brick.
  * For the regular grid with host axes x, y, z this gives *rows_points = sum
  * over bricks of (AO rows of its live chunks) x (grid points in the brick);
  * the screened contraction's flops are 2 * NMO * sets * *rows_points.
- * prec: OKMI_PREC_F64 for the FP64 paths' radii (terms below 1e-24), any
+ * prec: OKMI_PREC_F64 for the staged FP64 path's radii (terms below 1e-24), any
  * other precision for the radii of the paths whose AO values end in FP32
  * (terms below 1e-12).
  * No counterpart in the reference (orbkit evaluates every AO everywhere).
  */
 int okmi_fused_live_rows(const okmi_basis* b, const double* x, int64_t nx, const double* y, int64_t ny,
                          const double* z, int64_t nz, int prec, double* rows_points);
+
+/*
+ * The same for the fused FP64 kernel of okmi_rho and okmi_rho_fused, which
+ * contracts the shells whose screening radius (terms below 1e-24) reaches the
+ * brick, not whole chunks: *rows_points = sum over bricks of (AO rows of the
+ * shells in reach) x (grid points in the brick).
+ */
+int okmi_fused_shell_rows(const okmi_basis* b, const double* x, int64_t nx, const double* y, int64_t ny,
+                          const double* z, int64_t nz, double* rows_points);
 
 #ifdef __cplusplus
 }

@@ -45,6 +45,8 @@ SIGNATURES = {
     'okmi_rho_noalloc': (c_int, [c_vp, ctypes.POINTER(OkmiGrid), c_i64, c_i64, c_vp, c_vp, c_int, P_int, c_int,
                                  c_vp, c_vp, c_i64, c_vp, c_vp]),
     'okmi_profile_enable': (c_int, [c_int]),
+    'okmi_fused_shell_rows': (c_int, [c_vp, ctypes.POINTER(c_dbl), c_i64, ctypes.POINTER(c_dbl), c_i64,
+                                      ctypes.POINTER(c_dbl), c_i64, ctypes.POINTER(c_dbl)]),
     'okmi_fused_live_rows': (c_int, [c_vp, ctypes.POINTER(c_dbl), c_i64, ctypes.POINTER(c_dbl), c_i64,
                                      ctypes.POINTER(c_dbl), c_i64, c_int, ctypes.POINTER(c_dbl)]),
     'okmi_profile_query': (c_int, [ctypes.c_char_p, ctypes.POINTER(c_int), ctypes.POINTER(c_dbl)]),

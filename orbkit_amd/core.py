@@ -185,8 +185,8 @@ def eval_mos(basis, dgrid, codes, coeffs, p0=0, np_=None, sink=None):
 
 def eval_rho(basis, dgrid, coeffs, occ, codes, p0=0, np_=None, mo_norm=False, staged=False, device=False):
   '''Density (np,), derivative outputs (ncodes, np) and optionally the MO
-  norms sum_p phi^2 (nmo,), all FP64: okmi_rho (the fused FP64 kernel up to
-  64 MOs), or with ``staged`` okmi_rho_staged (AO sets through device memory,
+  norms sum_p phi^2 (nmo,), all FP64: okmi_rho (the fused FP64 kernel; see
+  include/orbkit_amd.h for when it stages), or with ``staged`` okmi_rho_staged (AO sets through device memory,
   then the FP64 GEMM).  ``device``: density and derivative rows as device
   tensors instead of host arrays.'''
   torch = _torch()

@@ -826,17 +826,10 @@ int64_t okmi_batch_ntile(const OkmiBatch* B) { return B->ntile; }
 
 int okmi_prepare_fused(OkmiBasis* b) { return prepare_fused_tables(b); }
 
-extern "C" int okmi_fused_live_rows(const okmi_basis* b, const double* x, int64_t nx, const double* y, int64_t ny,
-                                    const double* z, int64_t nz, int prec, double* rows_points)
+// sum over the grid's 4x4x4 bricks of rows(brick's box) x (grid points in it)
+template <typename F>
+static double over_bricks(const double* x, int64_t nx, const double* y, int64_t ny, const double* z, int64_t nz, F&& rows)
 {
-    if (!b || !x || !y || !z || nx <= 0 || ny <= 0 || nz <= 0 || !rows_points) {
-        okmi_set_error("fused_live_rows: invalid arguments");
-        return 1;
-    }
-    if (b->h_chunks.empty()) {
-        okmi_set_error("fused_live_rows: the basis has no fused tables");
-        return 1;
-    }
     // per axis and brick index: the span of the (up to 4) axis values
     auto spans = [](const double* a, int64_t n) {
         std::vector<std::pair<double, double>> s((size_t)((n + 3) / 4));
@@ -849,9 +842,6 @@ extern "C" int okmi_fused_live_rows(const okmi_basis* b, const double* x, int64_
         return s;
     };
     const auto sx = spans(x, nx), sy = spans(y, ny), sz = spans(z, nz);
-    const int nch = (int)b->h_chunks.size();
-    std::vector<int> used(nch);
-    for (int c = 0; c < nch; ++c) used[c] = b->h_chunks[c].y >> 16;
     double total = 0.0;
     for (size_t i = 0; i < sx.size(); ++i)
         for (size_t j = 0; j < sy.size(); ++j)
@@ -861,26 +851,57 @@ extern "C" int okmi_fused_live_rows(const okmi_basis* b, const double* x, int64_
                 const double pts = (double)(std::min<int64_t>(4, nx - 4 * (int64_t)i) *
                                             std::min<int64_t>(4, ny - 4 * (int64_t)j) *
                                             std::min<int64_t>(4, nz - 4 * (int64_t)k));
-                int rows = 0;
-                for (int c = 0; c < nch; ++c) {
-                    const int2 cw = b->h_chunks[c];
-                    const int nsh = cw.y & 0xffff;
-                    for (int e = 0; e < nsh; ++e) {
-                        const ShellRec& sh = (prec == OKMI_PREC_F64 ? b->h_fshells : b->h_fshells_s)[cw.x + e];
-                        const double cc[3] = {sh.cx, sh.cy, sh.cz};
-                        double d2 = 0.0;
-                        for (int d = 0; d < 3; ++d) {
-                            const double dd = std::max(std::max(lo[d] - cc[d], cc[d] - hi[d]), 0.0);
-                            d2 += dd * dd;
-                        }
-                        if (d2 < sh.rcut2) {
-                            rows += used[c];
-                            break;
-                        }
+                auto in_reach = [&](const ShellRec& sh, double rcut2) {
+                    const double cc[3] = {sh.cx, sh.cy, sh.cz};
+                    double d2 = 0.0;
+                    for (int d = 0; d < 3; ++d) {
+                        const double dd = std::max(std::max(lo[d] - cc[d], cc[d] - hi[d]), 0.0);
+                        d2 += dd * dd;
                     }
-                }
-                total += rows * pts;
+                    return d2 < rcut2;
+                };
+                total += rows(in_reach) * pts;
             }
-    *rows_points = total;
+    return total;
+}
+
+extern "C" int okmi_fused_live_rows(const okmi_basis* b, const double* x, int64_t nx, const double* y, int64_t ny,
+                                    const double* z, int64_t nz, int prec, double* rows_points)
+{
+    if (!b || !x || !y || !z || nx <= 0 || ny <= 0 || nz <= 0 || !rows_points) {
+        okmi_set_error("fused_live_rows: invalid arguments");
+        return 1;
+    }
+    if (b->h_chunks.empty()) {
+        okmi_set_error("fused_live_rows: the basis has no fused tables");
+        return 1;
+    }
+    const std::vector<ShellRec>& shells = prec == OKMI_PREC_F64 ? b->h_fshells : b->h_fshells_s;
+    *rows_points = over_bricks(x, nx, y, ny, z, nz, [&](auto in_reach) {
+        int rows = 0;
+        for (const int2& cw : b->h_chunks)   // first shell, shells | used rows << 16
+            for (int e = 0; e < (cw.y & 0xffff); ++e)
+                if (in_reach(shells[cw.x + e], shells[cw.x + e].rcut2)) {
+                    rows += cw.y >> 16;
+                    break;
+                }
+        return rows;
+    });
+    return 0;
+}
+
+extern "C" int okmi_fused_shell_rows(const okmi_basis* b, const double* x, int64_t nx, const double* y, int64_t ny,
+                                     const double* z, int64_t nz, double* rows_points)
+{
+    if (!b || !x || !y || !z || nx <= 0 || ny <= 0 || nz <= 0 || !rows_points) {
+        okmi_set_error("fused_shell_rows: invalid arguments");
+        return 1;
+    }
+    *rows_points = over_bricks(x, nx, y, ny, z, nz, [&](auto in_reach) {
+        int rows = 0;
+        for (int s = 0; s < b->nshell; ++s)
+            if (in_reach(b->h_shells[s], b->h_frcut2[s])) rows += b->h_shells[s].nrow;
+        return rows;
+    });
     return 0;
 }
