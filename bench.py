@@ -204,7 +204,7 @@ def screened_rows(L, basis, axes, path):
 
 def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
   """One way of computing rho (+ grad, + Laplacian) over the whole grid,
-  timed: path 'f64' (fused FP64), 'f64_staged' (AO sets through HBM, then
+  timed: path 'f64' (fused FP64, any number of MOs), 'f64_staged' (AO sets through HBM, then
   the FP64 GEMM with density epilogue), or a reduced precision of the fused
   kernel ('bf16x6', 'bf16x3', 'f32'; more than 64 MOs: the many-MO path).
   Returns (measurements, result getter)."""
@@ -222,13 +222,15 @@ def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
     def step():
-      _native.check(L.okmi_rho_staged(basis.handle, ctypes.byref(dg.desc), 0, npts, ctypes.c_void_p(dC.data_ptr()),
-                                      ctypes.c_void_p(docc.data_ptr()), nmo, codes.ctypes.data_as(_native.P_int),
-                                      len(codes), ctypes.c_void_p(rho.data_ptr()), ctypes.c_void_p(delta.data_ptr()),
-                                      npts, None, ctypes.c_void_p(ws.data_ptr()), ws.numel() * 8, st),
-                    'okmi_rho_staged')
-    names, result = ['ao_eval', 'rho_f64'], (lambda: (rho.cpu().numpy(), delta.cpu().numpy()))
-    dom = ('rho_f64', 'k_rho_f64', 'f64', 1)
+      _native.check(fn(basis.handle, ctypes.byref(dg.desc), 0, npts, ctypes.c_void_p(dC.data_ptr()),
+                       ctypes.c_void_p(docc.data_ptr()), nmo, codes.ctypes.data_as(_native.P_int), len(codes),
+                       ctypes.c_void_p(rho.data_ptr()), ctypes.c_void_p(delta.data_ptr()), npts, None,
+                       ctypes.c_void_p(ws.data_ptr()), ws.numel() * 8, st), 'okmi_rho')
+    result = lambda: (rho.cpu().numpy(), delta.cpu().numpy())
+    if path == 'f64':   # the fused kernel over groups of MOs
+      fn, names, dom = L.okmi_rho, ['rho_fused_f64'], ('rho_fused_f64', 'k_fused_f64', 'f64', 1)
+    else:
+      fn, names, dom = L.okmi_rho_staged, ['ao_eval', 'rho_f64'], ('rho_f64', 'k_rho_f64', 'f64', 1)
   else:
     plan = FusedPlan(basis, dg, C, occ, codes, precision=path)
     step, result = plan.launch, plan.result
@@ -258,15 +260,14 @@ def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
   if axes is not None:
     # the screened contraction: per brick only what is in reach (the work the
     # kernel does besides padding of MOs and of K steps, and the AO evaluation)
-    screen = 'f64_staged' if path == 'f64' and nmo > 64 else path
-    sflops = 2.0 * nmo * nsets * screened_rows(L, basis, axes, screen)
+    sflops = 2.0 * nmo * nsets * screened_rows(L, basis, axes, path)
     roof['screened'] = {'flop_per_step': sflops, 'achieved': sflops / t_launch / 1e12,
                         'frac': sflops / t_launch / 1e12 / peak, 'share_of_algorithmic': sflops / flops,
                         'note': 'algorithmic flops count every AO at every point; the kernel contracts only the %s '
                                 'whose screening radius reaches a brick, so frac (algorithmic) can exceed 1; '
                                 'screened.frac is the share of the matrix peak that this contraction takes, the AO '
                                 'evaluation (FP64 vector instructions) not counted'
-                                % ('shells' if screen == 'f64' else 'AO chunks with a shell')}
+                                % ('shells' if path == 'f64' else 'AO chunks with a shell')}
   roof['other_kernels_ms_per_step'] = {k: v[1] / args.steps for k, v in times.items() if k != dom[0]}
   return {'value': npts * args.steps / dt, 'ms_per_step': dt / args.steps * 1e3, 'roofline': roof}, result
 
@@ -309,7 +310,7 @@ def density_step(args, torch, info, qc, axes):
                                 'rho + grad rho%s' % (args.workload, info['natoms'], nao, nmo, info['side'],
                                                       ' + laplacian' if args.laplacian else ''),
                     'npts': dg.npts, 'nao': nao, 'nmo': nmo, 'ao_sets': nsets,
-                    'path': 'fused' if args.precision != 'f64' or nmo <= 64 else 'staged'},
+                    'path': 'fused'},
          'roofline': head['roofline']}
   legs = [] if args.no_legs else [p for p in ('f64_staged', 'bf16x6') if p != args.precision]
   ref = None
