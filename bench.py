@@ -204,9 +204,10 @@ def screened_rows(L, basis, axes, path):
 
 def density_leg(args, torch, info, basis, dg, C, occ, codes, path, axes=None):
   """One way of computing rho (+ grad, + Laplacian) over the whole grid,
-  timed: path 'f64' (fused FP64, any number of MOs), 'f64_staged' (AO sets through HBM, then
-  the FP64 GEMM with density epilogue), or a reduced precision of the fused
-  kernel ('bf16x6', 'bf16x3', 'f32'; more than 64 MOs: the many-MO path).
+  timed: path 'f64' (fused FP64, any number of MOs), 'f64_staged' (AO sets
+  through HBM, then the FP64 GEMM with density epilogue), or a reduced precision
+  of the fused kernel ('bf16x6', 'bf16x3', 'f32'; more than 64 MOs: the many-MO
+  path).
   Returns (measurements, result getter)."""
   from orbkit_amd import _native
   from orbkit_amd.fused import FusedPlan
