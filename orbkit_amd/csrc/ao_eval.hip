@@ -244,7 +244,11 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
 // go through L2: a row of an odd number of points begins inside a line, whose
 // two parts two waves write, and non-temporal stores sent the parts to memory one
 // by one (126,362 points x 162 rows: 68 us non-temporal, 42 through L2; rows of
-// whole lines, 400 x 4 x 261,568: 631 and 608 us).
+// whole lines, 400 x 4 x 261,568: 631 and 608 us).  The parts meet there only if
+// neighbouring tiles run on one XCD: workgroups are dealt to the eight XCDs in
+// turn, so each XCD takes one eighth of the tiles in order (1,200 rows, tiles
+// in turn and in eighths: 3 sets of 60,001 points 648 and 544 us, 4 sets of
+// 91,125 points 1,427 and 1,140 us; 1 set of 262,144, whole lines, 477 and 480 us).
 struct AoListArgs {
     const ListRec* shells;      // by class, output rows, radii of OKMI_SCREEN
     const PrimGroup* more;
@@ -359,7 +363,9 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a
 {
     constexpr int NS = AoSets<PASS>::n;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+    const unsigned xcd = blockIdx.x & 7, eighth = gridDim.x >> 3, rest = gridDim.x & 7;
+    const unsigned tile = xcd * eighth + (xcd < rest ? xcd : rest) + (blockIdx.x >> 3);
+    const int64_t i = (int64_t)tile * 64 + lane;
     const bool act = i < a.np;
     double px, py, pz;
     grid_point(a.grid, a.p0 + (act ? i : a.np - 1), px, py, pz);
