@@ -147,8 +147,10 @@ __device__ __forceinline__ void shell_out(const AoArgs& a, const ShellRec& sh, d
     }
 }
 
-// occupancy (waves/SIMD) the register allocation targets without spilling:
-// FP32 output 4 (group 0) and 3 (group 1), FP64 output 3 and 2
+// Second derivatives of live chunks (group 1), and every set of a basis with a
+// shell of more than 32 rows, which has no list tables.  Occupancy (waves/SIMD)
+// the register allocation targets without spilling: FP32 output 4 (group 0) and 3
+// (group 1), FP64 output 3 and 2
 template <typename OutT, int GRP>
 __global__ __launch_bounds__(256, sizeof(OutT) == 4 ? (GRP == 0 ? 4 : 3) : (GRP == 0 ? 3 : 2))
 void k_ao_eval(AoArgs a, OutT* __restrict__ out)
@@ -234,7 +236,7 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
     }
 }
 
-// FP64 values of every shell (codes of PASS: 0 value, 1 value and first
+// Values of every shell (codes of PASS: 0 value, 1 value and first
 // derivatives, 2 and 3 value and diagonal or mixed second ones), one lane per
 // point.  The four waves of a workgroup take the same 64 points and every
 // fourth shell each (blockIdx.y: a part of the shells, where the points alone
@@ -249,6 +251,9 @@ void k_ao_eval(AoArgs a, OutT* __restrict__ out)
 // turn, so each XCD takes one eighth of the tiles in order (1,200 rows, tiles
 // in turn and in eighths: 3 sets of 60,001 points 648 and 544 us, 4 sets of
 // 91,125 points 1,427 and 1,140 us; 1 set of 262,144, whole lines, 477 and 480 us).
+// FP32 (exponential of gauss_out): 1,200 rows x 3 sets of 91,125 points 469 us,
+// of 262,144 points 713 us (k_ao_eval, one wave per tile and non-temporal
+// stores: 715 and 843).
 struct AoListArgs {
     const ListRec* shells;      // by class, output rows, radii of OKMI_SCREEN
     const PrimGroup* more;
@@ -358,8 +363,8 @@ __device__ __forceinline__ void list_shell(const AoListArgs& a, const ListRec& s
 #undef OKMI_AO_CASE
 }
 
-template <int PASS>
-__global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a, double* __restrict__ out)
+template <int PASS, typename OutT>
+__global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a, OutT* __restrict__ out)
 {
     constexpr int NS = AoSets<PASS>::n;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -381,12 +386,12 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_list(AoListArgs a
     for (int s = (int)blockIdx.y * a.per + wave; s < end; s += 4) {
         const ListRec sh = load_list(a.shells, s);
         const double d2 = list_dist2(lo, hi, sh);
-        double* o = out + sh.row0 * a.ld + i;
+        OutT* o = out + sh.row0 * a.ld + i;
         if (!(d2 < sh.rcut2)) {   // every value and derivative below the screening bound
             if (act)
                 for (int q = 0; q < NS; ++q) {
                     if (a.dst[q] < 0) continue;
-                    for (int r = 0; r < sh.nrow; ++r) o[a.dst[q] * a.set_stride + r * a.ld] = 0.0;
+                    for (int r = 0; r < sh.nrow; ++r) o[a.dst[q] * a.set_stride + r * a.ld] = (OutT)0;
                 }
             continue;
         }
@@ -485,8 +490,9 @@ __global__ __launch_bounds__(256, PASS == 0 ? 4 : 3) void k_ao_live(AoLiveArgs a
 // until the points give as many (small grids).
 constexpr int64_t AO_WAVES = 16384;
 
-int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const int (&first)[OKMI_MAX_SETS],
-                   double* out, int64_t ld, int64_t set_stride, hipStream_t st)
+template <typename OutT>
+void launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np, const int (&first)[OKMI_MAX_SETS],
+                    OutT* out, int64_t ld, int64_t set_stride, hipStream_t st)
 {
     AoListArgs a{};
     a.shells = b->d_lshells_a;
@@ -506,7 +512,7 @@ int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np
             a.p0 = p0 + 64 * t;
             a.np = std::min(np - 64 * t, 64 * OKMI_MAX_BLOCKS);
             const dim3 grd((unsigned)((a.np + 63) / 64), (unsigned)((b->nshell + a.per - 1) / a.per));
-            hipLaunchKernelGGL((k_ao_list<decltype(pass)::value>), grd, blk, 0, st, a, out + 64 * t);
+            hipLaunchKernelGGL((k_ao_list<decltype(pass)::value, OutT>), grd, blk, 0, st, a, out + 64 * t);
         }
     };
     bool value = first[0] >= 0;   // written by the first pass launched
@@ -528,7 +534,6 @@ int launch_ao_list(const OkmiBasis* b, const GridDesc& g, int64_t p0, int64_t np
         a.dst[0] = first[0];
         launch(std::integral_constant<int, 0>{});
     }
-    return 0;
 }
 
 }  // namespace
@@ -585,8 +590,9 @@ int okmi_launch_ao_eval_ex(const OkmiBasis* b, const ShellRec* shells, const Pri
         width = bricks->nbk * 64;
     }
     OkmiProfScope prof("ao_eval", st);
-    const bool list = !bricks && !live && out_dtype == OKMI_F64 && shells == b->d_shells && b->d_lshells_a;
-    if (list && launch_ao_list(b, g, p0, np, first, (double*)out, ld, set_stride, st)) return 1;
+    const bool list = !bricks && !live && shells == b->d_shells && b->d_lshells_a;
+    if (list && out_dtype == OKMI_F64) launch_ao_list(b, g, p0, np, first, (double*)out, ld, set_stride, st);
+    else if (list) launch_ao_list(b, g, p0, np, first, (float*)out, ld, set_stride, st);
     // values and first derivatives of live chunks (second derivatives: k_ao_eval's group 1)
     if (live) {
         AoLiveArgs w{};
